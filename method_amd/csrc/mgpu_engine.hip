@@ -75,7 +75,7 @@ struct mgpu_engine {
   double *staging = nullptr;
   size_t staging_elems = 0;
   C2PCounters *dstats = nullptr;
-  int *fail_count = nullptr;
+  int *fail_count = nullptr;  // failed cells in the list, workgroups done with their retry
   long long *fail_list = nullptr;
   unsigned char *fail_flag = nullptr;
   double t = 0.0, dt = 0.0, dx = 0.0, dy = 0.0, dz = 0.0;
@@ -712,10 +712,10 @@ int mgpu_create(const mgpu_config *cfg, mgpu_engine **out) {
     if (c.integrator == MGPU_RK4_10 && hipMalloc(&e->rkF, n * e->ncons * g.dims * sizeof(double)) != hipSuccess)
       return cleanup(fail("hipMalloc of the RK4_10 flux store failed"));
   }
-  if (hipMalloc(&e->dstats, sizeof(C2PCounters) * kStatBuckets) != hipSuccess || hipMalloc(&e->fail_count, sizeof(int)) != hipSuccess ||
+  if (hipMalloc(&e->dstats, sizeof(C2PCounters) * kStatBuckets) != hipSuccess || hipMalloc(&e->fail_count, 2 * sizeof(int)) != hipSuccess ||
       hipMalloc(&e->fail_list, n * sizeof(long long)) != hipSuccess || hipMalloc(&e->fail_flag, n) != hipSuccess)
     return cleanup(fail("hipMalloc of C2P work arrays failed"));
-  if (hipMemset(e->fail_count, 0, sizeof(int)) != hipSuccess || hipMemset(e->fail_flag, 0, n) != hipSuccess ||
+  if (hipMemset(e->fail_count, 0, 2 * sizeof(int)) != hipSuccess || hipMemset(e->fail_flag, 0, n) != hipSuccess ||
       hipMemset(e->dstats, 0, sizeof(C2PCounters) * kStatBuckets) != hipSuccess)
     return cleanup(fail("hipMemset failed"));
   *out = e;

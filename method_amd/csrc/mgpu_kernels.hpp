@@ -95,9 +95,8 @@ void launch_c2p_srmhd(const Geo &g, const double *U, double *V, double *A, doubl
                       int *fail_count, long long *fail_list, unsigned char *fail_flag, int cold,
                       unsigned long long *hist, hipStream_t s);
 void launch_c2p_retry_srmhd(const Geo &g, const double *U, double *V, double *A, double *root, double gam,
-                            const int *fail_count, const long long *fail_list, unsigned char *fail_flag,
+                            int *fail_count, const long long *fail_list, unsigned char *fail_flag,
                             long long last_cell, C2PCounters *st, hipStream_t s);
-void launch_zero_int(int *p, hipStream_t s);
 // RKSplit's source half-step and cons2prim over interior cells.
 // A null: the cons2prim root (v^2, Z) goes to `root` in place of the aux.
 void launch_split_srmhd(const Geo &g, double *U, double *V, double *A, double *root, double dt, double gam,
