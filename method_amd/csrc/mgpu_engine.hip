@@ -197,10 +197,6 @@ int run_sweeps(mgpu_engine *e, SweepArgs a, int last_mode) {
     HIP_OK(hipGetLastError());
     return 0;
   }
-  if (dims == 1 && last_mode != kSweepWrite && last_mode != kSweepAdd) {
-    // the x sweep is the only one: the earlier axes' net flux it adds to is zero
-    HIP_OK(hipMemsetAsync(e->fnet, 0, sizeof(double) * e->ncons * e->geo.vstride, e->stream));
-  }
   static const char *names[3][6] = {
       {"sweep_x_write", "sweep_x_add", "sweep_x_stage1_c2p", "sweep_x_stage2_c2p", "sweep_x_imex2", "sweep_x_final"},
       {"sweep_y_write", "sweep_y_add", "sweep_y_stage1_c2p", "sweep_y_stage2_c2p", "sweep_y_imex2", "sweep_y_final"},

@@ -517,11 +517,12 @@ __device__ __forceinline__ void sweep_tile_faces(const SweepArgs &a, double (&s_
 }
 
 // One directional sweep of the flux divergence of model M.
-template <class M, int ORDER, int DAX, int CAX, bool DFAST, int MODE, bool QUIRK>
+template <class M, int ORDER, int DAX, int CAX, bool DFAST, int MODE, bool QUIRK, int TL_ = (DFAST ? 32 : 16),
+          int TC_ = (DFAST ? 8 : 16)>
 __global__ __launch_bounds__(kThreads) void k_sweep(SweepArgs a) {
-  using S = SweepShape<M, ORDER, DAX, CAX, DFAST>;
+  using S = SweepShape<M, ORDER, DAX, CAX, DFAST, TL_, TC_>;
   constexpr int R = S::R, TL = S::TL, TC = S::TC, TLH = S::TLH, EAX = S::EAX;
-  static_assert(TL * TC == kThreads, "one cell per thread in the difference phase");
+  static_assert(TL * TC <= kThreads, "at most one cell per thread in the difference phase");
   constexpr int NV = M::NC;
   // f+ (then f-) of each variable [NV][TLH][TC]; reused for face fluxes.
   __shared__ double s_f[S::kLds];
@@ -689,7 +690,7 @@ __global__ __launch_bounds__(kThreads) void k_sweep(SweepArgs a) {
   const int l = DFAST ? tid % TL : tid / TC;
   const int cc = DFAST ? tid / TL : tid % TC;
   const int gd = d0 + l, gc = c0 + cc;
-  const bool live = gd < nd && gc < nc;
+  const bool live = (TL * TC == kThreads || tid < TL * TC) && gd < nd && gc < nc;
   CellC2P cs;
   if (live) {
     const long long q = base_e + (long long)gd * g.stride[DAX] + (long long)gc * g.stride[CAX];
@@ -705,7 +706,8 @@ __global__ __launch_bounds__(kThreads) void k_sweep(SweepArgs a) {
     } else {
 #pragma unroll
       for (int v = 0; v < NV; ++v)
-        fn[v] = fma(s_f[S::gidx(v, l + 1, cc)] - s_f[S::gidx(v, l, cc)], inv_d, a.fnet[v * vs + q]);
+        fn[v] = fma(s_f[S::gidx(v, l + 1, cc)] - s_f[S::gidx(v, l, cc)], inv_d,
+                    TC_ == 1 ? 0.0 : a.fnet[v * vs + q]);
       if (MODE == kSweepAdd) {
 #pragma unroll
         for (int v = 0; v < NV; ++v) a.fnet[v * vs + q] = fn[v];
@@ -842,46 +844,51 @@ __global__ __launch_bounds__(kThreads, M::NC > 9 ? 1 : 4) void k_sweep_yzf(Sweep
 }
 
 // The y and x terms of a 2-D stage in one launch (sweep plan 3 on 2-D
-// grids): a 16 x 16 (x, y) tile reconstructs its y faces, then its x faces,
+// grids): a TX x TY (x, y) tile reconstructs its y faces, then its x faces,
 // each phase exactly as the separate y and x sweeps do it. Each cell's y net
 // flux waits in LDS for the x term, which is added as the separate x sweep
 // adds it (one fused multiply-add), and the x phase then applies the sweep's
 // mode; so the launch gives the separate sweeps' bits, and the y net flux
 // never makes an HBM round trip. The y phase runs along the contiguous axis.
-// As in k_sweep_yzf, SRRMHD takes each phase in two groups of 8 pencils; a
-// group's 160-176 tile-and-halo cells are one pass of the threads, so its
-// split fluxes go through LDS one half at a time as SRMHD's do (46.6-48.4 KB
-// instead of 64.5-68.2, 125-156 VGPRs instead of 130-182: 3 blocks per CU
-// instead of 2, and the OT 1024^2 steps 3-9 % faster).
-template <class M, int ORDER, int MODE>
+// As in k_sweep_yzf, SRRMHD takes each phase of a 16 x 16 tile in two groups
+// of 8 pencils; a group's 160-176 tile-and-halo cells are one pass of the
+// threads, so its split fluxes go through LDS one half at a time as SRMHD's do
+// (46.6-48.4 KB instead of 64.5-68.2, 125-156 VGPRs instead of 130-182: 3
+// blocks per CU instead of 2, and the OT 1024^2 steps 3-9 % faster). The tile
+// follows from the grid (launch_sweep_xyf_o): with fewer cells than threads a
+// tile's face items still go to every thread, and its first TX TY threads
+// finish the cells.
+template <class M, int ORDER, int MODE, int TX, int TY>
 __global__ __launch_bounds__(kThreads) void k_sweep_xyf(SweepArgs a) {
-  constexpr int kGroup = M::NC > 9 ? 8 : 16;  // pencils per group
-  using SY = SweepShape<M, ORDER, 1, 0, true, 16, kGroup, true>;
-  using SX = SweepShape<M, ORDER, 0, 1, false, 16, kGroup, true>;
+  constexpr int GX = M::NC > 9 ? 8 : TX, GY = M::NC > 9 ? 8 : TY;  // pencils per group of the y, the x phase
+  constexpr int kCellsT = TX * TY;
+  static_assert(kCellsT <= kThreads && TX % GX == 0 && TY % GY == 0, "at most one cell per thread, whole groups");
+  using SY = SweepShape<M, ORDER, 1, 0, true, TY, GX, true>;
+  using SX = SweepShape<M, ORDER, 0, 1, false, TX, GY, true>;
   constexpr int NV = M::NC;
   constexpr int kLds = SY::kLds > SX::kLds ? SY::kLds : SX::kLds;
   __shared__ double s_f[kLds];
-  __shared__ double s_acc[NV][kThreads];  // each cell's y net flux, then with the x term
+  __shared__ double s_acc[NV][kCellsT];  // each cell's y net flux, then with the x term
   const Geo &g = a.geo;
   const int nx = g.n[0], ny = g.n[1];
-  const int tiles_y = (ny + 15) / 16;
+  const int tiles_y = (ny + TY - 1) / TY;
   const int lb = xcd_block(blockIdx.x, gridDim.x);
   const int ty = lb % tiles_y, tx = lb / tiles_y;
-  const int x0 = tx * 16, y0 = ty * 16;
+  const int x0 = tx * TX, y0 = ty * TY;
   const unsigned tid = threadIdx.x;
   // the thread's cell is (x0 + r, y0 + c): neighbouring threads along y, the
   // contiguous axis
-  const int r = tid / 16, c = tid % 16;
-  const bool live = x0 + r < nx && y0 + c < ny;
+  const int r = tid / TY, c = tid % TY;
+  const bool live = (kCellsT == kThreads || tid < kCellsT) && x0 + r < nx && y0 + c < ny;
   const long long q = (long long)(x0 + r) * g.stride[0] + (long long)(y0 + c) * g.stride[1];
 
-  // y phase: faces along y; group h holds the kGroup x pencils from x0 + kGroup h,
-  // whose cells belong to the 16 kGroup threads from 16 kGroup h
+  // y phase: faces along y; group h holds the GX x pencils from x0 + GX h,
+  // whose cells belong to the TY GX threads from TY GX h
 #pragma unroll 1
-  for (int h = 0; h < 16 / kGroup; ++h) {
-    sweep_tile_faces<M, ORDER, 1, 0, true, 16, kGroup, false, true>(a, s_f, y0, x0 + h * kGroup, 0, ny, nx, tid);
-    const int rg = r - h * kGroup;
-    if (live && rg >= 0 && rg < kGroup) {
+  for (int h = 0; h < TX / GX; ++h) {
+    sweep_tile_faces<M, ORDER, 1, 0, true, TY, GX, false, true>(a, s_f, y0, x0 + h * GX, 0, ny, nx, tid);
+    const int rg = r - h * GX;
+    if (live && rg >= 0 && rg < GX) {
 #pragma unroll
       for (int v = 0; v < NV; ++v) s_acc[v][tid] = (s_f[SY::gidx(v, c + 1, rg)] - s_f[SY::gidx(v, c, rg)]) * g.inv_d[1];
     }
@@ -889,10 +896,10 @@ __global__ __launch_bounds__(kThreads) void k_sweep_xyf(SweepArgs a) {
     __builtin_amdgcn_sched_barrier(0);
   }
   CellC2P cs;
-  if constexpr (kGroup == 16) {
+  if constexpr (GY == TY) {
     // x phase over the whole tile, pencils along y: the thread's cell is tile
     // cell r of pencil c, and it finishes straight from the faces in LDS
-    sweep_tile_faces<M, ORDER, 0, 1, false, 16, 16, false>(a, s_f, x0, y0, 0, nx, ny, tid);
+    sweep_tile_faces<M, ORDER, 0, 1, false, TX, GY, false, true>(a, s_f, x0, y0, 0, nx, ny, tid);
     if (live) {
       double fn[NV];
 #pragma unroll
@@ -901,12 +908,12 @@ __global__ __launch_bounds__(kThreads) void k_sweep_xyf(SweepArgs a) {
       sweep_apply<M, MODE>(a, q, fn, cs);
     }
   } else {
-    // x phase: faces along x; group h holds the kGroup y pencils from y0 + kGroup h
+    // x phase: faces along x; group h holds the GY y pencils from y0 + GY h
 #pragma unroll 1
-    for (int h = 0; h < 16 / kGroup; ++h) {
-      sweep_tile_faces<M, ORDER, 0, 1, false, 16, kGroup, false, true>(a, s_f, x0, y0 + h * kGroup, 0, nx, ny, tid);
-      const int cg = c - h * kGroup;
-      if (live && cg >= 0 && cg < kGroup) {
+    for (int h = 0; h < TY / GY; ++h) {
+      sweep_tile_faces<M, ORDER, 0, 1, false, TX, GY, false, true>(a, s_f, x0, y0 + h * GY, 0, nx, ny, tid);
+      const int cg = c - h * GY;
+      if (live && cg >= 0 && cg < GY) {
 #pragma unroll
         for (int v = 0; v < NV; ++v)
           s_acc[v][tid] = fma(s_f[SX::gidx(v, r + 1, cg)] - s_f[SX::gidx(v, r, cg)], g.inv_d[0], s_acc[v][tid]);
@@ -1682,17 +1689,25 @@ __global__ __launch_bounds__(kThreads) void k_flux_vector_srrmhd(Geo g, PadGeo p
   for (int v = 0; v < kSrrmhdCons; ++v) dst[v * pg.ntot + p] = f[v];
 }
 
-template <class M, int ORDER, int DAX, int CAX, bool DFAST, int MODE>
+// Cells per workgroup along the only axis of a 1-D grid: one pencil of 32, so
+// that the 297 (variable, face) items of SRMHD take two passes of the threads
+// and 400 cells 13 workgroups. On the 16 x 16 tile of the strided x sweep 15
+// of 16 pencils were empty (one stage took 10.3-11.1 us at 400 cells, now 5.0-5.3),
+// and its net flux had to be cleared first, one more launch per stage.
+constexpr int kTile1D = 32;
+
+template <class M, int ORDER, int DAX, int CAX, bool DFAST, int MODE, int TL_ = (DFAST ? 32 : 16),
+          int TC_ = (DFAST ? 8 : 16)>
 void launch_sweep_t(const SweepArgs &a, int quirk, hipStream_t s) {
-  using S = SweepShape<M, ORDER, DAX, CAX, DFAST>;
+  using S = SweepShape<M, ORDER, DAX, CAX, DFAST, TL_, TC_>;
   const int tiles = ((a.geo.n[DAX] + S::TL - 1) / S::TL) * ((a.geo.n[CAX] + S::TC - 1) / S::TC) * a.geo.n[S::EAX];
   // stored fluxes already carry the z quirk (k_flux_stored)
   if (M::kStored)
-    hipLaunchKernelGGL((k_sweep<M, ORDER, DAX, CAX, DFAST, MODE, false>), dim3(tiles), dim3(kThreads), 0, s, a);
+    hipLaunchKernelGGL((k_sweep<M, ORDER, DAX, CAX, DFAST, MODE, false, TL_, TC_>), dim3(tiles), dim3(kThreads), 0, s, a);
   else if (quirk && DAX == 2)
-    hipLaunchKernelGGL((k_sweep<M, ORDER, DAX, CAX, DFAST, MODE, true>), dim3(tiles), dim3(kThreads), 0, s, a);
+    hipLaunchKernelGGL((k_sweep<M, ORDER, DAX, CAX, DFAST, MODE, true, TL_, TC_>), dim3(tiles), dim3(kThreads), 0, s, a);
   else
-    hipLaunchKernelGGL((k_sweep<M, ORDER, DAX, CAX, DFAST, MODE, false>), dim3(tiles), dim3(kThreads), 0, s, a);
+    hipLaunchKernelGGL((k_sweep<M, ORDER, DAX, CAX, DFAST, MODE, false, TL_, TC_>), dim3(tiles), dim3(kThreads), 0, s, a);
 }
 
 template <class M, int ORDER, int MODE>
@@ -1701,6 +1716,8 @@ void launch_sweep_o(const SweepArgs &a, int dir, int quirk, hipStream_t s) {
     if (dir == 0) launch_sweep_t<M, ORDER, 0, 2, false, MODE>(a, quirk, s);
     else if (dir == 1) launch_sweep_t<M, ORDER, 1, 2, false, MODE>(a, quirk, s);
     else launch_sweep_t<M, ORDER, 2, 1, true, MODE>(a, quirk, s);
+  } else if (a.geo.dims == 1) {
+    launch_sweep_t<M, ORDER, 0, 1, true, MODE, kTile1D, 1>(a, quirk, s);
   } else {
     if (dir == 0) launch_sweep_t<M, ORDER, 0, 1, false, MODE>(a, quirk, s);
     else launch_sweep_t<M, ORDER, 1, 0, true, MODE>(a, quirk, s);
@@ -1786,10 +1803,35 @@ void launch_sweep_yzf(const SweepArgs &a, int model, int order, int mode, int qu
   }
 }
 
+template <class M, int ORDER, int MODE, int TX, int TY>
+void launch_sweep_xyf_t(const SweepArgs &a, hipStream_t s) {
+  const int tiles = ((a.geo.n[0] + TX - 1) / TX) * ((a.geo.n[1] + TY - 1) / TY);
+  hipLaunchKernelGGL((k_sweep_xyf<M, ORDER, MODE, TX, TY>), dim3(tiles), dim3(kThreads), 0, s, a);
+}
+
+// Tiles of the 2-D launch (KH SRMHD RK2 and OT SRRMHD SSP2 steps, us, with
+// 8 x 8 | 8 x 16 | 16 x 16 tiles):
+//   SRMHD WENO3   64^2 17.7 | 19.9 | 26.4,  192^2 22.2 | 24.3 | 26.6,  256^2 25.8 | 25.3 | 27.4,
+//                 512^2 76.1 | 63.6 | 66.0, 768^2 154 | 117 | 122
+//   SRMHD WENO5   64^2 19.3 | 23.1 | 32.5,  192^2 25.6 | 28.5 | 32.5,  256^2 30.8 | 29.9 | 33.4,
+//                 512^2 88.5 | 76.6 | 78.9, 768^2 177 | 152 | 150
+//   SRRMHD WENO3  64^2 35.7 | 43.1 | 53.5,  192^2 50.4 | 54.8 | 57.1,  256^2 61.4 | 56.6 | 58.1,
+//                 512^2 211 | 171 | 148
+// A small grid does not fill the chip, and a step takes one workgroup's chain
+// of passes: 8 x 8 tiles have four threads per cell, so a quarter of the face
+// passes in it. They recompute more halo fluxes, and past about three
+// workgroups per CU (768 of them on 256 CUs) that costs more than it saves.
+// Beyond, SRMHD takes 8 x 16 tiles, whose 22-24 KB of LDS let 5 workgroups
+// share a CU instead of 3; SRRMHD's 14 variables stay on 16 x 16.
+constexpr int kSmallGridTiles = 768;
+
 template <class M, int ORDER, int MODE>
 void launch_sweep_xyf_o(const SweepArgs &a, hipStream_t s) {
-  const int tiles = ((a.geo.n[0] + 15) / 16) * ((a.geo.n[1] + 15) / 16);
-  hipLaunchKernelGGL((k_sweep_xyf<M, ORDER, MODE>), dim3(tiles), dim3(kThreads), 0, s, a);
+  const long long tiles8 = ((a.geo.n[0] + 7LL) / 8) * ((a.geo.n[1] + 7) / 8);
+  if (tiles8 <= kSmallGridTiles)
+    launch_sweep_xyf_t<M, ORDER, MODE, 8, 8>(a, s);
+  else
+    launch_sweep_xyf_t<M, ORDER, MODE, (M::NC > 9 ? 16 : 8), 16>(a, s);
 }
 
 template <class M, int ORDER>

@@ -6,6 +6,7 @@ import pytest
 
 from method_amd import engine as eng
 from method_amd import initdata as idt
+from oracle import oracle as orc
 
 pytestmark = pytest.mark.gpu
 
@@ -31,3 +32,56 @@ def test_retry_of_every_cell_clears_its_list(n):
             got = e.download()[1]
             assert rc == n**3 and st["failures"] == n**3 and st["fallbacks"] == 0, call
             assert np.abs(got - true).max() <= 1e-10
+
+
+@pytest.mark.parametrize("nx,ny", [(8, 15), (185, 252), (193, 257), (225, 233)])
+@pytest.mark.parametrize("resistive,weno", [(False, 3), (False, 5), (True, 3), (True, 5)])
+def test_2d_tiles_equal_separate_sweeps_bitwise(nx, ny, resistive, weno):
+    """The 2-D launch on its 8 x 8 tiles (up to 768 of them: 185 x 252 is 24 x 32)
+    and on the larger ones beyond, with ragged edges, against the y and x
+    launches of plan 0: the same sums in the same order, so the same bits."""
+    print(f"gpu: 2-D tiles {nx}x{ny} resistive={resistive} weno={weno}", flush=True)
+    g = idt.Grid(nx, ny, 0, 0.0, 1.0, 0.0, 1.0)
+    if resistive:
+        prims = idt.ot_prims_resistive(g)
+        cfg = dict(model=eng.SRRMHD, integrator=eng.SSP2, sigma=10.0)
+    else:
+        prims = idt.kh_prims(g, seed=9)
+        cfg = dict(model=eng.SRMHD, integrator=eng.RK2)
+    got = []
+    for plan in (3, 0):
+        with eng.Engine(eng.Config(nx, ny, 0, 0.0, 1.0, 0.0, 1.0, weno_order=weno,
+                                   bc=(eng.OUTFLOW, eng.PERIODIC, eng.PERIODIC), **cfg)) as e:
+            e.set_sweep_plan(plan)
+            e.set_prims(prims)
+            for _ in range(2):
+                e.update_time()
+            got.append(e.download())
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("nx", [5, 31, 32, 33, 97])
+@pytest.mark.parametrize("weno,periodic", [(3, 1), (5, 0)])
+def test_1d_tiles_match_oracle(nx, weno, periodic):
+    """1-D grids around the 32-cell tile against the oracle: three steps, each
+    exact to the Newton tolerance 1e-12 times the handful of fields it feeds."""
+    ng = 4
+    g = idt.Grid(nx, 0, 0, -0.5, 0.5, 0.0, 1.0)
+    x = np.linspace(-0.6, 0.6, nx + 2 * ng)
+    p = np.zeros((8,) + g.shape)
+    p[0, :, 0, 0], p[4, :, 0, 0] = 1.0 + 0.3 * np.sin(5 * x), 1.0 + 0.2 * np.cos(3 * x)
+    p[1, :, 0, 0], p[2, :, 0, 0], p[3, :, 0, 0] = 0.3 * np.cos(4 * x), 0.2 * np.sin(x), -0.1
+    p[5], p[6, :, 0, 0], p[7] = 0.4, 0.3 * np.sin(2 * x), 0.2
+    print(f"gpu: 1-D {nx} weno={weno}", flush=True)
+    bounds = dict(nx=nx, ny=0, nz=0, xmin=-0.5, xmax=0.5, ymin=0.0, ymax=1.0)
+    with eng.Engine(eng.Config(weno_order=weno, bc=(periodic,) * 3, **bounds)) as e:
+        e.set_prims(p)
+        for _ in range(3):
+            rc, st = e.update_time(stats=True)
+            assert rc == 0 and st["cells"] == 2 * nx
+        c, q, a = e.download()
+    oc, oq, oa, _, _ = orc.Oracle(orc.Case(weno_order=weno, periodic=(periodic,) * 3, **bounds)).run(p, 3)
+    for got, ref in ((c, oc), (q, oq), (a, oa)):
+        for u, v in zip(got[:, ng:-ng], ref[:, ng:-ng]):
+            assert np.abs(u - v).max() <= 1e-11 * max(1.0, np.abs(v).max())
