@@ -7,9 +7,9 @@
 // the tiles of all instances: for a TX x TY tile it reconstructs the y faces
 // and then the x faces through LDS, keeps the y net flux in registers, and
 // applies the stage update and the Newton cons2prim in place, so the net flux
-// never goes to HBM. A clock kernel advances each instance's t, iteration
-// count and dt on the device, and one step (stage one, stage two, clock) is
-// captured in a hipGraph and replayed. Tile shape, schedule and workgroup
+// never goes to HBM. A short launch ends each stage: it retries failed cells
+// and, after stage two, advances each instance's t, iteration count and dt.
+// One step (two stages and their ends) is captured in a hipGraph and replayed. Tile shape, schedule and workgroup
 // count come from an autotuner that times the candidates on the batch itself.
 #include <hip/hip_runtime.h>
 
@@ -31,6 +31,8 @@ int engine_fail(const char *fmt, ...);
 namespace {
 
 constexpr int kThreads = 256;
+constexpr int kSyncStep = 32;   // ints between counters: each has a 128-byte line of its own
+constexpr int kEndBlocks = 64;  // workgroups of a stage's end (the retry)
 constexpr int kXcds = 8;  // MI355X: workgroups go round robin over 8 XCDs, each with its own L2
 
 enum { kSchedStatic = 0, kSchedDynamic = 1 };
@@ -71,9 +73,8 @@ struct BatchArgs {
   int *fail_count;
   long long *fail_list;
   unsigned char *fail_flag;
-  int *sync;             // [0, 8): per-XCD tile counters; [8]: finished workgroups
+  int *sync;             // kSyncStep apart: 8 per-XCD tile counters, then the workgroups done with a retry
   int quirks;
-  int sched;
 };
 
 template <int ORDER, int TX, int TY>
@@ -86,7 +87,8 @@ struct BatchShape {
   static constexpr int kLdsY = NV * TX * WY;
   static constexpr int kLdsX = NV * HX * TY;
   static constexpr int kLds = kLdsY > kLdsX ? kLdsY : kLdsX;
-  static_assert(TX * TY == kThreads, "one cell per thread");
+  static constexpr int kCells = TX * TY;
+  static_assert(kCells <= kThreads, "at most one cell per thread");
 };
 
 // Lax-Friedrichs split flux (alpha = 1) of one cell along DIR
@@ -231,10 +233,13 @@ __device__ __forceinline__ void batch_tile(const BatchArgs &a, double *s_f, doub
         return (v * TX + rr) * WY + lf;
       });
   // the y net flux waits in LDS for the x term (registers are the scarcer)
+  const bool own = S::kCells == kThreads || tid < S::kCells;
+  if (own) {
 #pragma unroll
-  for (int v = 0; v < NV; ++v) {
-    const double *g = s_f + (v * TX + r) * (TY + 1) + c;
-    s_acc[v * kThreads + tid] = (g[1] - g[0]) * I.inv_dy;
+    for (int v = 0; v < NV; ++v) {
+      const double *g = s_f + (v * TX + r) * (TY + 1) + c;
+      s_acc[v * S::kCells + tid] = (g[1] - g[0]) * I.inv_dy;
+    }
   }
   __syncthreads();
 
@@ -256,13 +261,13 @@ __device__ __forceinline__ void batch_tile(const BatchArgs &a, double *s_f, doub
       });
 
   const int gx = x0 + r, gy = y0 + c;
-  if (gx >= I.nx || gy >= I.ny) return;
+  if (!own || gx >= I.nx || gy >= I.ny) return;
   const long long q = I.off + (long long)gx * I.ny + gy;
   double un[NV];
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
     const double *g = s_f + (v * (TX + 1) + r) * TY + c;
-    const double fn = fma(g[TY] - g[0], I.inv_dx, s_acc[v * kThreads + tid]);
+    const double fn = fma(g[TY] - g[0], I.inv_dx, s_acc[v * S::kCells + tid]);
     un[v] = STAGE == 1 ? rk2_stage1(a.U[v * vs + q], fn, dt) : rk2_stage2(a.Un[v * vs + q], a.U[v * vs + q], fn, dt);
   }
   // TimeIntegrator::finalise's cons2prim (timeInt.h:117-132, srmhd.cc:390-562)
@@ -333,15 +338,130 @@ __device__ __forceinline__ void reduce_acc(C2PCounters *st, Acc acc) {
   }
 }
 
-// Retry of the stage's failed cells from the mean root of converged face
-// neighbours (srmhd.cc:465-507), run by the last workgroup to finish, then the
-// fail list is cleared. With quirks, the system solved is the instance's last
-// cell's, as the reference's retry reuses the last cell's arguments.
-__device__ void batch_retry(const BatchArgs &a, bool stage2) {
-  const int nfail = __hip_atomic_load(a.fail_count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+__device__ __forceinline__ void xcd_range(int ntiles, int x, int &lo, int &hi) {
+  lo = (int)((long long)ntiles * x / kXcds);
+  hi = (int)((long long)ntiles * (x + 1) / kXcds);
+}
+
+// The next tile for a workgroup whose own XCD's range is used up, or -1 when
+// every range is: wave 0 reads the 8 counters at once and takes from the range
+// with the most tiles left. A range that another workgroup empties meanwhile
+// reads as empty from then on, so the loop ends.
+__device__ __forceinline__ int steal_tile(const BatchArgs &a) {
+  const int k = threadIdx.x & (kXcds - 1);
+  int lo, hi;
+  xcd_range(a.ntiles, k, lo, hi);
+  for (;;) {
+    int left = hi - lo - __hip_atomic_load(&a.sync[k * kSyncStep], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    int best = (max(left, 0) << 3) | k;
+    for (int off = 1; off < kXcds; off <<= 1) best = max(best, __shfl_xor(best, off));
+    if (best < kXcds) return -1;  // nothing left anywhere
+    const int w = best & (kXcds - 1);
+    int t = 0;
+    if (threadIdx.x == 0) t = atomicAdd(&a.sync[w * kSyncStep], 1);
+    t = __shfl(t, 0);
+    int wlo, whi;
+    xcd_range(a.ntiles, w, wlo, whi);
+    if (wlo + t < whi) return wlo + t;
+  }
+}
+
+// One RK2 stage of every active instance. Workgroup w runs on XCD w % 8; the
+// tiles are cut into 8 contiguous ranges, one per XCD, so neighbouring tiles
+// (which share halo cells) meet in the same L2. Static schedule: the XCD's
+// workgroups stride through its range. Dynamic: they take tiles from the
+// XCD's counter, the next one's number on its way while a tile is worked on,
+// and then from the fullest of the other ranges. (Trying the other counters in
+// turn, all in one cache line, cost 768 workgroups about 100 us a step at the
+// end of the 12-member ensemble: 177 us dynamic against 60 static; now 68.)
+// The schedule is a template parameter: with both in one loop the static one
+// ran 10 % slower (64 members, WENO3: 2.90 against 2.62 ms a step).
+template <int ORDER, int TX, int TY, int STAGE, int SCHED>
+__global__ __launch_bounds__(kThreads, TX * TY == kThreads ? 3 : 4) void k_batch_stage(BatchArgs a) {
+  __shared__ double s_f[BatchShape<ORDER, TX, TY>::kLds];
+  __shared__ double s_acc[kSrmhdCons * TX * TY];
+  __shared__ int s_tile;
+  Acc acc;
+  const int x = blockIdx.x % kXcds;
+  const int nbx = ((int)gridDim.x - x + kXcds - 1) / kXcds;
+  int lo, hi;
+  xcd_range(a.ntiles, x, lo, hi);
+  // the workgroup's next tile (dynamic: known to thread 0)
+  int next = 0;
+  if (SCHED == kSchedStatic) next = lo + (int)blockIdx.x / kXcds;
+  else if (threadIdx.x == 0) next = lo + atomicAdd(&a.sync[x * kSyncStep], 1);
+  for (;;) {
+    int t = next;
+    if (SCHED == kSchedStatic) {
+      next += nbx;
+      if (t >= hi) break;
+    } else {
+      __syncthreads();
+      if (threadIdx.x < 64) {
+        int n = __shfl(next, 0);
+        if (n >= hi) n = steal_tile(a);
+        if (threadIdx.x == 0) s_tile = n;
+      }
+      __syncthreads();
+      t = s_tile;
+      if (t < 0) break;
+      if (threadIdx.x == 0 && next < hi) next = lo + atomicAdd(&a.sync[x * kSyncStep], 1);
+    }
+    batch_tile<ORDER, TX, TY, STAGE>(a, s_f, s_acc, t, acc);
+  }
+  reduce_acc(a.stats, acc);
+}
+
+// Simulation::updateTime's bookkeeping (simulation.cc:113-132) for one
+// instance: with advance, the step just taken moves t by its dt and counts one
+// iteration; then the instance is active while t < end_time, and its next dt
+// is the CFL value with the slow-start factors, clamped to end at end_time.
+__device__ __forceinline__ Clock next_clock(const InstDev &I, Clock c, bool advance) {
+  if (advance && c.active) {
+    c.t = c.t + c.next_dt;
+    c.dt = c.next_dt;
+    c.iters += 1;
+  }
+  c.active = c.t < I.end_time;
+  double dt = I.dt_base;
+  if (c.iters < 15) dt *= 0.1;
+  if (c.iters >= 15 && c.iters < 30) dt *= 0.25;
+  if (c.t + dt > I.end_time) dt = I.end_time - c.t;
+  c.next_dt = dt;
+  return c;
+}
+
+// The clocks before the first step, or of instance `reset` when its state is
+// set anew (-1: none).
+__global__ void k_batch_clock(const InstDev *inst, Clock *clock, int ninst, int reset) {
+  for (int b = blockIdx.x * blockDim.x + threadIdx.x; b < ninst; b += gridDim.x * blockDim.x)
+    clock[b] = next_clock(inst[b], b == reset ? Clock{0.0, 0.0, 0.0, 0, 0} : clock[b], false);
+}
+
+// The end of a stage: the tile counters go back to zero, after stage two the
+// clocks advance, and the stage's failed cells are retried from the mean root
+// of converged face neighbours (srmhd.cc:465-507). With quirks, the system
+// solved is the instance's last cell's, as the reference's retry reuses the
+// last cell's arguments. Almost always no cell failed and this is one short
+// launch. It was the last stage workgroup's work, found by a release fence
+// and a count in every workgroup; on 8 XCDs that fence writes a whole L2
+// back, one after the other: a 12-member, 130,000-cell WENO3 step took 145 us
+// with 256 workgroups of 8 x 32 tiles per stage and 231 with 768, against 94
+// and 59 now.
+// As in k_c2p_retry_srmhd, the last workgroup to finish a retry clears the
+// flags and counters.
+template <int STAGE>
+__global__ __launch_bounds__(kThreads) void k_batch_end(BatchArgs a, Clock *clock) {
+  if (blockIdx.x == 0) {
+    for (int k = threadIdx.x; k < kXcds; k += kThreads) a.sync[k * kSyncStep] = 0;
+    if (STAGE == 2)
+      for (int b = threadIdx.x; b < a.ninst; b += kThreads) clock[b] = next_clock(a.inst[b], clock[b], true);
+  }
+  const int nfail = *a.fail_count;
+  if (nfail == 0) return;
   const long long vs = a.vs;
   const double gam = a.gamma;
-  for (int f = threadIdx.x; f < nfail; f += kThreads) {
+  for (int f = blockIdx.x * kThreads + threadIdx.x; f < nfail; f += gridDim.x * kThreads) {
     const long long q = a.fail_list[f];
     int lo = 0, hi = a.ninst - 1;  // the instance holding q: last with off <= q
     while (lo < hi) {
@@ -382,92 +502,23 @@ __device__ void batch_retry(const BatchArgs &a, bool stage2) {
     double P[8], aux[13];
     srmhd_recover(u, gam, v2, Z, P, aux);
     for (int v = 0; v < 8; ++v) a.Vout[v * vs + q] = P[v];
-    if (stage2) {
+    if (STAGE == 2) {
       a.root[q] = v2;
       a.root[vs + q] = Z;
     }
     if (its < 0) atomicAdd(&a.stats->retry_failures, 1ull);
   }
-  __syncthreads();
-  for (int f = threadIdx.x; f < nfail; f += kThreads) a.fail_flag[a.fail_list[f]] = 0;
-}
-
-__device__ __forceinline__ void xcd_range(int ntiles, int x, int &lo, int &hi) {
-  lo = (int)((long long)ntiles * x / kXcds);
-  hi = (int)((long long)ntiles * (x + 1) / kXcds);
-}
-
-// One RK2 stage of every active instance. Workgroup w runs on XCD w % 8; the
-// tiles are cut into 8 contiguous ranges, one per XCD, so neighbouring tiles
-// (which share halo cells) meet in the same L2. Static schedule: the XCD's
-// workgroups stride through its range. Dynamic: they take tiles from the
-// XCD's counter, then from the other XCDs' counters.
-template <int ORDER, int TX, int TY, int STAGE>
-__global__ __launch_bounds__(kThreads, 3) void k_batch_stage(BatchArgs a) {
-  __shared__ double s_f[BatchShape<ORDER, TX, TY>::kLds];
-  __shared__ double s_acc[kSrmhdCons * kThreads];
-  __shared__ int s_tile, s_last;
-  Acc acc;
-  const int x = blockIdx.x % kXcds;
-  if (a.sched == kSchedStatic) {
-    int lo, hi;
-    xcd_range(a.ntiles, x, lo, hi);
-    const int nbx = ((int)gridDim.x - x + kXcds - 1) / kXcds;
-    for (int t = lo + (int)blockIdx.x / kXcds; t < hi; t += nbx) batch_tile<ORDER, TX, TY, STAGE>(a, s_f, s_acc, t, acc);
-  } else {
-    for (int k = 0; k < kXcds; ++k) {
-      const int xx = (x + k) % kXcds;
-      int lo, hi;
-      xcd_range(a.ntiles, xx, lo, hi);
-      for (;;) {
-        __syncthreads();
-        if (threadIdx.x == 0) s_tile = lo + atomicAdd(&a.sync[xx], 1);
-        __syncthreads();
-        const int t = s_tile;
-        if (t >= hi) break;
-        batch_tile<ORDER, TX, TY, STAGE>(a, s_f, s_acc, t, acc);
-      }
-    }
-  }
-  reduce_acc(a.stats, acc);
-
-  // the last workgroup to finish sees every other one's stores (release
-  // fence before its count, acquire fence after), retries failed cells and
-  // resets the counters for the next launch
+  __shared__ int s_last;
   __threadfence();
   __syncthreads();
-  if (threadIdx.x == 0) s_last = atomicAdd(&a.sync[kXcds], 1) == (int)gridDim.x - 1;
+  if (threadIdx.x == 0) s_last = atomicAdd(&a.sync[kXcds * kSyncStep], 1) == (int)gridDim.x - 1;
   __syncthreads();
   if (!s_last) return;
   __threadfence();
-  batch_retry(a, STAGE == 2);
-  __syncthreads();
+  for (int f = threadIdx.x; f < nfail; f += kThreads) a.fail_flag[a.fail_list[f]] = 0;
   if (threadIdx.x == 0) {
     *a.fail_count = 0;
-    for (int k = 0; k <= kXcds; ++k) a.sync[k] = 0;
-  }
-}
-
-// Simulation::updateTime's bookkeeping (simulation.cc:113-132) per instance:
-// with advance, the step just taken moves t by its dt and counts one
-// iteration; then the instance is active while t < end_time, and its next dt
-// is the CFL value with the slow-start factors, clamped to end at end_time.
-__global__ void k_batch_clock(const InstDev *inst, Clock *clock, int ninst, int advance) {
-  for (int b = blockIdx.x * blockDim.x + threadIdx.x; b < ninst; b += gridDim.x * blockDim.x) {
-    Clock c = clock[b];
-    const InstDev I = inst[b];
-    if (advance && c.active) {
-      c.t = c.t + c.next_dt;
-      c.dt = c.next_dt;
-      c.iters += 1;
-    }
-    c.active = c.t < I.end_time;
-    double dt = I.dt_base;
-    if (c.iters < 15) dt *= 0.1;
-    if (c.iters >= 15 && c.iters < 30) dt *= 0.25;
-    if (c.t + dt > I.end_time) dt = I.end_time - c.t;
-    c.next_dt = dt;
-    clock[b] = c;
+    a.sync[kXcds * kSyncStep] = 0;
   }
 }
 
@@ -475,26 +526,31 @@ __global__ void k_batch_clock(const InstDev *inst, Clock *clock, int ninst, int 
 struct TileShape {
   int tx, ty;
 };
-constexpr TileShape kShapes[] = {{16, 16}, {8, 32}, {32, 8}};
+// 8 x 32 leads on large ensembles (64 members, WENO3: 2.62 ms a step against
+// 2.84 with 16 x 16, 3.06 with 8 x 16), 8 x 16 where the batch has few tiles
+// per CU (12 members: 56.1 us against 59.1); 8 x 8 lost everywhere.
+constexpr TileShape kShapes[] = {{16, 16}, {8, 32}, {32, 8}, {8, 16}};
 constexpr int kNumShapes = sizeof(kShapes) / sizeof(kShapes[0]);
 
 template <int ORDER, int TX, int TY, int STAGE>
-const void *kernel_ptr() {
-  return reinterpret_cast<const void *>(&k_batch_stage<ORDER, TX, TY, STAGE>);
+const void *kernel_ptr(int sched) {
+  return sched == kSchedStatic ? reinterpret_cast<const void *>(&k_batch_stage<ORDER, TX, TY, STAGE, kSchedStatic>)
+                               : reinterpret_cast<const void *>(&k_batch_stage<ORDER, TX, TY, STAGE, kSchedDynamic>);
 }
 
 template <int ORDER, int STAGE>
-const void *stage_kernel_o(int shape) {
+const void *stage_kernel_o(int shape, int sched) {
   switch (shape) {
-    case 0: return kernel_ptr<ORDER, 16, 16, STAGE>();
-    case 1: return kernel_ptr<ORDER, 8, 32, STAGE>();
-    default: return kernel_ptr<ORDER, 32, 8, STAGE>();
+    case 0: return kernel_ptr<ORDER, 16, 16, STAGE>(sched);
+    case 1: return kernel_ptr<ORDER, 8, 32, STAGE>(sched);
+    case 2: return kernel_ptr<ORDER, 32, 8, STAGE>(sched);
+    default: return kernel_ptr<ORDER, 8, 16, STAGE>(sched);
   }
 }
 
-const void *stage_kernel(int order, int shape, int stage) {
-  if (order == 3) return stage == 1 ? stage_kernel_o<3, 1>(shape) : stage_kernel_o<3, 2>(shape);
-  return stage == 1 ? stage_kernel_o<5, 1>(shape) : stage_kernel_o<5, 2>(shape);
+const void *stage_kernel(int order, int shape, int stage, int sched) {
+  if (order == 3) return stage == 1 ? stage_kernel_o<3, 1>(shape, sched) : stage_kernel_o<3, 2>(shape, sched);
+  return stage == 1 ? stage_kernel_o<5, 1>(shape, sched) : stage_kernel_o<5, 2>(shape, sched);
 }
 
 #define BATCH_OK(expr)                                                                               \
@@ -511,7 +567,7 @@ struct mgpu_batch {
   std::vector<mgpu_instance> inst;
   std::vector<long long> off;  // first cell of each instance
   long long vs = 0;            // total cells
-  long long max_cells = 0, max_pad = 0;
+  long long max_pad = 0;
   int ncu = 0;
   hipStream_t stream = nullptr;
   double *U = nullptr, *V = nullptr, *A = nullptr, *U1 = nullptr, *V1 = nullptr;
@@ -519,7 +575,7 @@ struct mgpu_batch {
   // values; the aux is formed from it before anything reads A.
   double *root = nullptr;
   bool aux_stale = false;
-  double *stage_pad = nullptr, *stage_cmp = nullptr;  // per-instance host transfer staging
+  double *stage_pad = nullptr;  // one instance's padded cons, prims and aux on their way to or from the host
   double *backup = nullptr;                           // autotuner's copy of U, V, A
   InstDev *dinst = nullptr;
   Clock *dclock = nullptr;
@@ -608,7 +664,6 @@ BatchArgs stage_args(mgpu_batch *b, int stage) {
   a.fail_flag = b->fail_flag;
   a.sync = b->dsync;
   a.quirks = b->cfg.quirks;
-  a.sched = b->tune.schedule;
   a.Vg = b->V;
   if (stage == 1) {  // U1 = U - dt F(U)
     a.U = b->U;
@@ -626,22 +681,28 @@ BatchArgs stage_args(mgpu_batch *b, int stage) {
   return a;
 }
 
-int launch_clock(mgpu_batch *b, int advance) {
+int launch_clock(mgpu_batch *b, int reset = -1) {
   hipLaunchKernelGGL(k_batch_clock, dim3((b->ninst + 63) / 64), dim3(64), 0, b->stream, b->dinst, b->dclock, b->ninst,
-                     advance);
+                     reset);
   BATCH_OK(hipGetLastError());
   return 0;
 }
 
-// RK2::step of every active instance followed by the clock update.
+// RK2::step of every active instance; the end of stage two updates the clocks.
 int enqueue_step(mgpu_batch *b) {
   for (int stage = 1; stage <= 2; ++stage) {
     BatchArgs a = stage_args(b, stage);
     void *args[] = {&a};
-    const void *k = stage_kernel(b->cfg.weno_order, shape_index(b->tune.tile_x, b->tune.tile_y), stage);
+    const void *k = stage_kernel(b->cfg.weno_order, shape_index(b->tune.tile_x, b->tune.tile_y), stage,
+                                 b->tune.schedule);
     BATCH_OK(hipLaunchKernel(k, dim3(b->tune.blocks), dim3(kThreads), args, 0, b->stream));
+    if (stage == 1)
+      hipLaunchKernelGGL(k_batch_end<1>, dim3(kEndBlocks), dim3(kThreads), 0, b->stream, a, b->dclock);
+    else
+      hipLaunchKernelGGL(k_batch_end<2>, dim3(kEndBlocks), dim3(kThreads), 0, b->stream, a, b->dclock);
+    BATCH_OK(hipGetLastError());
   }
-  return launch_clock(b, 1);
+  return 0;
 }
 
 int ensure_graph(mgpu_batch *b) {
@@ -685,9 +746,9 @@ int fresh_aux(mgpu_batch *b) {
   return 0;
 }
 
-int max_blocks_per_cu(mgpu_batch *b, int shape) {
+int max_blocks_per_cu(mgpu_batch *b, int shape, int sched) {
   int n = 0;
-  const void *k = stage_kernel(b->cfg.weno_order, shape, 2);
+  const void *k = stage_kernel(b->cfg.weno_order, shape, 2, sched);
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k, kThreads, 0) != hipSuccess) return 1;
   return std::max(n, 1);
 }
@@ -723,26 +784,6 @@ PadGeo instance_pad(const mgpu_batch *b, int i) {
   p.off[2] = 0;
   p.ntot = (long long)p.N[0] * p.N[1];
   return p;
-}
-
-// Copies nvar variable planes of instance i between the compact staging
-// buffer (stride = the instance's cells) and a batch field (stride = all cells).
-int move_planes(mgpu_batch *b, int i, int nvar, double *field, bool to_field) {
-  const long long n = (long long)b->inst[i].nx * b->inst[i].ny;
-  for (int v = 0; v < nvar; ++v) {
-    double *f = field + v * b->vs + b->off[i];
-    double *s = b->stage_cmp + v * n;
-    BATCH_OK(hipMemcpyAsync(to_field ? f : s, to_field ? s : f, n * sizeof(double), hipMemcpyDeviceToDevice,
-                            b->stream));
-  }
-  return 0;
-}
-
-int reset_clock(mgpu_batch *b, int i) {
-  Clock c;
-  memset(&c, 0, sizeof c);
-  BATCH_OK(hipMemcpyAsync(b->dclock + i, &c, sizeof c, hipMemcpyHostToDevice, b->stream));
-  return launch_clock(b, 0);
 }
 
 int check_index(const mgpu_batch *b, int i) {
@@ -798,7 +839,6 @@ int mgpu_batch_create(const mgpu_batch_config *cfg, const mgpu_instance *inst, i
     const long long cells = (long long)inst[i].nx * inst[i].ny;
     b->off.push_back(b->vs);
     b->vs += cells;
-    b->max_cells = std::max(b->max_cells, cells);
     b->max_pad = std::max(b->max_pad, (long long)(inst[i].nx + 2 * c.Ng) * (inst[i].ny + 2 * c.Ng));
   }
   auto cleanup = [&](int rc) {
@@ -820,8 +860,7 @@ int mgpu_batch_create(const mgpu_batch_config *cfg, const mgpu_instance *inst, i
               {&b->root, 2 * n},
               {&b->U1, 9 * n},
               {&b->V1, 8 * n},
-              {&b->stage_pad, 30 * (size_t)b->max_pad},
-              {&b->stage_cmp, 30 * (size_t)b->max_cells}};
+              {&b->stage_pad, 30 * (size_t)b->max_pad}};
   for (auto &bf : bufs) {
     if (hipMalloc(bf.p, bf.elems * sizeof(double)) != hipSuccess)
       return cleanup(engine_fail("hipMalloc of %zu bytes failed", bf.elems * sizeof(double)));
@@ -831,10 +870,10 @@ int mgpu_batch_create(const mgpu_batch_config *cfg, const mgpu_instance *inst, i
       hipMalloc(&b->dclock, ninst * sizeof(Clock)) != hipSuccess ||
       hipMalloc(&b->dstats, kStatBuckets * sizeof(C2PCounters)) != hipSuccess ||
       hipMalloc(&b->fail_count, sizeof(int)) != hipSuccess || hipMalloc(&b->fail_list, n * sizeof(long long)) != hipSuccess ||
-      hipMalloc(&b->fail_flag, n) != hipSuccess || hipMalloc(&b->dsync, 16 * sizeof(int)) != hipSuccess)
+      hipMalloc(&b->fail_flag, n) != hipSuccess || hipMalloc(&b->dsync, (kXcds + 1) * kSyncStep * sizeof(int)) != hipSuccess)
     return cleanup(engine_fail("hipMalloc of batch work arrays failed"));
   if (hipMemset(b->dclock, 0, ninst * sizeof(Clock)) != hipSuccess || hipMemset(b->fail_count, 0, sizeof(int)) != hipSuccess ||
-      hipMemset(b->fail_flag, 0, n) != hipSuccess || hipMemset(b->dsync, 0, 16 * sizeof(int)) != hipSuccess ||
+      hipMemset(b->fail_flag, 0, n) != hipSuccess || hipMemset(b->dsync, 0, (kXcds + 1) * kSyncStep * sizeof(int)) != hipSuccess ||
       hipMemset(b->dstats, 0, kStatBuckets * sizeof(C2PCounters)) != hipSuccess)
     return cleanup(engine_fail("hipMemset failed"));
   // default tuning until the autotuner runs: 16 x 16 tiles, static schedule,
@@ -842,10 +881,10 @@ int mgpu_batch_create(const mgpu_batch_config *cfg, const mgpu_instance *inst, i
   b->tune.tile_x = 16;
   b->tune.tile_y = 16;
   b->tune.schedule = kSchedStatic;
-  b->tune.blocks = b->ncu * max_blocks_per_cu(b, 0);
+  b->tune.blocks = b->ncu * max_blocks_per_cu(b, 0, kSchedStatic);
   b->tune.ms_per_step = 0.0;
   if (build_tiles(b)) return cleanup(-1);
-  if (launch_clock(b, 0) || hipStreamSynchronize(b->stream) != hipSuccess) return cleanup(engine_fail("clock init failed"));
+  if (launch_clock(b) || hipStreamSynchronize(b->stream) != hipSuccess) return cleanup(engine_fail("clock init failed"));
   *out = b;
   return 0;
 }
@@ -854,7 +893,7 @@ int mgpu_batch_destroy(mgpu_batch *b) {
   if (!b) return 0;
   if (b->stream) hipStreamSynchronize(b->stream);
   drop_graph(b);
-  double *bufs[] = {b->U, b->V, b->A, b->root, b->U1, b->V1, b->stage_pad, b->stage_cmp, b->backup};
+  double *bufs[] = {b->U, b->V, b->A, b->root, b->U1, b->V1, b->stage_pad, b->backup};
   for (double *p : bufs)
     if (p) hipFree(p);
   void *other[] = {b->dinst, b->dclock, b->dclock_backup, b->dtile_inst, b->dstats, b->fail_count, b->fail_list,
@@ -872,22 +911,11 @@ int mgpu_batch_set_prims(mgpu_batch *b, int i, const double *prims) {
   if (fresh_aux(b)) return -1;  // the other instances' aux first
   const Geo g = instance_geo(b, i);
   const PadGeo p = instance_pad(b, i);
-  const long long n = g.vstride;
   BATCH_OK(hipMemcpyAsync(b->stage_pad, prims, 8 * p.ntot * sizeof(double), hipMemcpyHostToDevice, b->stream));
-  // compact prims into planes 9..16 of the staging buffer, then primsToAll
-  // writes cons into planes 0..8 and aux into 17..29 (Simulation::set,
-  // simulation.cc:80-101)
-  double *sc = b->stage_cmp, *sv = sc + 9 * n, *sa = sc + 17 * n;
-  launch_compact(g, p, 8, b->stage_pad, sv, b->stream);
-  launch_prims_to_all_srmhd(g, sv, sc, sa, b->cfg.gamma, b->stream);
+  const long long o = b->off[i];
+  launch_set_srmhd(g, p, b->stage_pad, b->V + o, b->U + o, b->A + o, b->vs, b->cfg.gamma, b->stream);
   BATCH_OK(hipGetLastError());
-  for (int v = 0; v < 9; ++v)
-    BATCH_OK(hipMemcpyAsync(b->U + v * b->vs + b->off[i], sc + v * n, n * sizeof(double), hipMemcpyDeviceToDevice, b->stream));
-  for (int v = 0; v < 8; ++v)
-    BATCH_OK(hipMemcpyAsync(b->V + v * b->vs + b->off[i], sv + v * n, n * sizeof(double), hipMemcpyDeviceToDevice, b->stream));
-  for (int v = 0; v < 13; ++v)
-    BATCH_OK(hipMemcpyAsync(b->A + v * b->vs + b->off[i], sa + v * n, n * sizeof(double), hipMemcpyDeviceToDevice, b->stream));
-  if (reset_clock(b, i)) return -1;
+  if (launch_clock(b, i)) return -1;
   BATCH_OK(hipStreamSynchronize(b->stream));
   return 0;
 }
@@ -901,13 +929,14 @@ int mgpu_batch_upload_state(mgpu_batch *b, int i, const double *cons, const doub
   const double *src[3] = {cons, prims, aux};
   double *dst[3] = {b->U, b->V, b->A};
   const int nv[3] = {9, 8, 13};
+  double *pad = b->stage_pad;
   for (int f = 0; f < 3; ++f) {
-    BATCH_OK(hipMemcpyAsync(b->stage_pad, src[f], nv[f] * p.ntot * sizeof(double), hipMemcpyHostToDevice, b->stream));
-    launch_compact(g, p, nv[f], b->stage_pad, b->stage_cmp, b->stream);
+    BATCH_OK(hipMemcpyAsync(pad, src[f], nv[f] * p.ntot * sizeof(double), hipMemcpyHostToDevice, b->stream));
+    launch_compact(g, p, nv[f], pad, dst[f] + b->off[i], b->vs, b->stream);
     BATCH_OK(hipGetLastError());
-    if (move_planes(b, i, nv[f], dst[f], true)) return -1;
+    pad += nv[f] * p.ntot;
   }
-  if (reset_clock(b, i)) return -1;
+  if (launch_clock(b, i)) return -1;
   BATCH_OK(hipStreamSynchronize(b->stream));
   return 0;
 }
@@ -920,14 +949,16 @@ int mgpu_batch_download_state(mgpu_batch *b, int i, double *cons, double *prims,
   double *dst[3] = {cons, prims, aux};
   double *src[3] = {b->U, b->V, b->A};
   const int nv[3] = {9, 8, 13};
+  // each array has its own part of the staging buffer, so one wait serves all
+  double *pad = b->stage_pad;
   for (int f = 0; f < 3; ++f) {
     if (!dst[f]) continue;
-    if (move_planes(b, i, nv[f], src[f], false)) return -1;
-    launch_expand(g, p, nv[f], b->stage_cmp, b->stage_pad, 0, b->stream);
+    launch_expand(g, p, nv[f], src[f] + b->off[i], b->vs, pad, 0, b->stream);
     BATCH_OK(hipGetLastError());
-    BATCH_OK(hipMemcpyAsync(dst[f], b->stage_pad, nv[f] * p.ntot * sizeof(double), hipMemcpyDeviceToHost, b->stream));
-    BATCH_OK(hipStreamSynchronize(b->stream));
+    BATCH_OK(hipMemcpyAsync(dst[f], pad, nv[f] * p.ntot * sizeof(double), hipMemcpyDeviceToHost, b->stream));
+    pad += nv[f] * p.ntot;
   }
+  BATCH_OK(hipStreamSynchronize(b->stream));
   return 0;
 }
 
@@ -1016,9 +1047,9 @@ int mgpu_batch_autotune(mgpu_batch *b, int trial_steps, mgpu_batch_tuning *best,
   int count = 0;
   int rc = 0;
   for (int s = 0; s < kNumShapes && rc == 0; ++s) {
-    const int maxb = max_blocks_per_cu(b, s);
     for (int sched = kSchedStatic; sched <= kSchedDynamic && rc == 0; ++sched) {
-      for (int bpc = 1; bpc <= maxb && rc == 0; ++bpc) {
+      const int maxb = max_blocks_per_cu(b, s, sched);
+      for (int bpc = std::max(1, maxb - 1); bpc <= maxb && rc == 0; ++bpc) {
         mgpu_batch_tuning cand;
         cand.tile_x = kShapes[s].tx;
         cand.tile_y = kShapes[s].ty;

@@ -765,13 +765,15 @@ int mgpu_upload_state(mgpu_engine *e, const double *cons, const double *prims, c
   const double *src[3] = {cons, prims, aux};
   double *dst[3] = {e->U, e->V, e->A};
   const int nv[3] = {e->ncons, e->nprims, e->naux};
+  double *pad = e->staging;  // each array has its own part, so one wait serves all
   for (int a = 0; a < 3; ++a) {
     if (!src[a]) continue;
-    HIP_OK(hipMemcpyAsync(e->staging, src[a], sizeof(double) * nv[a] * e->pad.ntot, hipMemcpyHostToDevice, e->stream));
-    launch_compact(e->geo, e->pad, nv[a], e->staging, dst[a], e->stream);
+    HIP_OK(hipMemcpyAsync(pad, src[a], sizeof(double) * nv[a] * e->pad.ntot, hipMemcpyHostToDevice, e->stream));
+    launch_compact(e->geo, e->pad, nv[a], pad, dst[a], e->geo.vstride, e->stream);
     HIP_OK(hipGetLastError());
-    HIP_OK(hipStreamSynchronize(e->stream));
+    pad += nv[a] * e->pad.ntot;
   }
+  HIP_OK(hipStreamSynchronize(e->stream));
   if (aux) e->aux_stale = false;
   return 0;
 }
@@ -783,13 +785,15 @@ int mgpu_download_state(mgpu_engine *e, double *cons, double *prims, double *aux
   double *dst[3] = {cons, prims, aux};
   const double *src[3] = {e->U, e->V, e->A};
   const int nv[3] = {e->ncons, e->nprims, e->naux};
+  double *pad = e->staging;
   for (int a = 0; a < 3; ++a) {
     if (!dst[a]) continue;
-    launch_expand(e->geo, e->pad, nv[a], src[a], e->staging, 0, e->stream);
+    launch_expand(e->geo, e->pad, nv[a], src[a], e->geo.vstride, pad, 0, e->stream);
     HIP_OK(hipGetLastError());
-    HIP_OK(hipMemcpyAsync(dst[a], e->staging, sizeof(double) * nv[a] * e->pad.ntot, hipMemcpyDeviceToHost, e->stream));
-    HIP_OK(hipStreamSynchronize(e->stream));
+    HIP_OK(hipMemcpyAsync(dst[a], pad, sizeof(double) * nv[a] * e->pad.ntot, hipMemcpyDeviceToHost, e->stream));
+    pad += nv[a] * e->pad.ntot;
   }
+  HIP_OK(hipStreamSynchronize(e->stream));
   return 0;
 }
 
@@ -843,7 +847,7 @@ int mgpu_fnet(mgpu_engine *e, double *fnet) {
   if (ensure_staging(e)) return -1;
   SweepArgs a = sweep_args(e, e->U, e->V, nullptr);
   if (run_sweeps(e, a, kSweepAdd)) return -1;
-  launch_expand(e->geo, e->pad, e->ncons, e->fnet, e->staging, 1, e->stream);
+  launch_expand(e->geo, e->pad, e->ncons, e->fnet, e->geo.vstride, e->staging, 1, e->stream);
   HIP_OK(hipGetLastError());
   HIP_OK(hipMemcpyAsync(fnet, e->staging, sizeof(double) * e->ncons * e->pad.ntot, hipMemcpyDeviceToHost, e->stream));
   HIP_OK(hipStreamSynchronize(e->stream));
@@ -891,7 +895,7 @@ int mgpu_source_extension(mgpu_engine *e, double *source) {
   HIP_OK(hipGetLastError());
   // variables 0..7 of the reference's 9-variable source array; phi's stays 0
   HIP_OK(hipMemsetAsync(e->staging, 0, sizeof(double) * e->ncons * e->pad.ntot, e->stream));
-  launch_expand(e->geo, e->pad, 8, e->rg_src, e->staging, 1, e->stream);
+  launch_expand(e->geo, e->pad, 8, e->rg_src, e->geo.vstride, e->staging, 1, e->stream);
   HIP_OK(hipGetLastError());
   HIP_OK(hipMemcpyAsync(source, e->staging, sizeof(double) * e->ncons * e->pad.ntot, hipMemcpyDeviceToHost,
                         e->stream));
@@ -955,7 +959,7 @@ int mgpu_flux_reconstruction(mgpu_engine *e, const double *cons, const double *f
       HIP_OK(hipMemcpyAsync(sc, cons, sizeof(double) * nv * plane, hipMemcpyHostToDevice, e->stream));
       HIP_OK(hipMemcpyAsync(sf, f, sizeof(double) * nv * plane, hipMemcpyHostToDevice, e->stream));
     } else {
-      launch_expand(e->geo, e->pad, nv, e->U, sc, 0, e->stream);
+      launch_expand(e->geo, e->pad, nv, e->U, e->geo.vstride, sc, 0, e->stream);
       if (dir < e->geo.dims) {
         if (e->cfg.model == MGPU_SRMHD)
           launch_flux_vector_srmhd(e->geo, e->pad, e->U, e->V, sf, dir, e->cfg.quirks, e->stream);

@@ -1287,22 +1287,49 @@ __global__ __launch_bounds__(kThreads) void k_max_wavespeed_srmhd(Geo g, const d
   }
 }
 
-// Padded reference layout -> interior device layout for nvar variables.
-__global__ __launch_bounds__(kThreads) void k_compact(Geo g, PadGeo pg, int nvar, const double *src, double *dst) {
+// Padded reference layout -> interior device layout for nvar variables, whose
+// planes lie vs apart in dst.
+__global__ __launch_bounds__(kThreads) void k_compact(Geo g, PadGeo pg, int nvar, const double *src, double *dst,
+                                                       long long vs) {
   const long long q = (long long)blockIdx.x * kThreads + threadIdx.x;
   if (q >= g.vstride) return;
   const int i = (int)(q / g.stride[0]);
   const int j = (int)((q / g.stride[1]) % g.n[1]);
   const int k = (int)(q % g.n[2]);
   const long long p = ((long long)(i + pg.off[0]) * pg.N[1] + (j + pg.off[1])) * pg.N[2] + (k + pg.off[2]);
-  for (int v = 0; v < nvar; ++v) dst[v * g.vstride + q] = src[v * pg.ntot + p];
+  for (int v = 0; v < nvar; ++v) dst[v * vs + q] = src[v * pg.ntot + p];
+}
+
+// SRMHD's Simulation::set for one grid of an ensemble (simulation.cc:80-101):
+// padded host-layout prims into the prims, cons and aux fields, whose planes
+// lie vs apart. One pass; compacting into a buffer, converting there and
+// copying the 30 planes out one by one took 32 operations of 5-10 us a grid.
+__global__ __launch_bounds__(kThreads) void k_set_srmhd(Geo g, PadGeo pg, const double *src, double *V, double *U,
+                                                         double *A, long long vs, double gam) {
+  const long long q = (long long)blockIdx.x * kThreads + threadIdx.x;
+  if (q >= g.vstride) return;
+  const int i = (int)(q / g.stride[0]);
+  const int j = (int)((q / g.stride[1]) % g.n[1]);
+  const int k = (int)(q % g.n[2]);
+  const long long p = ((long long)(i + pg.off[0]) * pg.N[1] + (j + pg.off[1])) * pg.N[2] + (k + pg.off[2]);
+  double P[8], u[9], aux[13];
+#pragma unroll
+  for (int v = 0; v < 8; ++v) P[v] = src[v * pg.ntot + p];
+  srmhd_prims_to_all(P, gam, u, aux);
+#pragma unroll
+  for (int v = 0; v < 8; ++v) V[v * vs + q] = P[v];
+#pragma unroll
+  for (int v = 0; v < 9; ++v) U[v * vs + q] = u[v];
+#pragma unroll
+  for (int v = 0; v < 13; ++v) A[v * vs + q] = aux[v];
 }
 
 // Interior device layout -> padded reference layout with every ghost cell
 // holding the value Bcs::apply gives it (per-axis remap, x then y then z).
 // ghosts_zero: leave ghosts at zero instead (FVS::F writes interior only).
-__global__ __launch_bounds__(kThreads) void k_expand(Geo g, PadGeo pg, int nvar, const double *src, double *dst,
-                                                      int ghosts_zero) {
+// src's planes lie vs apart.
+__global__ __launch_bounds__(kThreads) void k_expand(Geo g, PadGeo pg, int nvar, const double *src, long long vs,
+                                                      double *dst, int ghosts_zero) {
   const long long p = (long long)blockIdx.x * kThreads + threadIdx.x;
   if (p >= pg.ntot) return;
   const int I = (int)(p / ((long long)pg.N[1] * pg.N[2]));
@@ -1317,7 +1344,7 @@ __global__ __launch_bounds__(kThreads) void k_expand(Geo g, PadGeo pg, int nvar,
     x = remap(x, g.n[ax], g.periodic[ax]);
     q += (long long)x * g.stride[ax];
   }
-  for (int v = 0; v < nvar; ++v) dst[v * pg.ntot + p] = (ghost && ghosts_zero) ? 0.0 : src[v * g.vstride + q];
+  for (int v = 0; v < nvar; ++v) dst[v * pg.ntot + p] = (ghost && ghosts_zero) ? 0.0 : src[v * vs + q];
 }
 
 // Model::fluxVector of the resident state for every padded cell (the padded
@@ -1947,13 +1974,20 @@ void launch_rk410_prepare2(const Geo &g, int ncons, double *U1, double *U2, hipS
   hipLaunchKernelGGL(k_rk410_prepare2, dim3(blocks_for(n)), dim3(kThreads), 0, s, n, U1, U2);
 }
 
-void launch_compact(const Geo &g, const PadGeo &pg, int nvar, const double *src, double *dst, hipStream_t s) {
-  hipLaunchKernelGGL(k_compact, dim3(blocks_for(g.vstride)), dim3(kThreads), 0, s, g, pg, nvar, src, dst);
+void launch_compact(const Geo &g, const PadGeo &pg, int nvar, const double *src, double *dst, long long vs,
+                    hipStream_t s) {
+  hipLaunchKernelGGL(k_compact, dim3(blocks_for(g.vstride)), dim3(kThreads), 0, s, g, pg, nvar, src, dst, vs);
 }
 
-void launch_expand(const Geo &g, const PadGeo &pg, int nvar, const double *src, double *dst, int ghosts_zero,
-                   hipStream_t s) {
-  hipLaunchKernelGGL(k_expand, dim3(blocks_for(pg.ntot)), dim3(kThreads), 0, s, g, pg, nvar, src, dst, ghosts_zero);
+void launch_set_srmhd(const Geo &g, const PadGeo &pg, const double *src, double *V, double *U, double *A,
+                      long long vs, double gam, hipStream_t s) {
+  hipLaunchKernelGGL(k_set_srmhd, dim3(blocks_for(g.vstride)), dim3(kThreads), 0, s, g, pg, src, V, U, A, vs, gam);
+}
+
+void launch_expand(const Geo &g, const PadGeo &pg, int nvar, const double *src, long long vs, double *dst,
+                   int ghosts_zero, hipStream_t s) {
+  hipLaunchKernelGGL(k_expand, dim3(blocks_for(pg.ntot)), dim3(kThreads), 0, s, g, pg, nvar, src, vs, dst,
+                     ghosts_zero);
 }
 
 void launch_imex1_srrmhd(const SweepArgs &a, hipStream_t s) {

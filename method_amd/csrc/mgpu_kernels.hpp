@@ -158,9 +158,15 @@ void launch_regime_dwdsb(const Geo &g, const PadGeo &pg, const double *V, const 
 // there. The two give the same source bit for bit.
 void launch_regime_source(const Geo &g, const PadGeo &pg, const double dx[3], const double *V, double *work,
                           double *src, double gam, double sigma, int order, bool fused, hipStream_t s);
-void launch_compact(const Geo &g, const PadGeo &pg, int nvar, const double *src, double *dst, hipStream_t s);
-void launch_expand(const Geo &g, const PadGeo &pg, int nvar, const double *src, double *dst, int ghosts_zero,
-                   hipStream_t s);
+// vs: the distance of the variables' planes in the interior layout (g.vstride
+// on a single grid, the cells of all grids in an ensemble's fields).
+void launch_compact(const Geo &g, const PadGeo &pg, int nvar, const double *src, double *dst, long long vs,
+                    hipStream_t s);
+void launch_expand(const Geo &g, const PadGeo &pg, int nvar, const double *src, long long vs, double *dst,
+                   int ghosts_zero, hipStream_t s);
+// Padded SRMHD prims into prims, cons and aux.
+void launch_set_srmhd(const Geo &g, const PadGeo &pg, const double *src, double *V, double *U, double *A,
+                      long long vs, double gam, hipStream_t s);
 void launch_source_srmhd(const Geo &g, const PadGeo &pg, const double *U, double *dst, double cp, hipStream_t s);
 
 // ---- reference-API operators outside the time step (mgpu_cells.hip)

@@ -85,3 +85,35 @@ def test_1d_tiles_match_oracle(nx, weno, periodic):
     for got, ref in ((c, oc), (q, oq), (a, oa)):
         for u, v in zip(got[:, ng:-ng], ref[:, ng:-ng]):
             assert np.abs(u - v).max() <= 1e-11 * max(1.0, np.abs(v).max())
+
+
+def test_batch_tilings_and_retry_launch():
+    """Every tile shape and schedule, with fewer workgroups than tiles on an
+    XCD and more than there are tiles, gives the same bits; a member whose
+    every cell starts from |v| = 1 is retried by the launch that ends a stage,
+    once per stage and step, which it can only count when the list is cleared."""
+    sizes = [(17, 33), (8, 8), (40, 31)]
+    print("gpu: batch tilings", flush=True)
+    prims = [idt.kh_prims(idt.Grid(nx, ny, 0, -0.5, 0.5, -1.0, 1.0), seed=k) for k, (nx, ny) in enumerate(sizes)]
+    ref = None
+    for tile in ((16, 16), (8, 32), (32, 8), (8, 16)):
+        for sched in (0, 1):
+            for blocks in (8, 2048):
+                with eng.Batch([eng.Instance(nx, ny) for nx, ny in sizes], weno_order=3, quirks=0) as b:
+                    for k, p in enumerate(prims):
+                        b.set_prims(k, p)
+                    b.set_tuning(*tile, sched, blocks)
+                    assert b.step(3) == 0
+                    out = [b.download(k) for k in range(len(sizes))]
+                    c, p, a = b.download(0)
+                    bad = p.copy()
+                    bad[0] = 1e-310  # the starting root Z = rho h / (1 - v^2) is infinite
+                    b.upload(0, c, bad, a)
+                    rc, st = b.step(2, stats=True)
+                    # both stages of the first step start from the bad prims, the second step from good ones
+                    assert st["failures"] == rc == 2 * 17 * 33 and st["fallbacks"] == 0, (tile, sched, blocks)
+                if ref is None:
+                    ref = out
+                for x, y in zip(out, ref):
+                    for u, v in zip(x, y):
+                        assert np.array_equal(u, v)
