@@ -43,7 +43,7 @@ struct InstDev {
   int tile_base;       // first tile of this instance in the batch's tile list
   int tiles_y;         // tiles along y
   long long off;       // index of cell (0, 0) in the concatenated cell range
-  double inv_dx, inv_dy;
+  double half_inv_dx, half_inv_dy;  // 1 / (2 dx), 1 / (2 dy)
   double dt_base;      // cfl min(dx, dy) / sqrt(2) before the slow-start factors
   double end_time;
 };
@@ -104,8 +104,8 @@ __device__ __forceinline__ void split_flux(const BatchArgs &a, long long q, doub
   srmhd_flux<DIR, false>(u, vx, vy, vz, p, f);
 #pragma unroll
   for (int v = 0; v < 9; ++v) {
-    fp[v] = 0.5 * (f[v] + u[v]);
-    fm[v] = 0.5 * (f[v] - u[v]);
+    fp[v] = f[v] + u[v];  // doubled
+    fm[v] = f[v] - u[v];
   }
 }
 
@@ -152,7 +152,7 @@ __device__ __forceinline__ void tile_faces(const BatchArgs &a, double *s_f, int 
     const int item = tid + k * kThreads;
     if (item < NITEMS) {
       const double *fpv = s_f + item_at(item);
-      Weno<ORDER>::up([&](int m) { return fpv[m * STEP]; }, nu[k], du[k]);
+      Weno<ORDER, true>::up([&](int m) { return fpv[m * STEP]; }, nu[k], du[k]);
     }
   }
   // the upwind halves are formed before the barrier after which f- overwrites f+
@@ -174,7 +174,7 @@ __device__ __forceinline__ void tile_faces(const BatchArgs &a, double *s_f, int 
     if (item < NITEMS) {
       const double *fmv = s_f + item_at(item);
       double nd, dd;
-      Weno<ORDER>::down([&](int m) { return fmv[m * STEP]; }, nd, dd);
+      Weno<ORDER, true>::down([&](int m) { return fmv[m * STEP]; }, nd, dd);
       nu[k] = weno_combine(nu[k], du[k], nd, dd);
     }
   }
@@ -238,7 +238,7 @@ __device__ __forceinline__ void batch_tile(const BatchArgs &a, double *s_f, doub
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
       const double *g = s_f + (v * TX + r) * (TY + 1) + c;
-      s_acc[v * S::kCells + tid] = (g[1] - g[0]) * I.inv_dy;
+      s_acc[v * S::kCells + tid] = (g[1] - g[0]) * I.half_inv_dy;
     }
   }
   __syncthreads();
@@ -267,7 +267,7 @@ __device__ __forceinline__ void batch_tile(const BatchArgs &a, double *s_f, doub
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
     const double *g = s_f + (v * (TX + 1) + r) * TY + c;
-    const double fn = fma(g[TY] - g[0], I.inv_dx, s_acc[v * S::kCells + tid]);
+    const double fn = fma(g[TY] - g[0], I.half_inv_dx, s_acc[v * S::kCells + tid]);
     un[v] = STAGE == 1 ? rk2_stage1(a.U[v * vs + q], fn, dt) : rk2_stage2(a.Un[v * vs + q], a.U[v * vs + q], fn, dt);
   }
   // TimeIntegrator::finalise's cons2prim (timeInt.h:117-132, srmhd.cc:390-562)
@@ -622,8 +622,8 @@ int build_tiles(mgpu_batch *b) {
     // Data::initData / Simulation::Simulation (simData.cc:74-79, simulation.cc:34-36)
     const double dx = (in.xmax - in.xmin) / in.nx;
     const double dy = (in.ymax - in.ymin) / in.ny;
-    d.inv_dx = 1.0 / dx;
-    d.inv_dy = 1.0 / dy;
+    d.half_inv_dx = 0.5 / dx;
+    d.half_inv_dy = 0.5 / dy;
     // Simulation::updateTime (simulation.cc:113-118): 2-D, dz infinite, alpha = 1
     const double sd = std::sqrt(2.0);
     const double dtX = in.cfl * dx / (1.0 * sd);

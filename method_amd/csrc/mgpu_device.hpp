@@ -18,6 +18,7 @@ struct Geo {
   long long vstride;    // elements per variable plane = n0*n1*n2
   int periodic[3];      // 1 periodic, 0 outflow
   double inv_d[3];      // 1/dx, 1/dy, 1/dz
+  double half_inv_d[3]; // half of those, for differences of face fluxes kept doubled
   int dims;
 };
 
@@ -58,6 +59,11 @@ __device__ __forceinline__ int remap(int i, int n, int periodic) {
 // quantity up to rounding. The indicators and candidate values are written in
 // first differences of the stencil so that they share their terms.
 
+// The sweeps stage the split fluxes doubled, f + u and f - u, which spares a
+// multiplication per value (DBL): every quantity below is then a power of two
+// times the plain one, eps with it, so the face value is exactly twice the
+// plain one and the factor leaves in the difference's 1 / (2 dx).
+
 constexpr double kWenoEps = 1e-16;
 
 // Upwind reconstruction at the right face of v1 from (v0, v1, v2), as a
@@ -65,10 +71,12 @@ constexpr double kWenoEps = 1e-16;
 // face of v1 is the same function of (v2, v1, v0). Linear weights (1/3, 2/3)
 // over 1/3 give t0 = s1, t1 = 2 s0; candidates q0 = v1 + (v1 - v0)/2 and
 // q1 = (v1 + v2)/2, so t1 q1 = s0 (v1 + v2).
+template <bool DBL>
 __device__ __forceinline__ void weno3_nd(double v0, double v1, double v2, double &n, double &d) {
   const double a0 = v1 - v0, a1 = v2 - v1;
+  constexpr double eps = (DBL ? 16.0 : 1.0) * kWenoEps;
   const double b0 = a0 * a0, b1 = a1 * a1;
-  const double s0 = fma(b0, b0, kWenoEps), s1 = fma(b1, b1, kWenoEps);
+  const double s0 = fma(b0, b0, eps), s1 = fma(b1, b1, eps);
   n = fma(s1, fma(0.5, a0, v1), s0 * (v1 + v2));
   d = fma(2.0, s0, s1);
 }
@@ -84,10 +92,11 @@ __device__ __forceinline__ void weno3_nd(double v0, double v1, double v2, double
 //   q0     = (2 v0 - 7 v1 + 11 v2)/6 = a0/3 + v2 - d12/2,
 //   6 q1   = -v1 + 5 v2 + 2 v3      = 6 v2 - d12 - 2 d23,
 //   3 q2   = (2 v2 + 5 v3 - v4)/2   = 3 v3 + d23 + d34/2.
+template <bool DBL>
 __device__ __forceinline__ void weno5_nd(double v0, double v1, double v2, double v3, double v4, double &n,
                                          double &d) {
   constexpr double c13 = 13.0 / 3.0;
-  constexpr double eps16 = 16.0 * kWenoEps;
+  constexpr double eps16 = (DBL ? 256.0 : 16.0) * kWenoEps;
   const double d01 = v0 - v1, d12 = v1 - v2, d23 = v2 - v3, d34 = v3 - v4;
   const double a0 = d01 - d12, a1 = d12 - d23, a2 = d23 - d34;
   const double e0 = fma(-3.0, d12, d01), e1 = d12 + d23, e2 = fma(3.0, d23, -d34);
@@ -103,20 +112,37 @@ __device__ __forceinline__ void weno5_nd(double v0, double v1, double v2, double
   d = fma(6.0, p1, fma(3.0, p2, p0));
 }
 
-// a / b for a positive normal b whose reciprocal is normal too (the WENO
-// denominators, products of eps-bounded positive sums): the hardware
-// reciprocal estimate refined by two Newton-Raphson steps, then one residual
-// correction of the quotient. It skips the operand scaling and special-case
-// fix-up of the general IEEE division and can differ from it in the last bit.
+// a / b, 1 / b and 1 / sqrt(b) for a positive normal b whose reciprocal is
+// normal too, from the hardware's estimates (relative error below 2^-24 and
+// 2^-23 over 6.7e7 random operands). They skip the operand scaling and the
+// special-case fix-up of the IEEE operations, 11 and 13 dependent
+// instructions, and give NaN for b = 0 or infinite.
+//   div_pos: one Newton-Raphson step takes the reciprocal's error to 2^-48,
+//     and the residual correction the quotient's to its rounding: it equalled
+//     a / b in every bit on those operands (the second step it used to take
+//     changed none).
+//   rcp_pos: e = 1 - b r, then r (1 + e + e^2), error e^3: at most 1 ulp.
+//   rsqrt_pos: e = 1 - b y^2, then y (1 + e/2 + 3/8 e^2): at most 1.3 ulp.
 __device__ __forceinline__ double div_pos(double a, double b) {
   double r = __builtin_amdgcn_rcp(b);
-  r = fma(fma(-b, r, 1.0), r, r);
   r = fma(fma(-b, r, 1.0), r, r);
   const double q = a * r;
   return fma(fma(-b, q, a), r, q);
 }
 
-template <int ORDER>
+__device__ __forceinline__ double rcp_pos(double b) {
+  const double r = __builtin_amdgcn_rcp(b);
+  const double e = fma(-b, r, 1.0);
+  return fma(fma(e, e, e), r, r);
+}
+
+__device__ __forceinline__ double rsqrt_pos(double b) {
+  const double y = __builtin_amdgcn_rsq(b);
+  const double e = fma(-(b * y), y, 1.0);
+  return fma(y * e, fma(0.375, e, 0.5), y);
+}
+
+template <int ORDER, bool DBL = false>
 struct Weno;
 
 // Face value = upwind reconstruction of f+ plus downwind reconstruction of
@@ -127,17 +153,17 @@ __device__ __forceinline__ double weno_combine(double nu, double du, double nd, 
   return div_pos(fma(nu, dd, nd * du), du * dd);
 }
 
-template <>
-struct Weno<3> {
+template <bool DBL>
+struct Weno<3, DBL> {
   static constexpr int R = 2;  // stencil radius = (order + 1) / 2
   // Face between cells R-1 and R of p[0 .. 2R-1] (upwind on fp, downwind on fm).
   template <class LP>
   __device__ __forceinline__ static void up(LP fp, double &n, double &d) {
-    weno3_nd(fp(0), fp(1), fp(2), n, d);
+    weno3_nd<DBL>(fp(0), fp(1), fp(2), n, d);
   }
   template <class LM>
   __device__ __forceinline__ static void down(LM fm, double &n, double &d) {
-    weno3_nd(fm(3), fm(2), fm(1), n, d);
+    weno3_nd<DBL>(fm(3), fm(2), fm(1), n, d);
   }
   template <class LP, class LM>
   __device__ __forceinline__ static double face(LP fp, LM fm) {
@@ -148,16 +174,16 @@ struct Weno<3> {
   }
 };
 
-template <>
-struct Weno<5> {
+template <bool DBL>
+struct Weno<5, DBL> {
   static constexpr int R = 3;
   template <class LP>
   __device__ __forceinline__ static void up(LP fp, double &n, double &d) {
-    weno5_nd(fp(0), fp(1), fp(2), fp(3), fp(4), n, d);
+    weno5_nd<DBL>(fp(0), fp(1), fp(2), fp(3), fp(4), n, d);
   }
   template <class LM>
   __device__ __forceinline__ static void down(LM fm, double &n, double &d) {
-    weno5_nd(fm(5), fm(4), fm(3), fm(2), fm(1), n, d);
+    weno5_nd<DBL>(fm(5), fm(4), fm(3), fm(2), fm(1), n, d);
   }
   template <class LP, class LM>
   __device__ __forceinline__ static double face(LP fp, LM fm) {
@@ -183,8 +209,8 @@ __device__ __forceinline__ void srmhd_flux(const double u[9], double vx, double 
                                            double f[9]) {
   const double Bx = u[5], By = u[6], Bz = u[7];
   const double v2 = vx * vx + vy * vy + vz * vz;
-  const double iW = sqrt(1.0 - v2);  // 1/W
-  const double W = 1.0 / iW;
+  const double W = rsqrt_pos(1.0 - v2);
+  const double iW = (1.0 - v2) * W;  // 1/W
   const double b0 = W * (vx * Bx + vy * By + vz * Bz);
   const double bx = fma(Bx, iW, b0 * vx), by = fma(By, iW, b0 * vy), bz = fma(Bz, iW, b0 * vz);
   const double bsq = (Bx * Bx + By * By + Bz * Bz + b0 * b0) * (iW * iW);
@@ -242,26 +268,26 @@ __device__ __forceinline__ int srmhd_newton(double D, double tau, double Bsq, do
                                             double &v2, double &Z) {
   if (!(v2 >= 0.0 && v2 < 1.0)) v2 = 0.0;
   if (!(Z > 0.0)) Z = D + tau + Bsq;
-  const double gf = (gam - 1.0) / gam;
+  const double gf = (gam - 1.0) * rcp_pos(gam);
   const double BS2 = BS * BS;
   for (int it = 0; it <= kNewtonMaxIt; ++it) {
-    const double s = 1.0 - v2, sq = sqrt(s);
+    const double s = 1.0 - v2, isq = rsqrt_pos(s), sq = s * isq;
     const double p = gf * (Z * s - D * sq);
     const double ZB = Z + Bsq;
-    const double iZ = 1.0 / Z;
+    const double iZ = rcp_pos(Z);
     const double iZ2 = iZ * iZ;
     const double f0 = ZB * ZB * v2 - (2.0 * Z + Bsq) * BS2 * iZ2 - Ssq;
     const double f1 = ZB - p - 0.5 * Bsq * s - 0.5 * BS2 * iZ2 - D - tau;
-    const double iZB = 1.0 / ZB;
+    const double iZB = rcp_pos(ZB);
     const double r = fmax(fabs(f0) * iZB * iZB, fabs(f1) * iZB);
     if (r <= kNewtonTol) return it;
     if (!(r == r) || it == kNewtonMaxIt) break;
     const double BS2iZ3 = BS2 * iZ2 * iZ;
     const double J00 = ZB * ZB;
     const double J01 = 2.0 * ZB * (v2 + BS2iZ3);
-    const double J10 = gf * (Z - 0.5 * D / sq) + 0.5 * Bsq;
+    const double J10 = gf * (Z - 0.5 * D * isq) + 0.5 * Bsq;
     const double J11 = 1.0 - gf * s + BS2iZ3;
-    const double idet = 1.0 / (J00 * J11 - J01 * J10);
+    const double idet = rcp_pos(J00 * J11 - J01 * J10);
     const double d0 = (J11 * f0 - J01 * f1) * idet;
     const double d1 = (J00 * f1 - J10 * f0) * idet;
     double nv2 = v2 - d0, nZ = Z - d1;
@@ -280,17 +306,17 @@ __device__ __forceinline__ void srmhd_recover(const double U[9], double gam, dou
   const double BS = U[5] * U[1] + U[6] * U[2] + U[7] * U[3];
   const double Bsq = U[5] * U[5] + U[6] * U[6] + U[7] * U[7];
   const double Ssq = U[1] * U[1] + U[2] * U[2] + U[3] * U[3];
-  const double W = 1.0 / sqrt(1.0 - v2);
-  const double rho = U[0] / W;
-  const double h = Z / (rho * W * W);
-  const double p = (h - 1.0) * rho * (gam - 1.0) / gam;
+  const double W = rsqrt_pos(1.0 - v2);
+  const double iW = (1.0 - v2) * W;
+  const double rho = U[0] * iW;
+  const double h = div_pos(Z, rho * W * W);
+  const double p = (h - 1.0) * rho * ((gam - 1.0) * rcp_pos(gam));
   const double e = p / (rho * (gam - 1.0));
-  const double den = 1.0 / (Z * (Bsq + Z));
+  const double den = rcp_pos(Z * (Bsq + Z));
   const double vx = (U[5] * BS + U[1] * Z) * den;
   const double vy = (U[6] * BS + U[2] * Z) * den;
   const double vz = (U[7] * BS + U[3] * Z) * den;
   const double b0 = W * (U[5] * vx + U[6] * vy + U[7] * vz);
-  const double iW = 1.0 / W;
   P[0] = rho;
   P[1] = vx;
   P[2] = vy;

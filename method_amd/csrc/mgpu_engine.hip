@@ -650,6 +650,7 @@ int mgpu_create(const mgpu_config *cfg, mgpu_engine **out) {
   g.inv_d[0] = 1.0 / e->dx;
   g.inv_d[1] = c.ny > 0 ? 1.0 / e->dy : 0.0;
   g.inv_d[2] = c.nz > 0 ? 1.0 / e->dz : 0.0;
+  for (int ax = 0; ax < 3; ++ax) g.half_inv_d[ax] = 0.5 * g.inv_d[ax];
   PadGeo &p = e->pad;
   p.N[0] = c.nx + 2 * c.Ng;
   p.N[1] = c.ny > 0 ? c.ny + 2 * c.Ng : 1;

@@ -387,8 +387,8 @@ __device__ __forceinline__ void sweep_tile_faces(const SweepArgs &a, double (&s_
           M::template flux<DAX, QUIRK>(u, pl, a, q, f);
   #pragma unroll
           for (int v = 0; v < NV; ++v) {
-            fp[v] = 0.5 * (f[v] + u[v]);
-            fm_keep[cp][v] = 0.5 * (f[v] - u[v]);
+            fp[v] = f[v] + u[v];  // doubled
+            fm_keep[cp][v] = f[v] - u[v];
           }
         } else {
   #pragma unroll
@@ -418,7 +418,7 @@ __device__ __forceinline__ void sweep_tile_faces(const SweepArgs &a, double (&s_
       const unsigned item = tid + k * kThreads;
       if (item < kItems) {
         const double *fpv = s_f + S::item_fidx(item);
-        Weno<ORDER>::up([&](int m) { return fpv[m * S::kStrideL]; }, nu[k], du[k]);
+        Weno<ORDER, true>::up([&](int m) { return fpv[m * S::kStrideL]; }, nu[k], du[k]);
       }
     }
     // the upwind halves are formed here, before the barrier after which f-
@@ -444,7 +444,7 @@ __device__ __forceinline__ void sweep_tile_faces(const SweepArgs &a, double (&s_
       if (item < kItems) {
         const double *fmv = s_f + S::item_fidx(item);
         double nd, dd;
-        Weno<ORDER>::down([&](int m) { return fmv[m * S::kStrideL]; }, nd, dd);
+        Weno<ORDER, true>::down([&](int m) { return fmv[m * S::kStrideL]; }, nd, dd);
         nu[k] = weno_combine(nu[k], du[k], nd, dd);
       }
     }
@@ -478,8 +478,8 @@ __device__ __forceinline__ void sweep_tile_faces(const SweepArgs &a, double (&s_
         M::template flux<DAX, QUIRK>(u, pl, a, q, f);
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
-          fp[v] = 0.5 * (f[v] + u[v]);
-          fm[v] = 0.5 * (f[v] - u[v]);
+          fp[v] = f[v] + u[v];  // doubled
+          fm[v] = f[v] - u[v];
         }
       } else {
 #pragma unroll
@@ -501,7 +501,7 @@ __device__ __forceinline__ void sweep_tile_faces(const SweepArgs &a, double (&s_
       if (item < kItems) {
         const double *fpv = s_f + S::item_fidx(item);
         const double *fmv = fpv + NV * TLH * TC;
-        face[k] = Weno<ORDER>::face([&](int m) { return fpv[m * S::kStrideL]; },
+        face[k] = Weno<ORDER, true>::face([&](int m) { return fpv[m * S::kStrideL]; },
                                     [&](int m) { return fmv[m * S::kStrideL]; });
       }
     }
@@ -571,8 +571,8 @@ __global__ __launch_bounds__(kThreads) void k_sweep(SweepArgs a) {
           M::template flux<DAX, QUIRK>(u, pl, a, q, f);
   #pragma unroll
           for (int v = 0; v < NV; ++v) {
-            fp[v] = 0.5 * (f[v] + u[v]);
-            fm_keep[cp][v] = 0.5 * (f[v] - u[v]);
+            fp[v] = f[v] + u[v];  // doubled
+            fm_keep[cp][v] = f[v] - u[v];
           }
         } else {
   #pragma unroll
@@ -597,7 +597,7 @@ __global__ __launch_bounds__(kThreads) void k_sweep(SweepArgs a) {
       const unsigned item = tid + k * kThreads;
       if (item < kItems) {
         const double *fpv = s_f + S::item_fidx(item);
-        Weno<ORDER>::up([&](int m) { return fpv[m * S::kStrideL]; }, nu[k], du[k]);
+        Weno<ORDER, true>::up([&](int m) { return fpv[m * S::kStrideL]; }, nu[k], du[k]);
       }
     }
     __syncthreads();
@@ -618,7 +618,7 @@ __global__ __launch_bounds__(kThreads) void k_sweep(SweepArgs a) {
       if (item < kItems) {
         const double *fmv = s_f + S::item_fidx(item);
         double nd, dd;
-        Weno<ORDER>::down([&](int m) { return fmv[m * S::kStrideL]; }, nd, dd);
+        Weno<ORDER, true>::down([&](int m) { return fmv[m * S::kStrideL]; }, nd, dd);
         nu[k] = weno_combine(nu[k], du[k], nd, dd);
       }
     }
@@ -650,8 +650,8 @@ __global__ __launch_bounds__(kThreads) void k_sweep(SweepArgs a) {
         M::template flux<DAX, QUIRK>(u, pl, a, q, f);
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
-          fp[v] = 0.5 * (f[v] + u[v]);
-          fm[v] = 0.5 * (f[v] - u[v]);
+          fp[v] = f[v] + u[v];  // doubled
+          fm[v] = f[v] - u[v];
         }
       } else {
 #pragma unroll
@@ -673,7 +673,7 @@ __global__ __launch_bounds__(kThreads) void k_sweep(SweepArgs a) {
       if (item < kItems) {
         const double *fpv = s_f + S::item_fidx(item);
         const double *fmv = fpv + NV * TLH * TC;
-        face[k] = Weno<ORDER>::face([&](int m) { return fpv[m * S::kStrideL]; },
+        face[k] = Weno<ORDER, true>::face([&](int m) { return fpv[m * S::kStrideL]; },
                                     [&](int m) { return fmv[m * S::kStrideL]; });
       }
     }
@@ -694,7 +694,7 @@ __global__ __launch_bounds__(kThreads) void k_sweep(SweepArgs a) {
   CellC2P cs;
   if (live) {
     const long long q = base_e + (long long)gd * g.stride[DAX] + (long long)gc * g.stride[CAX];
-    const double inv_d = g.inv_d[DAX];
+    const double inv_d = g.half_inv_d[DAX];
     // net flux of this axis, added to the earlier axes' as one fused
     // multiply-add so every kernel that accumulates it rounds alike
     double fn[NV];
@@ -782,7 +782,7 @@ __global__ __launch_bounds__(kThreads, M::NC > 9 ? 1 : 4) void k_sweep_yzf(Sweep
     if (live) {
 #pragma unroll
       for (int v = 0; v < NV; ++v)
-        acc[v] = fma(s_f[SY::gidx(v, r + 1, c)] - s_f[SY::gidx(v, r, c)], g.inv_d[1],
+        acc[v] = fma(s_f[SY::gidx(v, r + 1, c)] - s_f[SY::gidx(v, r, c)], g.half_inv_d[1],
                      __builtin_nontemporal_load(&a.fnet[v * vs + q]));  // read once
     }
     __syncthreads();  // every y face is read before the z phase refills LDS
@@ -801,7 +801,7 @@ __global__ __launch_bounds__(kThreads, M::NC > 9 ? 1 : 4) void k_sweep_yzf(Sweep
       double fn[NV];
 #pragma unroll
       for (int v = 0; v < NV; ++v)
-        fn[v] = fma(s_f[SZ::gidx(v, c + 1, r)] - s_f[SZ::gidx(v, c, r)], g.inv_d[2], acc[v]);
+        fn[v] = fma(s_f[SZ::gidx(v, c + 1, r)] - s_f[SZ::gidx(v, c, r)], g.half_inv_d[2], acc[v]);
       sweep_apply<M, MODE>(a, q, fn, cs);
     }
   } else {
@@ -814,7 +814,7 @@ __global__ __launch_bounds__(kThreads, M::NC > 9 ? 1 : 4) void k_sweep_yzf(Sweep
       if (live && cg >= 0 && cg < kGroup) {
 #pragma unroll
         for (int v = 0; v < NV; ++v)
-          s_acc[v][tid] = fma(s_f[SY::gidx(v, r + 1, cg)] - s_f[SY::gidx(v, r, cg)], g.inv_d[1], a.fnet[v * vs + q]);
+          s_acc[v][tid] = fma(s_f[SY::gidx(v, r + 1, cg)] - s_f[SY::gidx(v, r, cg)], g.half_inv_d[1], a.fnet[v * vs + q]);
       }
       __syncthreads();  // every face is read before LDS is refilled
       __builtin_amdgcn_sched_barrier(0);
@@ -828,7 +828,7 @@ __global__ __launch_bounds__(kThreads, M::NC > 9 ? 1 : 4) void k_sweep_yzf(Sweep
       if (live && rg >= 0 && rg < kGroup) {
 #pragma unroll
         for (int v = 0; v < NV; ++v)
-          s_acc[v][tid] = fma(s_f[SZ::gidx(v, c + 1, rg)] - s_f[SZ::gidx(v, c, rg)], g.inv_d[2], s_acc[v][tid]);
+          s_acc[v][tid] = fma(s_f[SZ::gidx(v, c + 1, rg)] - s_f[SZ::gidx(v, c, rg)], g.half_inv_d[2], s_acc[v][tid]);
       }
       __syncthreads();
       __builtin_amdgcn_sched_barrier(0);
@@ -890,7 +890,7 @@ __global__ __launch_bounds__(kThreads) void k_sweep_xyf(SweepArgs a) {
     const int rg = r - h * GX;
     if (live && rg >= 0 && rg < GX) {
 #pragma unroll
-      for (int v = 0; v < NV; ++v) s_acc[v][tid] = (s_f[SY::gidx(v, c + 1, rg)] - s_f[SY::gidx(v, c, rg)]) * g.inv_d[1];
+      for (int v = 0; v < NV; ++v) s_acc[v][tid] = (s_f[SY::gidx(v, c + 1, rg)] - s_f[SY::gidx(v, c, rg)]) * g.half_inv_d[1];
     }
     __syncthreads();  // every face is read before LDS is refilled
     __builtin_amdgcn_sched_barrier(0);
@@ -904,7 +904,7 @@ __global__ __launch_bounds__(kThreads) void k_sweep_xyf(SweepArgs a) {
       double fn[NV];
 #pragma unroll
       for (int v = 0; v < NV; ++v)
-        fn[v] = fma(s_f[SX::gidx(v, r + 1, c)] - s_f[SX::gidx(v, r, c)], g.inv_d[0], s_acc[v][tid]);
+        fn[v] = fma(s_f[SX::gidx(v, r + 1, c)] - s_f[SX::gidx(v, r, c)], g.half_inv_d[0], s_acc[v][tid]);
       sweep_apply<M, MODE>(a, q, fn, cs);
     }
   } else {
@@ -916,7 +916,7 @@ __global__ __launch_bounds__(kThreads) void k_sweep_xyf(SweepArgs a) {
       if (live && cg >= 0 && cg < GY) {
 #pragma unroll
         for (int v = 0; v < NV; ++v)
-          s_acc[v][tid] = fma(s_f[SX::gidx(v, r + 1, cg)] - s_f[SX::gidx(v, r, cg)], g.inv_d[0], s_acc[v][tid]);
+          s_acc[v][tid] = fma(s_f[SX::gidx(v, r + 1, cg)] - s_f[SX::gidx(v, r, cg)], g.half_inv_d[0], s_acc[v][tid]);
       }
       __syncthreads();
       __builtin_amdgcn_sched_barrier(0);
@@ -958,8 +958,8 @@ __device__ __forceinline__ void split_cell(const SweepArgs &a, long long q, doub
   M::template flux<DIR, QUIRK>(u, pl, a, q, f);
 #pragma unroll
   for (int v = 0; v < M::NC; ++v) {
-    fp[v] = 0.5 * (f[v] + u[v]);
-    fm[v] = 0.5 * (f[v] - u[v]);
+    fp[v] = f[v] + u[v];  // doubled
+    fm[v] = f[v] - u[v];
   }
 }
 
@@ -1012,7 +1012,7 @@ __global__ __launch_bounds__(kThreads) void k_sweep_yz(SweepArgs a) {
       const int rr = idx / (TZT + 1), lf = idx - rr * (TZT + 1);
       const double *fpv = s_f + (v * TYT + rr) * WZ + lf;
       const double *fmv = s_f + ((NV + v) * TYT + rr) * WZ + lf;
-      face_z[k] = Weno<ORDER>::face([&](int m) { return fpv[m]; }, [&](int m) { return fmv[m]; });
+      face_z[k] = Weno<ORDER, true>::face([&](int m) { return fpv[m]; }, [&](int m) { return fmv[m]; });
     }
     __builtin_amdgcn_sched_barrier(0);  // keep the passes from piling up their LDS reads
   }
@@ -1032,7 +1032,7 @@ __global__ __launch_bounds__(kThreads) void k_sweep_yz(SweepArgs a) {
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
       const double *gf = s_f + (v * TYT + r) * (TZT + 1) + c;
-      a.fnet[v * vs + q] = (gf[1] - gf[0]) * g.inv_d[2];
+      a.fnet[v * vs + q] = (gf[1] - gf[0]) * g.half_inv_d[2];
     }
   }
   __syncthreads();
@@ -1067,7 +1067,7 @@ __global__ __launch_bounds__(kThreads) void k_sweep_yz(SweepArgs a) {
       const int lf = idx / TZT, cc = idx - lf * TZT;
       const double *fpv = s_f + (v * HY + lf) * TZT + cc;
       const double *fmv = s_f + ((NV + v) * HY + lf) * TZT + cc;
-      face_y[k] = Weno<ORDER>::face([&](int m) { return fpv[m * TZT]; }, [&](int m) { return fmv[m * TZT]; });
+      face_y[k] = Weno<ORDER, true>::face([&](int m) { return fpv[m * TZT]; }, [&](int m) { return fmv[m * TZT]; });
     }
     __builtin_amdgcn_sched_barrier(0);  // keep the passes from piling up their LDS reads
   }
@@ -1083,7 +1083,7 @@ __global__ __launch_bounds__(kThreads) void k_sweep_yz(SweepArgs a) {
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
     const double *gf = s_f + (v * (TYT + 1) + r) * TZT + c;
-    a.fnet[v * vs + q] = fma(gf[TZT] - gf[0], g.inv_d[1], a.fnet[v * vs + q]);
+    a.fnet[v * vs + q] = fma(gf[TZT] - gf[0], g.half_inv_d[1], a.fnet[v * vs + q]);
   }
 }
 

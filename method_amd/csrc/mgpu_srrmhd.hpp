@@ -78,10 +78,9 @@ __device__ __forceinline__ void srrmhd_flux(const double u[14], double rho, doub
                                             double gam, double sigma, double f[14]) {
   const double Bx = u[5], By = u[6], Bz = u[7], Ex = u[8], Ey = u[9], Ez = u[10];
   const double v2 = vx * vx + vy * vy + vz * vz;
-  const double W = 1.0 / sqrt(1.0 - v2);
-  const double e = p / (rho * (gam - 1.0));
-  const double h = 1.0 + e * gam;
-  const double Z = rho * h * W * W;
+  const double W = rsqrt_pos(1.0 - v2);
+  // rho h with h = 1 + gam e, e = p / (rho (gam - 1))
+  const double Z = fma(p, gam * rcp_pos(gam - 1.0), rho) * W * W;
   const double hs = 0.5 * (Bx * Bx + By * By + Bz * Bz + Ex * Ex + Ey * Ey + Ez * Ez);
   const double vE = vx * Ex + vy * Ey + vz * Ez;
   const double q = u[13];
@@ -102,25 +101,31 @@ __device__ __forceinline__ void srrmhd_flux_stored(const double u[14], const dou
   srrmhd_flux_core<DIR, QUIRK>(u, P[1], P[2], P[3], P[4], A[10], 0.5 * (A[7] + A[8]), A[4 + DIR], f);
 }
 
-// Residual of the recovery equation in Z = rho h W^2 (srrmhd.cc:512-537).
-__device__ __forceinline__ double srrmhd_c2p_residual(double Z, double SbSq, double D, double tauBar, double gam) {
-  const double vsq = SbSq / (Z * Z);
-  if (vsq >= 1.0 || Z < 0) return 1.0e6;
-  const double W = 1.0 / sqrt(1.0 - vsq);
-  const double rho = D / W;
-  const double h = Z / (rho * W * W);
-  const double p = (gam - 1.0) * (h - rho) / gam;
-  if (rho < 0 || p < 0 || W < 1 || h < 0) return 1.0e6;
-  return (1.0 - (gam - 1.0) / (W * W * gam)) * Z + ((gam - 1.0) / (W * gam) - 1.0) * D - tauBar;
+// Residual of the recovery equation in Z = rho h W^2 (srrmhd.cc:512-537), with
+// gf = (gam - 1) / gam and iD = 1 / D: v^2 = Sbar^2 / Z^2, 1 / W^2 = 1 - v^2,
+// rho = D / W and h = Z / (rho W^2) = Z / (D W).
+__device__ __forceinline__ double srrmhd_c2p_residual(double Z, double SbSq, double D, double tauBar, double gf,
+                                                      double iD) {
+  const double iZ = rcp_pos(Z);
+  const double vsq = SbSq * iZ * iZ;
+  if (!(vsq < 1.0) || Z < 0) return 1.0e6;
+  const double s = 1.0 - vsq;
+  const double iW = s * rsqrt_pos(s);
+  const double rho = D * iW;
+  const double h = Z * iD * iW;
+  const double p = gf * (h - rho);
+  if (rho < 0 || p < 0 || h < 0) return 1.0e6;
+  return (1.0 - gf * s) * Z + (gf * iW - 1.0) * D - tauBar;
 }
 
 // The reference's secant iteration on Z (srrmhd.cc:539-581): first step 1e-4,
 // stop at |residual| < 1e-12, at most 50 iterations; returns iterations or -1
 // (Z then holds the best iterate).
 __device__ __forceinline__ int srrmhd_secant(double &Z, double SbSq, double D, double tauBar, double gam) {
+  const double gf = (gam - 1.0) * rcp_pos(gam), iD = 1.0 / D;
   double x0 = Z, x1 = x0 + 1.0e-4;
-  double f0 = srrmhd_c2p_residual(x0, SbSq, D, tauBar, gam);
-  double f1 = srrmhd_c2p_residual(x1, SbSq, D, tauBar, gam);
+  double f0 = srrmhd_c2p_residual(x0, SbSq, D, tauBar, gf, iD);
+  double f1 = srrmhd_c2p_residual(x1, SbSq, D, tauBar, gf, iD);
   double bestX = x0, bestF = f0;
   for (int it = 0; it < 50; ++it) {
     if (fabs(f0) < 1.0e-12) {
@@ -131,7 +136,7 @@ __device__ __forceinline__ int srrmhd_secant(double &Z, double SbSq, double D, d
     x1 = x0;
     x0 = x2;
     f1 = f0;
-    f0 = srrmhd_c2p_residual(x0, SbSq, D, tauBar, gam);
+    f0 = srrmhd_c2p_residual(x0, SbSq, D, tauBar, gf, iD);
     if (fabs(f0) < fabs(bestF)) {
       bestX = x0;
       bestF = f0;
@@ -166,14 +171,14 @@ __device__ __forceinline__ void srrmhd_recover(const double u[14], double gam, d
   P[10] = u[10];
   srrmhd_aux_of_cons(u, A);
   A[10] = Z;
-  A[9] = A[15] / (Z * Z);
-  A[1] = 1.0 / sqrt(1.0 - A[9]);
-  P[0] = u[0] / A[1];
-  A[0] = Z / (P[0] * A[1] * A[1]);
-  A[2] = (A[0] - 1.0) / gam;
+  const double iZ = rcp_pos(Z);
+  A[9] = A[15] * iZ * iZ;
+  A[1] = rsqrt_pos(1.0 - A[9]);
+  P[0] = u[0] * ((1.0 - A[9]) * A[1]);
+  A[0] = div_pos(Z, P[0] * A[1] * A[1]);
+  A[2] = (A[0] - 1.0) * rcp_pos(gam);
   A[3] = sqrt((A[2] * gam * (gam - 1.0)) / A[0]);
   P[4] = P[0] * A[2] * (gam - 1.0);
-  const double iZ = 1.0 / Z;
   P[1] = A[12] * iZ;
   P[2] = A[13] * iZ;
   P[3] = A[14] * iZ;
@@ -272,12 +277,13 @@ __device__ __forceinline__ bool imex_residual(const double c[14], double dtg, do
   const double Sbz = c[3] - (Ex * By - Ey * Bx);
   const double tauBar = c[4] - 0.5 * (Bx * Bx + By * By + Bz * Bz + Ex * Ex + Ey * Ey + Ez * Ez);
   if (!(Z > 0.0)) return false;
-  const double iZ = 1.0 / Z;
+  const double iZ = rcp_pos(Z);
   const double vx = Sbx * iZ, vy = Sby * iZ, vz = Sbz * iZ;
   const double vsq = vx * vx + vy * vy + vz * vz;
   if (!(vsq < 1.0)) return false;
-  const double W = 1.0 / sqrt(1.0 - vsq);
-  F[3] = (1.0 - (gam - 1.0) / (W * W * gam)) * Z + ((gam - 1.0) / (W * gam) - 1.0) * c[0] - tauBar;
+  const double iW2 = 1.0 - vsq, W = rsqrt_pos(iW2), iW = iW2 * W;
+  const double gf = (gam - 1.0) * rcp_pos(gam);
+  F[3] = (1.0 - gf * iW2) * Z + (gf * iW - 1.0) * c[0] - tauBar;
   const double vE = vx * Ex + vy * Ey + vz * Ez;
   const double q = c[13], ws = W * sigma;
   F[0] = Ex - c[8] + dtg * (q * vx + ws * (Ex + (vy * Bz - vz * By) - vE * vx));
@@ -302,12 +308,13 @@ __device__ __forceinline__ bool imex_residual_jac(const double c[14], double dtg
   const double Sbz = c[3] - (Ex * By - Ey * Bx);
   const double tauBar = c[4] - 0.5 * (Bx * Bx + By * By + Bz * Bz + Ex * Ex + Ey * Ey + Ez * Ez);
   if (!(Z > 0.0)) return false;
-  const double iZ = 1.0 / Z;
+  const double iZ = rcp_pos(Z);
   const double vx = Sbx * iZ, vy = Sby * iZ, vz = Sbz * iZ;
   const double vsq = vx * vx + vy * vy + vz * vz;
   if (!(vsq < 1.0)) return false;
-  const double W = 1.0 / sqrt(1.0 - vsq);
-  F[3] = (1.0 - (gam - 1.0) / (W * W * gam)) * Z + ((gam - 1.0) / (W * gam) - 1.0) * c[0] - tauBar;
+  const double iW2 = 1.0 - vsq, W = rsqrt_pos(iW2), iW = iW2 * W;
+  const double gf = (gam - 1.0) * rcp_pos(gam);
+  F[3] = (1.0 - gf * iW2) * Z + (gf * iW - 1.0) * c[0] - tauBar;
   const double vE = vx * Ex + vy * Ey + vz * Ez;
   const double q = c[13], ws = W * sigma;
   const double G[3] = {Ex + (vy * Bz - vz * By) - vE * vx, Ey + (vz * Bx - vx * Bz) - vE * vy,
@@ -318,15 +325,15 @@ __device__ __forceinline__ bool imex_residual_jac(const double c[14], double dtg
   const double v[3] = {vx, vy, vz}, E[3] = {Ex, Ey, Ez};
   // dSb/dE_k: columns (0, Bz, -By), (-Bz, 0, Bx), (By, -Bx, 0)
   const double dSb[3][3] = {{0.0, -Bz, By}, {Bz, 0.0, -Bx}, {-By, Bx, 0.0}};  // [component][k]
-  const double g = gam - 1.0, W2 = W * W, W3 = W2 * W;
-  const double cW = 2.0 * g / (W3 * gam) * Z - g / (W2 * gam) * c[0];  // dF_Z/dW
+  const double W3 = W * W * W;
+  const double cW = gf * iW2 * (2.0 * iW * Z - c[0]);  // dF_Z/dW
 #pragma unroll
   for (int a = 0; a < 4; ++a) {
     double dv[3];
 #pragma unroll
     for (int i = 0; i < 3; ++i) dv[i] = a < 3 ? dSb[i][a] * iZ : -v[i] * iZ;
     const double dW = W3 * (v[0] * dv[0] + v[1] * dv[1] + v[2] * dv[2]);
-    J[3][a] = cW * dW + (a == 3 ? 1.0 - g / (W2 * gam) : E[a]);
+    J[3][a] = cW * dW + (a == 3 ? 1.0 - gf * iW2 : E[a]);
     const double dvE = dv[0] * E[0] + dv[1] * E[1] + dv[2] * E[2] + (a < 3 ? v[a] : 0.0);
     const double dvxB[3] = {dv[1] * Bz - dv[2] * By, dv[2] * Bx - dv[0] * Bz, dv[0] * By - dv[1] * Bx};
 #pragma unroll
@@ -342,7 +349,7 @@ __device__ __forceinline__ bool imex_residual_jac(const double c[14], double dtg
 // the physical region are halved. Returns iterations or -1. The residual and Jacobian
 // the step search forms at the accepted point serve the next iteration.
 __device__ __forceinline__ int imex_solve(const double c[14], double dtg, double gam, double sigma, double y[4]) {
-  double F[4], J[4][4], M[4][5], dprev = HUGE_VAL;
+  double F[4], J[4][4], M[4][5], inv[4], dprev = HUGE_VAL;
   if (!imex_residual_jac(c, dtg, gam, sigma, y, F, J)) return -1;
   for (int it = 0; it < 60; ++it) {
 #pragma unroll
@@ -365,10 +372,10 @@ __device__ __forceinline__ int imex_solve(const double c[14], double dtg, double
         }
       }
       if (M[k][k] == 0.0) return -1;
-      const double inv = 1.0 / M[k][k];
+      inv[k] = rcp_pos(M[k][k]);
 #pragma unroll
       for (int i = k + 1; i < 4; ++i) {
-        const double m = M[i][k] * inv;
+        const double m = M[i][k] * inv[k];
 #pragma unroll
         for (int j = k; j < 5; ++j) M[i][j] -= m * M[k][j];
       }
@@ -379,7 +386,7 @@ __device__ __forceinline__ int imex_solve(const double c[14], double dtg, double
       double s = M[k][4];
 #pragma unroll
       for (int j = k + 1; j < 4; ++j) s -= M[k][j] * d[j];
-      d[k] = s / M[k][k];
+      d[k] = s * inv[k];
     }
     double ymax = 1.0, dmax = 0.0;
 #pragma unroll
