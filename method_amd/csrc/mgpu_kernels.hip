@@ -9,6 +9,7 @@
 // applies the stage update and the per-cell Newton cons2prim, so the stage's
 // new cons and prims leave the kernel without another pass over HBM.
 #include "mgpu_kernels.hpp"
+#include "mgpu_tile.hpp"
 
 #include <hip/hip_runtime.h>
 
@@ -17,8 +18,6 @@
 namespace mgpu {
 
 namespace {
-
-constexpr int kThreads = 256;
 
 // Block-level reduction of C2P counters into one of the stats buckets.
 __device__ __forceinline__ void reduce_stats(C2PCounters *st, int cells, int iters, int fails, int maxit) {
@@ -63,7 +62,7 @@ struct SrmhdM {
   static constexpr int P0 = 1, NPL = 4;  // vx, vy, vz, p
   static constexpr bool kStored = false;
   template <int DIR, bool Q>
-  __device__ __forceinline__ static void flux(const double *u, const double *pl, const SweepArgs &, long long,
+  __device__ __forceinline__ static void flux(const double *u, const double *pl, const SweepArgs &, unsigned,
                                               double *f) {
     srmhd_flux<DIR, Q>(u, pl[0], pl[1], pl[2], pl[3], f);
   }
@@ -74,7 +73,7 @@ struct SrrmhdM {
   static constexpr int P0 = 0, NPL = 5;  // rho, vx, vy, vz, p
   static constexpr bool kStored = false;
   template <int DIR, bool Q>
-  __device__ __forceinline__ static void flux(const double *u, const double *pl, const SweepArgs &a, long long,
+  __device__ __forceinline__ static void flux(const double *u, const double *pl, const SweepArgs &a, unsigned,
                                               double *f) {
     srrmhd_flux<DIR, Q>(u, pl[0], pl[1], pl[2], pl[3], pl[4], a.gamma, a.sigma, f);
   }
@@ -87,12 +86,12 @@ struct StoredM {
   static constexpr int P0 = 0, NPL = 1;
   static constexpr bool kStored = true;
   template <int DIR, bool Q>
-  __device__ __forceinline__ static void flux(const double *, const double *, const SweepArgs &a, long long q,
+  __device__ __forceinline__ static void flux(const double *, const double *, const SweepArgs &a, unsigned o,
                                               double *f) {
     const long long vs = a.geo.vstride;
     const double *F = a.Fin + (long long)DIR * NC * vs;
 #pragma unroll
-    for (int v = 0; v < NC; ++v) f[v] = F[v * vs + q];
+    for (int v = 0; v < NC; ++v) f[v] = F[v * vs + o / 8];
   }
 };
 
@@ -169,17 +168,22 @@ struct SweepShape {
     return DFAST ? (v * TC + c) * (TL + 1) + lf : (v * (TL + 1) + lf) * TC + c;
   }
   static constexpr int kStrideL = DFAST ? 1 : TC;  // LDS step between neighbouring cells of a pencil
-  // fidx(v, lf, cc) of work item v * kFaces + idx, idx enumerating (lf, cc) in
-  // gidx order: for the strided layout idx = lf * TC + cc already is the
-  // offset within the variable; for the contiguous one each pencil skips the
-  // 2R - 1 halo slots past its TL + 1 faces.
-  __device__ static unsigned item_fidx(unsigned item) {
-    const unsigned v = item / kFaces;
-    unsigned off = item + v * (unsigned)(TLH * TC - kFaces);
-    if (DFAST) off += (item - v * kFaces) / (TL + 1) * (unsigned)(TLH - TL - 1);
-    return off;
+  // LDS offset within a variable of the first stencil cell of face f = (lf, cc)
+  // in gidx order: f itself for the strided layout, where f = lf * TC + cc;
+  // for the contiguous one each pencil skips the 2R - 1 halo slots past its
+  // TL + 1 faces.
+  __device__ __forceinline__ static unsigned at(unsigned f) {
+    return DFAST ? f + f / (TL + 1) * (unsigned)(TLH - TL - 1) : f;
   }
+  using Items = FaceItems<M::NC, kFaces, TLH * TC, SweepShape>;
 };
+
+// Byte offset of the cell at index d along axis DAX and c along CAX of the
+// plane whose first cell is base.
+template <int DAX, int CAX>
+__device__ __forceinline__ unsigned cell_offset(const Geo &g, unsigned base, int d, int c) {
+  return (base + d * (unsigned)g.stride[DAX] + c * (unsigned)g.stride[CAX]) * 8u;
+}
 
 // Counters of one cell's cons2prim, accumulated over a block.
 struct CellC2P {
@@ -196,15 +200,15 @@ struct CellC2P {
 };
 
 // RK2 stage end for SRMHD: update, Newton C2P, write.
-__device__ __forceinline__ void finish_rk2(const SweepArgs &a, long long q, const double *un, SrmhdM,
+__device__ __forceinline__ void finish_rk2(const SweepArgs &a, unsigned o, const double *un, SrmhdM,
                                            CellC2P &cs) {
   const long long vs = a.geo.vstride;
   double v2, Z;
   // the guess is read once per cell: non-temporal loads keep it from evicting
   // the tiles' halo cells from the L2
-  srmhd_plain_guess(__builtin_nontemporal_load(&a.Vg[0 * vs + q]), __builtin_nontemporal_load(&a.Vg[1 * vs + q]),
-                    __builtin_nontemporal_load(&a.Vg[2 * vs + q]), __builtin_nontemporal_load(&a.Vg[3 * vs + q]),
-                    __builtin_nontemporal_load(&a.Vg[4 * vs + q]), a.gamma, v2, Z);
+  srmhd_plain_guess(ld_nt(a.Vg + 0 * vs, o), ld_nt(a.Vg + 1 * vs, o),
+                    ld_nt(a.Vg + 2 * vs, o), ld_nt(a.Vg + 3 * vs, o),
+                    ld_nt(a.Vg + 4 * vs, o), a.gamma, v2, Z);
   const double BS = un[5] * un[1] + un[6] * un[2] + un[7] * un[3];
   const double Bsq = un[5] * un[5] + un[6] * un[6] + un[7] * un[7];
   const double Ssq = un[1] * un[1] + un[2] * un[2] + un[3] * un[3];
@@ -215,55 +219,55 @@ __device__ __forceinline__ void finish_rk2(const SweepArgs &a, long long q, cons
   // reads them, but they do not fit in the caches and would only evict the
   // tiles' halo cells from the L2)
 #pragma unroll
-  for (int v = 0; v < kSrmhdCons; ++v) __builtin_nontemporal_store(un[v], &a.Uout[v * vs + q]);
+  for (int v = 0; v < kSrmhdCons; ++v) st_nt(a.Uout + v * vs, o, un[v]);
   const int nvout = a.vout_n ? a.vout_n : kSrmhdPrims;
 #pragma unroll
   for (int v = 0; v < kSrmhdPrims; ++v)
-    if (v < nvout) __builtin_nontemporal_store(P[v], &a.Vout[v * vs + q]);
+    if (v < nvout) st_nt(a.Vout + v * vs, o, P[v]);
   if (a.Aout) {
 #pragma unroll
-    for (int v = 0; v < kSrmhdAux; ++v) a.Aout[v * vs + q] = A[v];
+    for (int v = 0; v < kSrmhdAux; ++v) st(a.Aout + v * vs, o, A[v]);
   } else if (a.root) {
-    __builtin_nontemporal_store(v2, &a.root[q]);
-    __builtin_nontemporal_store(Z, &a.root[vs + q]);
+    st_nt(a.root, o, v2);
+    st_nt(a.root + vs, o, Z);
   }
   cs.add(its);
   if (its < 0) {
     const int slot = atomicAdd(a.fail_count, 1);
-    a.fail_list[slot] = q;
-    a.fail_flag[q] = 1;
+    a.fail_list[slot] = o >> 3;
+    a.fail_flag[o >> 3] = 1;
   }
 }
 
 // Cons2prim of a resistive stage value with the secant rule, writing cons,
 // prims and (if requested) aux; returns the recovered aux in A.
-__device__ __forceinline__ void c2p_store_srrmhd(const SweepArgs &a, long long q, const double *un, double *A,
+__device__ __forceinline__ void c2p_store_srrmhd(const SweepArgs &a, unsigned o, const double *un, double *A,
                                                  CellC2P &cs) {
   const long long vs = a.geo.vstride;
-  const double Zg = srrmhd_guess_Z(a.Vg[0 * vs + q], a.Vg[1 * vs + q], a.Vg[2 * vs + q], a.Vg[3 * vs + q],
-                                   a.Vg[4 * vs + q], a.gamma);
+  const double Zg = srrmhd_guess_Z(ld(a.Vg + 0 * vs, o), ld(a.Vg + 1 * vs, o), ld(a.Vg + 2 * vs, o), ld(a.Vg + 3 * vs, o),
+                                   ld(a.Vg + 4 * vs, o), a.gamma);
   double P[kSrrmhdPrims];
   const int its = srrmhd_c2p_cell(un, a.gamma, a.sigma, Zg, P, A);
   // streamed out, as finish_rk2 does for SRMHD
 #pragma unroll
-  for (int v = 0; v < kSrrmhdCons; ++v) __builtin_nontemporal_store(un[v], &a.Uout[v * vs + q]);
+  for (int v = 0; v < kSrrmhdCons; ++v) st_nt(a.Uout + v * vs, o, un[v]);
   const int nvout = a.vout_n ? a.vout_n : kSrrmhdPrims;
 #pragma unroll
   for (int v = 0; v < kSrrmhdPrims; ++v)
-    if (v < nvout) __builtin_nontemporal_store(P[v], &a.Vout[v * vs + q]);
+    if (v < nvout) st_nt(a.Vout + v * vs, o, P[v]);
   if (a.Aout) {
 #pragma unroll
-    for (int v = 0; v < kSrrmhdAux; ++v) a.Aout[v * vs + q] = A[v];
+    for (int v = 0; v < kSrrmhdAux; ++v) st(a.Aout + v * vs, o, A[v]);
   } else if (a.root) {
-    __builtin_nontemporal_store(A[10], &a.root[q]);  // Z: the aux follows from it and the cons (srrmhd_recover)
+    st_nt(a.root, o, A[10]);  // Z: the aux follows from it and the cons (srrmhd_recover)
   }
   cs.add(its);
 }
 
-__device__ __forceinline__ void finish_rk2(const SweepArgs &a, long long q, const double *un, SrrmhdM,
+__device__ __forceinline__ void finish_rk2(const SweepArgs &a, unsigned o, const double *un, SrrmhdM,
                                            CellC2P &cs) {
   double A[kSrrmhdAux];
-  c2p_store_srrmhd(a, q, un, A, cs);
+  c2p_store_srrmhd(a, o, un, A, cs);
 }
 
 // SSP2 stage two at one cell once flux1 is complete (SSP2.cc:112-148): solve
@@ -271,72 +275,72 @@ __device__ __forceinline__ void finish_rk2(const SweepArgs &a, long long q, cons
 // of the final combination known now, U^n - dt/2 flux1 + dt/2 (source1 +
 // source2), so the final sweep reads one array instead of U^n, flux1 and
 // both sources.
-__device__ __forceinline__ void imex2_apply(const SweepArgs &a, long long q, const double *fn, CellC2P &cs) {
+__device__ __forceinline__ void imex2_apply(const SweepArgs &a, unsigned o, const double *fn, CellC2P &cs) {
   const long long vs = a.geo.vstride;
   double c[kSrrmhdCons], pf[kSrrmhdCons], x[kSrrmhdCons], A[kSrrmhdAux], s1[5];
 #pragma unroll
   for (int v = 0; v < kSrrmhdCons; ++v) {
-    const double un = a.Un[v * vs + q];
+    const double un = ld(a.Un + v * vs, o);
     c[v] = un - a.dt * fn[v];
     pf[v] = un - 0.5 * a.dt * fn[v];
   }
 #pragma unroll
   for (int m = 0; m < 5; ++m) {
-    s1[m] = a.S1[m * vs + q];
+    s1[m] = ld(a.S1 + m * vs, o);
     c[8 + m] += a.dt * kSsp2Om2Gam * s1[m];
   }
-  const double Zg = srrmhd_guess_Z(a.Vg[0 * vs + q], a.Vg[1 * vs + q], a.Vg[2 * vs + q], a.Vg[3 * vs + q],
-                                   a.Vg[4 * vs + q], a.gamma);
+  const double Zg = srrmhd_guess_Z(ld(a.Vg + 0 * vs, o), ld(a.Vg + 1 * vs, o), ld(a.Vg + 2 * vs, o), ld(a.Vg + 3 * vs, o),
+                                   ld(a.Vg + 4 * vs, o), a.gamma);
   const int its = imex_stage(c, a.dt, a.gamma, a.sigma, a.cp, Zg, x);
-  c2p_store_srrmhd(a, q, x, A, cs);
+  c2p_store_srrmhd(a, o, x, A, cs);
   if (its < 0) cs.fails = 1;
   double s5[5];
   srrmhd_source5(x, A, a.cp, s5);
 #pragma unroll
   for (int m = 0; m < 5; ++m) pf[8 + m] += 0.5 * a.dt * (s1[m] + s5[m]);
 #pragma unroll
-  for (int v = 0; v < kSrrmhdCons; ++v) __builtin_nontemporal_store(pf[v], &a.Pf[v * vs + q]);
+  for (int v = 0; v < kSrrmhdCons; ++v) st_nt(a.Pf + v * vs, o, pf[v]);
 }
 
 // SSP2's final combination at one cell, cons += -dt/2 (flux1 + flux2 -
 // source1 - source2) (SSP2.cc:156-166), from the part stage two stored, then
 // cons2prim.
-__device__ __forceinline__ void imex_final_apply(const SweepArgs &a, long long q, const double *fn, CellC2P &cs) {
+__device__ __forceinline__ void imex_final_apply(const SweepArgs &a, unsigned o, const double *fn, CellC2P &cs) {
   const long long vs = a.geo.vstride;
   double un[kSrrmhdCons], A[kSrrmhdAux];
 #pragma unroll
-  for (int v = 0; v < kSrrmhdCons; ++v) un[v] = a.Pf[v * vs + q] - 0.5 * a.dt * fn[v];
-  c2p_store_srrmhd(a, q, un, A, cs);
+  for (int v = 0; v < kSrrmhdCons; ++v) un[v] = ld(a.Pf + v * vs, o) - 0.5 * a.dt * fn[v];
+  c2p_store_srrmhd(a, o, un, A, cs);
 }
 
 // Stored-flux sweeps only accumulate the net flux (write and add modes).
 template <class M>
-__device__ __forceinline__ void finish_rk2(const SweepArgs &, long long, const double *, StoredM<M>, CellC2P &) {}
+__device__ __forceinline__ void finish_rk2(const SweepArgs &, unsigned, const double *, StoredM<M>, CellC2P &) {}
 
 // What a sweep does with a cell's net flux fn once its own axis is added
 // (the sweep's mode): keep it for the next sweep, or finish the stage there.
 template <class M, int MODE>
-__device__ __forceinline__ void sweep_apply(const SweepArgs &a, long long q, const double *fn, CellC2P &cs) {
+__device__ __forceinline__ void sweep_apply(const SweepArgs &a, unsigned o, const double *fn, CellC2P &cs) {
   constexpr int NV = M::NC;
   const long long vs = a.geo.vstride;
   if (MODE == kSweepWrite || MODE == kSweepAdd) {
 #pragma unroll
-    for (int v = 0; v < NV; ++v) a.fnet[v * vs + q] = fn[v];
+    for (int v = 0; v < NV; ++v) st(a.fnet + v * vs, o, fn[v]);
   } else if (MODE == kSweepStage1 || MODE == kSweepStage2) {
     double un[NV];
     if (MODE == kSweepStage1) {
 #pragma unroll
-      for (int v = 0; v < NV; ++v) un[v] = rk2_stage1(a.U[v * vs + q], fn[v], a.dt);
+      for (int v = 0; v < NV; ++v) un[v] = rk2_stage1(ld(a.U + v * vs, o), fn[v], a.dt);
     } else {
 #pragma unroll
       for (int v = 0; v < NV; ++v)
-        un[v] = rk2_stage2(__builtin_nontemporal_load(&a.Un[v * vs + q]), a.U[v * vs + q], fn[v], a.dt);
+        un[v] = rk2_stage2(ld_nt(a.Un + v * vs, o), ld(a.U + v * vs, o), fn[v], a.dt);
     }
-    finish_rk2(a, q, un, M(), cs);
+    finish_rk2(a, o, un, M(), cs);
   } else if (MODE == kSweepImex2) {
-    imex2_apply(a, q, fn, cs);
+    imex2_apply(a, o, fn, cs);
   } else if (MODE == kSweepImexFinal) {
-    imex_final_apply(a, q, fn, cs);
+    imex_final_apply(a, o, fn, cs);
   }
 }
 
@@ -350,7 +354,7 @@ __device__ __forceinline__ void sweep_apply(const SweepArgs &a, long long q, con
 template <class M, int ORDER, int DAX, int CAX, bool DFAST, int TL_, int TC_, bool QUIRK, bool SPLIT_ALL = false,
           int NLDS>
 __device__ __forceinline__ void sweep_tile_faces(const SweepArgs &a, double (&s_f)[NLDS], int d0, int c0,
-                                                 long long base_e, int nd, int nc, unsigned tid) {
+                                                 unsigned base_e, int nd, int nc, unsigned tid) {
   using S = SweepShape<M, ORDER, DAX, CAX, DFAST, TL_, TC_, SPLIT_ALL>;
   constexpr int R = S::R, TC = S::TC, TLH = S::TLH;
   constexpr int NV = M::NC;
@@ -371,28 +375,26 @@ __device__ __forceinline__ void sweep_tile_faces(const SweepArgs &a, double (&s_
       if (idx < kCells) {
         const int l = DFAST ? idx % TLH : idx / TC;
         const int cc = DFAST ? idx / TLH : idx % TC;
-        const int gc = c0 + cc;
+        // a pencil past the grid takes the last one's cells; nothing reads its faces
+        const int gc = min(c0 + cc, nc - 1);
         double fp[NV];
-        if (gc < nc) {
+        {
           // cells past nd + R - 1 only feed faces outside the grid; clamping
           // them keeps the periodic image inside [0, nd) for any tile overhang
           const int gd = remap(min(d0 + l - R, nd - 1 + R), nd, g.periodic[DAX]);
-          const long long q = base_e + (long long)gd * g.stride[DAX] + (long long)gc * g.stride[CAX];
+          const unsigned o = cell_offset<DAX, CAX>(g, base_e, gd, gc);
           double u[NV], pl[M::NPL];
   #pragma unroll
-          for (int v = 0; v < NV; ++v) u[v] = a.U[v * vs + q];
+          for (int v = 0; v < NV; ++v) u[v] = ld(a.U + v * vs, o);
   #pragma unroll
-          for (int v = 0; v < M::NPL; ++v) pl[v] = a.V[(M::P0 + v) * vs + q];
+          for (int v = 0; v < M::NPL; ++v) pl[v] = ld(a.V + (M::P0 + v) * vs, o);
           double f[NV];
-          M::template flux<DAX, QUIRK>(u, pl, a, q, f);
+          M::template flux<DAX, QUIRK>(u, pl, a, o, f);
   #pragma unroll
           for (int v = 0; v < NV; ++v) {
             fp[v] = f[v] + u[v];  // doubled
             fm_keep[cp][v] = f[v] - u[v];
           }
-        } else {
-  #pragma unroll
-          for (int v = 0; v < NV; ++v) fp[v] = fm_keep[cp][v] = 0.0;
         }
   #pragma unroll
         for (int v = 0; v < NV; ++v) s_f[S::fidx(v, l, cc)] = fp[v];
@@ -406,20 +408,18 @@ __device__ __forceinline__ void sweep_tile_faces(const SweepArgs &a, double (&s_
     __syncthreads();
 
     // Phase 2: WENO face values, face lf being the left face of tile cell lf.
-    // The (variable, face) pairs are dealt out one per thread per pass, so the
-    // faces beyond one per thread cost a fraction of a pass spread over the
-    // waves instead of a full pass of all variables on one wave. Upwind halves
-    // from f+ first, then downwind halves from f-.
-    constexpr int kItems = NV * S::kFaces;
-    constexpr int kPasses = (kItems + kThreads - 1) / kThreads;
+    // The (variable, face) pairs go to the threads as FaceItems says. Upwind
+    // halves from f+ first, then downwind halves from f-.
+    const typename S::Items items(tid);
+    constexpr int kPasses = S::Items::kPasses;
     double nu[kPasses], du[kPasses];
   #pragma unroll
     for (int k = 0; k < kPasses; ++k) {
-      const unsigned item = tid + k * kThreads;
-      if (item < kItems) {
-        const double *fpv = s_f + S::item_fidx(item);
+      if (items.has(k)) {
+        const double *fpv = s_f + items.lds(k);
         Weno<ORDER, true>::up([&](int m) { return fpv[m * S::kStrideL]; }, nu[k], du[k]);
       }
+      if (S::Items::kRegular) pass_end(nu[k], du[k]);
     }
     // the upwind halves are formed here, before the barrier after which f-
     // overwrites f+: left to itself the compiler keeps the loaded f+ stencils
@@ -440,23 +440,22 @@ __device__ __forceinline__ void sweep_tile_faces(const SweepArgs &a, double (&s_
     __syncthreads();
   #pragma unroll
     for (int k = 0; k < kPasses; ++k) {
-      const unsigned item = tid + k * kThreads;
-      if (item < kItems) {
-        const double *fmv = s_f + S::item_fidx(item);
+      if (items.has(k)) {
+        const double *fmv = s_f + items.lds(k);
         double nd, dd;
         Weno<ORDER, true>::down([&](int m) { return fmv[m * S::kStrideL]; }, nd, dd);
         nu[k] = weno_combine(nu[k], du[k], nd, dd);
       }
+      if (S::Items::kRegular) pass_end(nu[k]);
     }
 #pragma unroll
     for (int k = 0; k < kPasses; ++k) asm volatile("" : "+v"(nu[k]));
     __syncthreads();
-    // item = v * kFaces + idx, idx enumerating (lf, cc) in gidx order for both
-    // layouts, so the face of item goes to s_f[item]
+    // an item's place v * kFaces + f, f enumerating (lf, cc) in gidx order for
+    // both layouts, is its face's place in s_f
   #pragma unroll
     for (int k = 0; k < kPasses; ++k) {
-      const unsigned item = tid + k * kThreads;
-      if (item < kItems) s_f[item] = nu[k];
+      if (items.has(k)) s_f[items.item(k)] = nu[k];
     }
     __syncthreads();
   } else {
@@ -464,26 +463,23 @@ __device__ __forceinline__ void sweep_tile_faces(const SweepArgs &a, double (&s_
     for (unsigned idx = tid; idx < TLH * TC; idx += kThreads) {
       const int l = DFAST ? idx % TLH : idx / TC;
       const int cc = DFAST ? idx / TLH : idx % TC;
-      const int gc = c0 + cc;
+      const int gc = min(c0 + cc, nc - 1);
       double fp[NV], fm[NV];
-      if (gc < nc) {
+      {
         const int gd = remap(min(d0 + l - R, nd - 1 + R), nd, g.periodic[DAX]);
-        const long long q = base_e + (long long)gd * g.stride[DAX] + (long long)gc * g.stride[CAX];
+        const unsigned o = cell_offset<DAX, CAX>(g, base_e, gd, gc);
         double u[NV], pl[M::NPL];
 #pragma unroll
-        for (int v = 0; v < NV; ++v) u[v] = a.U[v * vs + q];
+        for (int v = 0; v < NV; ++v) u[v] = ld(a.U + v * vs, o);
 #pragma unroll
-        for (int v = 0; v < M::NPL; ++v) pl[v] = a.V[(M::P0 + v) * vs + q];
+        for (int v = 0; v < M::NPL; ++v) pl[v] = ld(a.V + (M::P0 + v) * vs, o);
         double f[NV];
-        M::template flux<DAX, QUIRK>(u, pl, a, q, f);
+        M::template flux<DAX, QUIRK>(u, pl, a, o, f);
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
           fp[v] = f[v] + u[v];  // doubled
           fm[v] = f[v] - u[v];
         }
-      } else {
-#pragma unroll
-        for (int v = 0; v < NV; ++v) fp[v] = fm[v] = 0.0;
       }
 #pragma unroll
       for (int v = 0; v < NV; ++v) {
@@ -492,24 +488,23 @@ __device__ __forceinline__ void sweep_tile_faces(const SweepArgs &a, double (&s_
       }
     }
     __syncthreads();
-    constexpr int kItems = NV * S::kFaces;
-    constexpr int kPasses = (kItems + kThreads - 1) / kThreads;
+    const typename S::Items items(tid);
+    constexpr int kPasses = S::Items::kPasses;
     double face[kPasses];
 #pragma unroll
     for (int k = 0; k < kPasses; ++k) {
-      const unsigned item = tid + k * kThreads;
-      if (item < kItems) {
-        const double *fpv = s_f + S::item_fidx(item);
+      if (items.has(k)) {
+        const double *fpv = s_f + items.lds(k);
         const double *fmv = fpv + NV * TLH * TC;
         face[k] = Weno<ORDER, true>::face([&](int m) { return fpv[m * S::kStrideL]; },
                                     [&](int m) { return fmv[m * S::kStrideL]; });
       }
+      if (S::Items::kRegular) pass_end(face[k]);
     }
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < kPasses; ++k) {
-      const unsigned item = tid + k * kThreads;
-      if (item < kItems) s_f[item] = face[k];
+      if (items.has(k)) s_f[items.item(k)] = face[k];
     }
     __syncthreads();
   }
@@ -537,7 +532,7 @@ __global__ __launch_bounds__(kThreads) void k_sweep(SweepArgs a) {
   const int tc = rest % tiles_c;
   const int e = rest / tiles_c;
   const int d0 = td * TL, c0 = tc * TC;
-  const long long base_e = (long long)e * g.stride[EAX];
+  const unsigned base_e = e * (unsigned)g.stride[EAX];
   const long long vs = g.vstride;
   const unsigned tid = threadIdx.x;
 
@@ -555,28 +550,26 @@ __global__ __launch_bounds__(kThreads) void k_sweep(SweepArgs a) {
       if (idx < kCells) {
         const int l = DFAST ? idx % TLH : idx / TC;
         const int cc = DFAST ? idx / TLH : idx % TC;
-        const int gc = c0 + cc;
+        // a pencil past the grid takes the last one's cells; nothing reads its faces
+        const int gc = min(c0 + cc, nc - 1);
         double fp[NV];
-        if (gc < nc) {
+        {
           // cells past nd + R - 1 only feed faces outside the grid; clamping
           // them keeps the periodic image inside [0, nd) for any tile overhang
           const int gd = remap(min(d0 + l - R, nd - 1 + R), nd, g.periodic[DAX]);
-          const long long q = base_e + (long long)gd * g.stride[DAX] + (long long)gc * g.stride[CAX];
+          const unsigned o = cell_offset<DAX, CAX>(g, base_e, gd, gc);
           double u[NV], pl[M::NPL];
   #pragma unroll
-          for (int v = 0; v < NV; ++v) u[v] = a.U[v * vs + q];
+          for (int v = 0; v < NV; ++v) u[v] = ld(a.U + v * vs, o);
   #pragma unroll
-          for (int v = 0; v < M::NPL; ++v) pl[v] = a.V[(M::P0 + v) * vs + q];
+          for (int v = 0; v < M::NPL; ++v) pl[v] = ld(a.V + (M::P0 + v) * vs, o);
           double f[NV];
-          M::template flux<DAX, QUIRK>(u, pl, a, q, f);
+          M::template flux<DAX, QUIRK>(u, pl, a, o, f);
   #pragma unroll
           for (int v = 0; v < NV; ++v) {
             fp[v] = f[v] + u[v];  // doubled
             fm_keep[cp][v] = f[v] - u[v];
           }
-        } else {
-  #pragma unroll
-          for (int v = 0; v < NV; ++v) fp[v] = fm_keep[cp][v] = 0.0;
         }
   #pragma unroll
         for (int v = 0; v < NV; ++v) s_f[S::fidx(v, l, cc)] = fp[v];
@@ -585,20 +578,18 @@ __global__ __launch_bounds__(kThreads) void k_sweep(SweepArgs a) {
     __syncthreads();
 
     // Phase 2: WENO face values, face lf being the left face of tile cell lf.
-    // The (variable, face) pairs are dealt out one per thread per pass, so the
-    // faces beyond one per thread cost a fraction of a pass spread over the
-    // waves instead of a full pass of all variables on one wave. Upwind halves
-    // from f+ first, then downwind halves from f-.
-    constexpr int kItems = NV * S::kFaces;
-    constexpr int kPasses = (kItems + kThreads - 1) / kThreads;
+    // The (variable, face) pairs go to the threads as FaceItems says. Upwind
+    // halves from f+ first, then downwind halves from f-.
+    const typename S::Items items(tid);
+    constexpr int kPasses = S::Items::kPasses;
     double nu[kPasses], du[kPasses];
   #pragma unroll
     for (int k = 0; k < kPasses; ++k) {
-      const unsigned item = tid + k * kThreads;
-      if (item < kItems) {
-        const double *fpv = s_f + S::item_fidx(item);
+      if (items.has(k)) {
+        const double *fpv = s_f + items.lds(k);
         Weno<ORDER, true>::up([&](int m) { return fpv[m * S::kStrideL]; }, nu[k], du[k]);
       }
+      if (S::Items::kRegular) pass_end(nu[k], du[k]);
     }
     __syncthreads();
   #pragma unroll
@@ -614,21 +605,20 @@ __global__ __launch_bounds__(kThreads) void k_sweep(SweepArgs a) {
     __syncthreads();
   #pragma unroll
     for (int k = 0; k < kPasses; ++k) {
-      const unsigned item = tid + k * kThreads;
-      if (item < kItems) {
-        const double *fmv = s_f + S::item_fidx(item);
+      if (items.has(k)) {
+        const double *fmv = s_f + items.lds(k);
         double nd, dd;
         Weno<ORDER, true>::down([&](int m) { return fmv[m * S::kStrideL]; }, nd, dd);
         nu[k] = weno_combine(nu[k], du[k], nd, dd);
       }
+      if (S::Items::kRegular) pass_end(nu[k]);
     }
     __syncthreads();
-    // item = v * kFaces + idx, idx enumerating (lf, cc) in gidx order for both
-    // layouts, so the face of item goes to s_f[item]
+    // an item's place v * kFaces + f, f enumerating (lf, cc) in gidx order for
+    // both layouts, is its face's place in s_f
   #pragma unroll
     for (int k = 0; k < kPasses; ++k) {
-      const unsigned item = tid + k * kThreads;
-      if (item < kItems) s_f[item] = nu[k];
+      if (items.has(k)) s_f[items.item(k)] = nu[k];
     }
     __syncthreads();
   } else {
@@ -636,26 +626,23 @@ __global__ __launch_bounds__(kThreads) void k_sweep(SweepArgs a) {
     for (unsigned idx = tid; idx < TLH * TC; idx += kThreads) {
       const int l = DFAST ? idx % TLH : idx / TC;
       const int cc = DFAST ? idx / TLH : idx % TC;
-      const int gc = c0 + cc;
+      const int gc = min(c0 + cc, nc - 1);
       double fp[NV], fm[NV];
-      if (gc < nc) {
+      {
         const int gd = remap(min(d0 + l - R, nd - 1 + R), nd, g.periodic[DAX]);
-        const long long q = base_e + (long long)gd * g.stride[DAX] + (long long)gc * g.stride[CAX];
+        const unsigned o = cell_offset<DAX, CAX>(g, base_e, gd, gc);
         double u[NV], pl[M::NPL];
 #pragma unroll
-        for (int v = 0; v < NV; ++v) u[v] = a.U[v * vs + q];
+        for (int v = 0; v < NV; ++v) u[v] = ld(a.U + v * vs, o);
 #pragma unroll
-        for (int v = 0; v < M::NPL; ++v) pl[v] = a.V[(M::P0 + v) * vs + q];
+        for (int v = 0; v < M::NPL; ++v) pl[v] = ld(a.V + (M::P0 + v) * vs, o);
         double f[NV];
-        M::template flux<DAX, QUIRK>(u, pl, a, q, f);
+        M::template flux<DAX, QUIRK>(u, pl, a, o, f);
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
           fp[v] = f[v] + u[v];  // doubled
           fm[v] = f[v] - u[v];
         }
-      } else {
-#pragma unroll
-        for (int v = 0; v < NV; ++v) fp[v] = fm[v] = 0.0;
       }
 #pragma unroll
       for (int v = 0; v < NV; ++v) {
@@ -664,24 +651,23 @@ __global__ __launch_bounds__(kThreads) void k_sweep(SweepArgs a) {
       }
     }
     __syncthreads();
-    constexpr int kItems = NV * S::kFaces;
-    constexpr int kPasses = (kItems + kThreads - 1) / kThreads;
+    const typename S::Items items(tid);
+    constexpr int kPasses = S::Items::kPasses;
     double face[kPasses];
 #pragma unroll
     for (int k = 0; k < kPasses; ++k) {
-      const unsigned item = tid + k * kThreads;
-      if (item < kItems) {
-        const double *fpv = s_f + S::item_fidx(item);
+      if (items.has(k)) {
+        const double *fpv = s_f + items.lds(k);
         const double *fmv = fpv + NV * TLH * TC;
         face[k] = Weno<ORDER, true>::face([&](int m) { return fpv[m * S::kStrideL]; },
                                     [&](int m) { return fmv[m * S::kStrideL]; });
       }
+      if (S::Items::kRegular) pass_end(face[k]);
     }
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < kPasses; ++k) {
-      const unsigned item = tid + k * kThreads;
-      if (item < kItems) s_f[item] = face[k];
+      if (items.has(k)) s_f[items.item(k)] = face[k];
     }
     __syncthreads();
   }
@@ -693,7 +679,7 @@ __global__ __launch_bounds__(kThreads) void k_sweep(SweepArgs a) {
   const bool live = (TL * TC == kThreads || tid < TL * TC) && gd < nd && gc < nc;
   CellC2P cs;
   if (live) {
-    const long long q = base_e + (long long)gd * g.stride[DAX] + (long long)gc * g.stride[CAX];
+    const unsigned o = cell_offset<DAX, CAX>(g, base_e, gd, gc);
     const double inv_d = g.half_inv_d[DAX];
     // net flux of this axis, added to the earlier axes' as one fused
     // multiply-add so every kernel that accumulates it rounds alike
@@ -702,29 +688,29 @@ __global__ __launch_bounds__(kThreads) void k_sweep(SweepArgs a) {
       // streamed out, as the stage outputs are (finish_rk2)
 #pragma unroll
       for (int v = 0; v < NV; ++v)
-        __builtin_nontemporal_store((s_f[S::gidx(v, l + 1, cc)] - s_f[S::gidx(v, l, cc)]) * inv_d, &a.fnet[v * vs + q]);
+        st_nt(a.fnet + v * vs, o, (s_f[S::gidx(v, l + 1, cc)] - s_f[S::gidx(v, l, cc)]) * inv_d);
     } else {
 #pragma unroll
       for (int v = 0; v < NV; ++v)
         fn[v] = fma(s_f[S::gidx(v, l + 1, cc)] - s_f[S::gidx(v, l, cc)], inv_d,
-                    TC_ == 1 ? 0.0 : a.fnet[v * vs + q]);
+                    TC_ == 1 ? 0.0 : ld(a.fnet + v * vs, o));
       if (MODE == kSweepAdd) {
 #pragma unroll
-        for (int v = 0; v < NV; ++v) a.fnet[v * vs + q] = fn[v];
+        for (int v = 0; v < NV; ++v) st(a.fnet + v * vs, o, fn[v]);
       } else if (MODE == kSweepStage1 || MODE == kSweepStage2) {
         double un[NV];
         if (MODE == kSweepStage1) {
 #pragma unroll
-          for (int v = 0; v < NV; ++v) un[v] = rk2_stage1(a.U[v * vs + q], fn[v], a.dt);
+          for (int v = 0; v < NV; ++v) un[v] = rk2_stage1(ld(a.U + v * vs, o), fn[v], a.dt);
         } else {
 #pragma unroll
-          for (int v = 0; v < NV; ++v) un[v] = rk2_stage2(a.Un[v * vs + q], a.U[v * vs + q], fn[v], a.dt);
+          for (int v = 0; v < NV; ++v) un[v] = rk2_stage2(ld(a.Un + v * vs, o), ld(a.U + v * vs, o), fn[v], a.dt);
         }
-        finish_rk2(a, q, un, M(), cs);
+        finish_rk2(a, o, un, M(), cs);
       } else if (MODE == kSweepImex2) {
-        imex2_apply(a, q, fn, cs);
+        imex2_apply(a, o, fn, cs);
       } else if (MODE == kSweepImexFinal) {
-        imex_final_apply(a, q, fn, cs);
+        imex_final_apply(a, o, fn, cs);
       }
     }
   }
@@ -763,13 +749,13 @@ __global__ __launch_bounds__(kThreads, M::NC > 9 ? 1 : 4) void k_sweep_yzf(Sweep
   const int ty = rest % tiles_y;
   const int i = rest / tiles_y;
   const int y0 = ty * 16, z0 = tz * 16;
-  const long long base_e = (long long)i * g.stride[0];
+  const unsigned base_e = i * (unsigned)g.stride[0];
   const long long vs = g.vstride;
   const unsigned tid = threadIdx.x;
   // the thread's cell is (y0 + r, z0 + c)
   const int r = tid / 16, c = tid % 16;
   const bool live = y0 + r < ny && z0 + c < nz;
-  const long long q = base_e + (long long)(y0 + r) * g.stride[1] + (z0 + c);
+  const unsigned o = cell_offset<1, 2>(g, base_e, y0 + r, z0 + c);
 
   CellC2P cs;
   if constexpr (kGroup == 16) {
@@ -783,7 +769,7 @@ __global__ __launch_bounds__(kThreads, M::NC > 9 ? 1 : 4) void k_sweep_yzf(Sweep
 #pragma unroll
       for (int v = 0; v < NV; ++v)
         acc[v] = fma(s_f[SY::gidx(v, r + 1, c)] - s_f[SY::gidx(v, r, c)], g.half_inv_d[1],
-                     __builtin_nontemporal_load(&a.fnet[v * vs + q]));  // read once
+                     ld_nt(a.fnet + v * vs, o));  // read once
     }
     __syncthreads();  // every y face is read before the z phase refills LDS
     // the z phase's loads stay after the y phase, so its registers are free
@@ -802,7 +788,7 @@ __global__ __launch_bounds__(kThreads, M::NC > 9 ? 1 : 4) void k_sweep_yzf(Sweep
 #pragma unroll
       for (int v = 0; v < NV; ++v)
         fn[v] = fma(s_f[SZ::gidx(v, c + 1, r)] - s_f[SZ::gidx(v, c, r)], g.half_inv_d[2], acc[v]);
-      sweep_apply<M, MODE>(a, q, fn, cs);
+      sweep_apply<M, MODE>(a, o, fn, cs);
     }
   } else {
     __shared__ double s_acc[NV][kThreads];  // each cell's net flux, y term added, then z
@@ -814,7 +800,7 @@ __global__ __launch_bounds__(kThreads, M::NC > 9 ? 1 : 4) void k_sweep_yzf(Sweep
       if (live && cg >= 0 && cg < kGroup) {
 #pragma unroll
         for (int v = 0; v < NV; ++v)
-          s_acc[v][tid] = fma(s_f[SY::gidx(v, r + 1, cg)] - s_f[SY::gidx(v, r, cg)], g.half_inv_d[1], a.fnet[v * vs + q]);
+          s_acc[v][tid] = fma(s_f[SY::gidx(v, r + 1, cg)] - s_f[SY::gidx(v, r, cg)], g.half_inv_d[1], ld(a.fnet + v * vs, o));
       }
       __syncthreads();  // every face is read before LDS is refilled
       __builtin_amdgcn_sched_barrier(0);
@@ -837,7 +823,7 @@ __global__ __launch_bounds__(kThreads, M::NC > 9 ? 1 : 4) void k_sweep_yzf(Sweep
       double fn[NV];
 #pragma unroll
       for (int v = 0; v < NV; ++v) fn[v] = s_acc[v][tid];
-      sweep_apply<M, MODE>(a, q, fn, cs);
+      sweep_apply<M, MODE>(a, o, fn, cs);
     }
   }
   if (MODE >= kSweepStage1) reduce_stats(a.stats, cs.cells, cs.iters, cs.fails, cs.maxit);
@@ -880,7 +866,7 @@ __global__ __launch_bounds__(kThreads) void k_sweep_xyf(SweepArgs a) {
   // contiguous axis
   const int r = tid / TY, c = tid % TY;
   const bool live = (kCellsT == kThreads || tid < kCellsT) && x0 + r < nx && y0 + c < ny;
-  const long long q = (long long)(x0 + r) * g.stride[0] + (long long)(y0 + c) * g.stride[1];
+  const unsigned o = cell_offset<0, 1>(g, 0, x0 + r, y0 + c);
 
   // y phase: faces along y; group h holds the GX x pencils from x0 + GX h,
   // whose cells belong to the TY GX threads from TY GX h
@@ -905,7 +891,7 @@ __global__ __launch_bounds__(kThreads) void k_sweep_xyf(SweepArgs a) {
 #pragma unroll
       for (int v = 0; v < NV; ++v)
         fn[v] = fma(s_f[SX::gidx(v, r + 1, c)] - s_f[SX::gidx(v, r, c)], g.half_inv_d[0], s_acc[v][tid]);
-      sweep_apply<M, MODE>(a, q, fn, cs);
+      sweep_apply<M, MODE>(a, o, fn, cs);
     }
   } else {
     // x phase: faces along x; group h holds the GY y pencils from y0 + GY h
@@ -925,7 +911,7 @@ __global__ __launch_bounds__(kThreads) void k_sweep_xyf(SweepArgs a) {
       double fn[NV];
 #pragma unroll
       for (int v = 0; v < NV; ++v) fn[v] = s_acc[v][tid];
-      sweep_apply<M, MODE>(a, q, fn, cs);
+      sweep_apply<M, MODE>(a, o, fn, cs);
     }
   }
   if (MODE >= kSweepStage1) reduce_stats(a.stats, cs.cells, cs.iters, cs.fails, cs.maxit);
@@ -955,7 +941,7 @@ __device__ __forceinline__ void split_cell(const SweepArgs &a, long long q, doub
   for (int v = 0; v < M::NC; ++v) u[v] = a.U[v * vs + q];
 #pragma unroll
   for (int v = 0; v < M::NPL; ++v) pl[v] = a.V[(M::P0 + v) * vs + q];
-  M::template flux<DIR, QUIRK>(u, pl, a, q, f);
+  M::template flux<DIR, QUIRK>(u, pl, a, (unsigned)q * 8u, f);
 #pragma unroll
   for (int v = 0; v < M::NC; ++v) {
     fp[v] = f[v] + u[v];  // doubled
@@ -1458,7 +1444,7 @@ __global__ __launch_bounds__(kThreads) void k_imex1_srrmhd(SweepArgs a) {
     const double Zg = srrmhd_guess_Z(a.Vg[0 * vs + q], a.Vg[1 * vs + q], a.Vg[2 * vs + q], a.Vg[3 * vs + q],
                                      a.Vg[4 * vs + q], a.gamma);
     const int its = imex_stage(c, a.dt, a.gamma, a.sigma, a.cp, Zg, x);
-    c2p_store_srrmhd(a, q, x, A, cs);
+    c2p_store_srrmhd(a, (unsigned)q * 8u, x, A, cs);
     if (its < 0) cs.fails = 1;
     double s5[5];
     srrmhd_source5(x, A, a.cp, s5);
