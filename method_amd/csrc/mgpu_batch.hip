@@ -21,6 +21,7 @@
 
 #include "method_gpu.h"
 #include "mgpu_kernels.hpp"
+#include "mgpu_tile.hpp"
 
 using namespace mgpu;
 
@@ -30,7 +31,6 @@ int engine_fail(const char *fmt, ...);
 
 namespace {
 
-constexpr int kThreads = 256;
 constexpr int kSyncStep = 32;   // ints between counters: each has a 128-byte line of its own
 constexpr int kEndBlocks = 64;  // workgroups of a stage's end (the retry)
 constexpr int kXcds = 8;  // MI355X: workgroups go round robin over 8 XCDs, each with its own L2
@@ -92,50 +92,47 @@ struct BatchShape {
 };
 
 // Lax-Friedrichs split flux (alpha = 1) of one cell along DIR
-// (fluxVectorSplitting.cc:4-28).
+// (fluxVectorSplitting.cc:4-28), doubled. org: the instance's first cell, o
+// the cell's byte offset from it.
 template <int DIR>
-__device__ __forceinline__ void split_flux(const BatchArgs &a, long long q, double fp[9], double fm[9]) {
+__device__ __forceinline__ void split_flux(const BatchArgs &a, long long org, unsigned o, double fp[9], double fm[9]) {
+  const double *U = a.U + org, *V = a.V + org;
   const long long vs = a.vs;
   double u[9];
 #pragma unroll
-  for (int v = 0; v < 9; ++v) u[v] = a.U[v * vs + q];
-  const double vx = a.V[1 * vs + q], vy = a.V[2 * vs + q], vz = a.V[3 * vs + q], p = a.V[4 * vs + q];
+  for (int v = 0; v < 9; ++v) u[v] = ld(U + v * vs, o);
+  const double vx = ld(V + 1 * vs, o), vy = ld(V + 2 * vs, o), vz = ld(V + 3 * vs, o), p = ld(V + 4 * vs, o);
   double f[9];
   srmhd_flux<DIR, false>(u, vx, vy, vz, p, f);
 #pragma unroll
   for (int v = 0; v < 9; ++v) {
-    fp[v] = f[v] + u[v];  // doubled
+    fp[v] = f[v] + u[v];
     fm[v] = f[v] - u[v];
   }
 }
 
-// The WENO face values of one tile phase along DIR, left in s_f[item] for
-// the NITEMS (variable, face) items. Phase 1 forms the split fluxes of the
-// NCELLS tile-and-halo cells (cell_q gives a cell's index, or -1 outside the
-// instance, where the fluxes are zero), puts f+ in LDS at s_f[v NCELLS +
-// idx] and keeps f- in registers; the upwind half of every item is formed
-// from f+ (item_at gives the LDS offset of its first stencil cell, STEP the
-// offset between stencil cells), f- takes f+'s place and the downwind halves
-// follow. Holding one half at a time halves the LDS of a workgroup, so more
-// of them share a CU; the items are dealt out one per thread per pass.
-template <int ORDER, int DIR, int NCELLS, int NITEMS, int STEP, class CellQ, class ItemAt>
-__device__ __forceinline__ void tile_faces(const BatchArgs &a, double *s_f, int tid, CellQ cell_q, ItemAt item_at) {
+// The WENO face values of one tile phase along DIR, left in s_f[v FACES + f]
+// for the FACES faces of each variable. Phase 1 forms the split fluxes of the
+// NCELLS tile-and-halo cells (cell_o gives a cell's byte offset from the
+// instance's first), puts f+ in LDS at s_f[v NCELLS + idx] and keeps f- in
+// registers; the upwind half of every face is formed from f+ (Off::at(f) is
+// the LDS offset of its first stencil cell, STEP the offset between stencil
+// cells), f- takes f+'s place and the downwind halves follow. Holding one half
+// at a time halves the LDS of a workgroup, so more of them share a CU; the
+// items are dealt out as FaceItems says.
+template <int ORDER, int DIR, int NCELLS, int FACES, int STEP, class Off, class CellO>
+__device__ __forceinline__ void tile_faces(const BatchArgs &a, double *s_f, int tid, long long org, CellO cell_o) {
   constexpr int NV = kSrmhdCons;
+  using Items = FaceItems<NV, FACES, NCELLS, Off>;
   constexpr int kCellPasses = (NCELLS + kThreads - 1) / kThreads;
-  constexpr int kPasses = (NITEMS + kThreads - 1) / kThreads;
+  constexpr int kPasses = Items::kPasses;
   double fm_keep[kCellPasses][NV];
 #pragma unroll
   for (int cp = 0; cp < kCellPasses; ++cp) {
     const int idx = tid + cp * kThreads;
     if (idx < NCELLS) {
       double fp[NV];
-      const long long q = cell_q(idx);
-      if (q >= 0) {
-        split_flux<DIR>(a, q, fp, fm_keep[cp]);
-      } else {
-#pragma unroll
-        for (int v = 0; v < NV; ++v) fp[v] = fm_keep[cp][v] = 0.0;
-      }
+      split_flux<DIR>(a, org, cell_o(idx), fp, fm_keep[cp]);
 #pragma unroll
       for (int v = 0; v < NV; ++v) s_f[v * NCELLS + idx] = fp[v];
     }
@@ -146,14 +143,15 @@ __device__ __forceinline__ void tile_faces(const BatchArgs &a, double *s_f, int 
 #pragma unroll
     for (int v = 0; v < NV; ++v) asm volatile("" : "+v"(fm_keep[cp][v]));
   __syncthreads();
+  const Items items(tid);
   double nu[kPasses], du[kPasses];
 #pragma unroll
   for (int k = 0; k < kPasses; ++k) {
-    const int item = tid + k * kThreads;
-    if (item < NITEMS) {
-      const double *fpv = s_f + item_at(item);
+    if (items.has(k)) {
+      const double *fpv = s_f + items.lds(k);
       Weno<ORDER, true>::up([&](int m) { return fpv[m * STEP]; }, nu[k], du[k]);
     }
+    if (Items::kRegular) pass_end(nu[k], du[k]);
   }
   // the upwind halves are formed before the barrier after which f- overwrites f+
 #pragma unroll
@@ -170,22 +168,20 @@ __device__ __forceinline__ void tile_faces(const BatchArgs &a, double *s_f, int 
   __syncthreads();
 #pragma unroll
   for (int k = 0; k < kPasses; ++k) {
-    const int item = tid + k * kThreads;
-    if (item < NITEMS) {
-      const double *fmv = s_f + item_at(item);
+    if (items.has(k)) {
+      const double *fmv = s_f + items.lds(k);
       double nd, dd;
       Weno<ORDER, true>::down([&](int m) { return fmv[m * STEP]; }, nd, dd);
       nu[k] = weno_combine(nu[k], du[k], nd, dd);
     }
+    if (Items::kRegular) pass_end(nu[k]);
   }
 #pragma unroll
   for (int k = 0; k < kPasses; ++k) asm volatile("" : "+v"(nu[k]));
   __syncthreads();
 #pragma unroll
-  for (int k = 0; k < kPasses; ++k) {
-    const int item = tid + k * kThreads;
-    if (item < NITEMS) s_f[item] = nu[k];
-  }
+  for (int k = 0; k < kPasses; ++k)
+    if (items.has(k)) s_f[items.item(k)] = nu[k];
   __syncthreads();
 }
 
@@ -216,22 +212,18 @@ __device__ __forceinline__ void batch_tile(const BatchArgs &a, double *s_f, doub
 
   // ---- y faces: rows x0 .. x0+TX-1, cells y0-R .. y0+TY+R-1; cell idx = rr WY + cy.
   // The stencil of face lf of row rr (the left face of tile cell lf) starts
-  // at cell lf of the row.
+  // at cell lf of the row. Cells past the instance's edge take its last row's
+  // (column's) place: nothing reads their faces.
   constexpr int kFacesY = TX * (TY + 1);
-  tile_faces<ORDER, 1, TX * WY, NV * kFacesY, 1>(
-      a, s_f, tid,
-      [&](int idx) -> long long {
-        const int rr = idx / WY, cy = idx - rr * WY;
-        const int gx = x0 + rr;
-        if (gx >= I.nx) return -1;
-        const int gy = remap(min(y0 + cy - R, I.ny - 1 + R), I.ny, a.py);
-        return I.off + (long long)gx * I.ny + gy;
-      },
-      [&](int item) {
-        const int v = item / kFacesY, idx = item - v * kFacesY;
-        const int rr = idx / (TY + 1), lf = idx - rr * (TY + 1);
-        return (v * TX + rr) * WY + lf;
-      });
+  struct OffY {
+    __device__ __forceinline__ static unsigned at(unsigned f) { return f + f / (TY + 1) * (unsigned)(WY - TY - 1); }
+  };
+  tile_faces<ORDER, 1, TX * WY, kFacesY, 1, OffY>(a, s_f, tid, I.off, [&](int idx) -> unsigned {
+    const int rr = idx / WY, cy = idx - rr * WY;
+    const int gx = min(x0 + rr, I.nx - 1);
+    const int gy = remap(min(y0 + cy - R, I.ny - 1 + R), I.ny, a.py);
+    return ((unsigned)gx * (unsigned)I.ny + (unsigned)gy) * 8u;
+  });
   // the y net flux waits in LDS for the x term (registers are the scarcer)
   const bool own = S::kCells == kThreads || tid < S::kCells;
   if (own) {
@@ -245,35 +237,32 @@ __device__ __forceinline__ void batch_tile(const BatchArgs &a, double *s_f, doub
 
   // ---- x faces: rows x0-R .. x0+TX+R-1, cells y0 .. y0+TY-1; cell idx = rx TY + cc
   constexpr int kFacesX = (TX + 1) * TY;
-  tile_faces<ORDER, 0, HX * TY, NV * kFacesX, TY>(
-      a, s_f, tid,
-      [&](int idx) -> long long {
-        const int rx = idx / TY, cc = idx - rx * TY;
-        const int gy = y0 + cc;
-        if (gy >= I.ny) return -1;
-        const int gx = remap(min(x0 + rx - R, I.nx - 1 + R), I.nx, a.px);
-        return I.off + (long long)gx * I.ny + gy;
-      },
-      [&](int item) {
-        const int v = item / kFacesX, idx = item - v * kFacesX;
-        const int lf = idx / TY, cc = idx - lf * TY;
-        return (v * HX + lf) * TY + cc;
-      });
+  struct OffX {
+    __device__ __forceinline__ static unsigned at(unsigned f) { return f; }
+  };
+  tile_faces<ORDER, 0, HX * TY, kFacesX, TY, OffX>(a, s_f, tid, I.off, [&](int idx) -> unsigned {
+    const int rx = idx / TY, cc = idx - rx * TY;
+    const int gy = min(y0 + cc, I.ny - 1);
+    const int gx = remap(min(x0 + rx - R, I.nx - 1 + R), I.nx, a.px);
+    return ((unsigned)gx * (unsigned)I.ny + (unsigned)gy) * 8u;
+  });
 
   const int gx = x0 + r, gy = y0 + c;
   if (!own || gx >= I.nx || gy >= I.ny) return;
-  const long long q = I.off + (long long)gx * I.ny + gy;
+  const unsigned o = ((unsigned)gx * (unsigned)I.ny + (unsigned)gy) * 8u;
   double un[NV];
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
     const double *g = s_f + (v * (TX + 1) + r) * TY + c;
     const double fn = fma(g[TY] - g[0], I.half_inv_dx, s_acc[v * S::kCells + tid]);
-    un[v] = STAGE == 1 ? rk2_stage1(a.U[v * vs + q], fn, dt) : rk2_stage2(a.Un[v * vs + q], a.U[v * vs + q], fn, dt);
+    const double u = ld(a.U + I.off + v * vs, o);
+    un[v] = STAGE == 1 ? rk2_stage1(u, fn, dt) : rk2_stage2(ld(a.Un + I.off + v * vs, o), u, fn, dt);
   }
   // TimeIntegrator::finalise's cons2prim (timeInt.h:117-132, srmhd.cc:390-562)
   double v2, Z;
-  srmhd_plain_guess(a.Vg[0 * vs + q], a.Vg[1 * vs + q], a.Vg[2 * vs + q], a.Vg[3 * vs + q], a.Vg[4 * vs + q],
-                    a.gamma, v2, Z);
+  const double *Vg = a.Vg + I.off;
+  srmhd_plain_guess(ld(Vg, o), ld(Vg + vs, o), ld(Vg + 2 * vs, o), ld(Vg + 3 * vs, o), ld(Vg + 4 * vs, o), a.gamma, v2,
+                    Z);
   const double BS = un[5] * un[1] + un[6] * un[2] + un[7] * un[3];
   const double Bsq = un[5] * un[5] + un[6] * un[6] + un[7] * un[7];
   const double Ssq = un[1] * un[1] + un[2] * un[2] + un[3] * un[3];
@@ -283,18 +272,19 @@ __device__ __forceinline__ void batch_tile(const BatchArgs &a, double *s_f, doub
   // streamed out with non-temporal stores: they do not fit in the caches and
   // would only evict the tiles' halo cells from the L2
 #pragma unroll
-  for (int v = 0; v < kSrmhdCons; ++v) __builtin_nontemporal_store(un[v], &a.Uout[v * vs + q]);
+  for (int v = 0; v < kSrmhdCons; ++v) st_nt(a.Uout + I.off + v * vs, o, un[v]);
   // stage one: rho .. p of V1, all that stage two's sweeps, guess and retry read
 #pragma unroll
-  for (int v = 0; v < (STAGE == 1 ? 5 : kSrmhdPrims); ++v) __builtin_nontemporal_store(P[v], &a.Vout[v * vs + q]);
+  for (int v = 0; v < (STAGE == 1 ? 5 : kSrmhdPrims); ++v) st_nt(a.Vout + I.off + v * vs, o, P[v]);
   if (STAGE == 2) {
-    __builtin_nontemporal_store(v2, &a.root[q]);
-    __builtin_nontemporal_store(Z, &a.root[vs + q]);
+    st_nt(a.root + I.off, o, v2);
+    st_nt(a.root + I.off + vs, o, Z);
   }
   acc.cells += 1;
   if (its < 0) {
     acc.fails += 1;
     const int slot = atomicAdd(a.fail_count, 1);
+    const long long q = I.off + (o >> 3);
     a.fail_list[slot] = q;
     a.fail_flag[q] = 1;
   } else {
