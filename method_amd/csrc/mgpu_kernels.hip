@@ -718,52 +718,55 @@ __global__ __launch_bounds__(kThreads) void k_sweep(SweepArgs a) {
 }
 
 // The y and z terms of a 3-D stage in one launch, after an x sweep has
-// written the x term (sweep plan 3): a 16 x 16 (y, z) tile of one x plane
+// written the x term (sweep plan 3): a TY x TZ (y, z) tile of one x plane
 // reconstructs its y faces, then its z faces, each phase exactly as a
 // separate sweep does it. Each cell's net flux with the y term added waits
 // (in registers or LDS) for the z term, and the z phase then applies the
-// sweep's mode. The sums
-// are formed in the separate sweeps' order, so plan 3 gives plan 2's bits,
-// and the y-added net flux never makes an HBM round trip. SRRMHD's 14
-// variables take each phase over the tile's pencils in two groups of 8, so
-// that a thread keeps the split fluxes of one tile-or-halo cell and the face
+// sweep's mode. The sums are formed in the separate sweeps' order, so plan 3
+// gives plan 2's bits, and the y-added net flux never makes an HBM round trip.
+// SRRMHD's 14 variables take each phase over the tile's pencils in groups of 8,
+// so that a thread keeps the split fluxes of one tile-or-halo cell and the face
 // values of about five (variable, face) items at a time (174-203 VGPRs where
-// the whole tile takes 184-256); SRMHD's 9 variables run faster as one group
-// of 16, with each cell's y-added net flux kept in registers instead of LDS:
-// 116-128 VGPRs and 23-25 KB of LDS, 4 waves per SIMD (in groups of 8 they
-// fit 4 waves per SIMD too but took 1 % longer).
-template <class M, int ORDER, int MODE, bool QUIRK>
+// the whole 16 x 16 tile took 184-256); SRMHD's 9 variables run faster with all
+// pencils at once and each cell's y-added net flux in registers instead of LDS:
+// 126-128 VGPRs and 23-32 KB of LDS, 4 waves per SIMD (in groups of 8 they
+// fit 4 waves per SIMD too but took 1 % longer). The tile follows from the grid
+// (launch_sweep_yzf_o).
+template <class M, int ORDER, int MODE, bool QUIRK, int TY, int TZ>
 __global__ __launch_bounds__(kThreads, M::NC > 9 ? 1 : 4) void k_sweep_yzf(SweepArgs a) {
-  constexpr int kGroup = M::NC > 9 ? 8 : 16;  // pencils per group
-  using SY = SweepShape<M, ORDER, 1, 2, false, 16, kGroup>;
-  using SZ = SweepShape<M, ORDER, 2, 1, true, 16, kGroup>;
+  constexpr bool kWhole = M::NC <= 9;                          // all pencils of a phase at once
+  constexpr int GY = kWhole ? TY : 8, GZ = kWhole ? TZ : 8;    // pencils per group of the z, the y phase
+  constexpr int kCellsT = TY * TZ;
+  static_assert(kCellsT <= kThreads && TY % GY == 0 && TZ % GZ == 0, "at most one cell per thread, whole groups");
+  using SY = SweepShape<M, ORDER, 1, 2, false, TY, GZ>;
+  using SZ = SweepShape<M, ORDER, 2, 1, true, TZ, GY>;
   constexpr int NV = M::NC;
   constexpr int kLds = SY::kLds > SZ::kLds ? SY::kLds : SZ::kLds;
   __shared__ double s_f[kLds];
   const Geo &g = a.geo;
   const int ny = g.n[1], nz = g.n[2];
-  const int tiles_y = (ny + 15) / 16, tiles_z = (nz + 15) / 16;
+  const int tiles_y = (ny + TY - 1) / TY, tiles_z = (nz + TZ - 1) / TZ;
   const int lb = xcd_block(blockIdx.x, gridDim.x);
   const int tz = lb % tiles_z;
   const int rest = lb / tiles_z;
   const int ty = rest % tiles_y;
   const int i = rest / tiles_y;
-  const int y0 = ty * 16, z0 = tz * 16;
+  const int y0 = ty * TY, z0 = tz * TZ;
   const unsigned base_e = i * (unsigned)g.stride[0];
   const long long vs = g.vstride;
   const unsigned tid = threadIdx.x;
   // the thread's cell is (y0 + r, z0 + c)
-  const int r = tid / 16, c = tid % 16;
-  const bool live = y0 + r < ny && z0 + c < nz;
+  const int r = tid / TZ, c = tid % TZ;
+  const bool live = (kCellsT == kThreads || tid < kCellsT) && y0 + r < ny && z0 + c < nz;
   const unsigned o = cell_offset<1, 2>(g, base_e, y0 + r, z0 + c);
 
   CellC2P cs;
-  if constexpr (kGroup == 16) {
+  if constexpr (kWhole) {
     // y phase over the whole tile, pencils along z
     // each cell's net flux with the y term added waits in registers
     unsigned ty = tid;
     asm volatile("" : "+v"(ty));
-    sweep_tile_faces<M, ORDER, 1, 2, false, 16, 16, false>(a, s_f, y0, z0, base_e, ny, nz, ty);
+    sweep_tile_faces<M, ORDER, 1, 2, false, TY, TZ, false>(a, s_f, y0, z0, base_e, ny, nz, ty);
     double acc[NV];
     if (live) {
 #pragma unroll
@@ -782,7 +785,7 @@ __global__ __launch_bounds__(kThreads, M::NC > 9 ? 1 : 4) void k_sweep_yzf(Sweep
     asm volatile("" : "+v"(tz));
     // z phase, pencils along y: the thread's cell is tile cell c of pencil r,
     // and it finishes straight from the faces in LDS
-    sweep_tile_faces<M, ORDER, 2, 1, true, 16, 16, QUIRK>(a, s_f, z0, y0, base_e, nz, ny, tz);
+    sweep_tile_faces<M, ORDER, 2, 1, true, TZ, TY, QUIRK>(a, s_f, z0, y0, base_e, nz, ny, tz);
     if (live) {
       double fn[NV];
 #pragma unroll
@@ -791,13 +794,13 @@ __global__ __launch_bounds__(kThreads, M::NC > 9 ? 1 : 4) void k_sweep_yzf(Sweep
       sweep_apply<M, MODE>(a, o, fn, cs);
     }
   } else {
-    __shared__ double s_acc[NV][kThreads];  // each cell's net flux, y term added, then z
-    // y phase: faces along y; group h holds the kGroup pencils from z0 + kGroup h
+    __shared__ double s_acc[NV][kCellsT];  // each cell's net flux, y term added, then z
+    // y phase: faces along y; group h holds the GZ pencils from z0 + GZ h
 #pragma unroll 1
-    for (int h = 0; h < 16 / kGroup; ++h) {
-      sweep_tile_faces<M, ORDER, 1, 2, false, 16, kGroup, false>(a, s_f, y0, z0 + h * kGroup, base_e, ny, nz, tid);
-      const int cg = c - h * kGroup;
-      if (live && cg >= 0 && cg < kGroup) {
+    for (int h = 0; h < TZ / GZ; ++h) {
+      sweep_tile_faces<M, ORDER, 1, 2, false, TY, GZ, false>(a, s_f, y0, z0 + h * GZ, base_e, ny, nz, tid);
+      const int cg = c - h * GZ;
+      if (live && cg >= 0 && cg < GZ) {
 #pragma unroll
         for (int v = 0; v < NV; ++v)
           s_acc[v][tid] = fma(s_f[SY::gidx(v, r + 1, cg)] - s_f[SY::gidx(v, r, cg)], g.half_inv_d[1], ld(a.fnet + v * vs, o));
@@ -805,13 +808,13 @@ __global__ __launch_bounds__(kThreads, M::NC > 9 ? 1 : 4) void k_sweep_yzf(Sweep
       __syncthreads();  // every face is read before LDS is refilled
       __builtin_amdgcn_sched_barrier(0);
     }
-    // z phase: faces along z; group h holds the kGroup pencils from y0 + kGroup h,
-    // whose cells belong to the 16 kGroup threads from 16 kGroup h
+    // z phase: faces along z; group h holds the GY pencils from y0 + GY h,
+    // whose cells belong to the TZ GY threads from TZ GY h
 #pragma unroll 1
-    for (int h = 0; h < 16 / kGroup; ++h) {
-      sweep_tile_faces<M, ORDER, 2, 1, true, 16, kGroup, QUIRK>(a, s_f, z0, y0 + h * kGroup, base_e, nz, ny, tid);
-      const int rg = r - h * kGroup;
-      if (live && rg >= 0 && rg < kGroup) {
+    for (int h = 0; h < TY / GY; ++h) {
+      sweep_tile_faces<M, ORDER, 2, 1, true, TZ, GY, QUIRK>(a, s_f, z0, y0 + h * GY, base_e, nz, ny, tid);
+      const int rg = r - h * GY;
+      if (live && rg >= 0 && rg < GY) {
 #pragma unroll
         for (int v = 0; v < NV; ++v)
           s_acc[v][tid] = fma(s_f[SZ::gidx(v, c + 1, rg)] - s_f[SZ::gidx(v, c, rg)], g.half_inv_d[2], s_acc[v][tid]);
@@ -1702,6 +1705,10 @@ __global__ __launch_bounds__(kThreads) void k_flux_vector_srrmhd(Geo g, PadGeo p
   for (int v = 0; v < kSrrmhdCons; ++v) dst[v * pg.ntot + p] = f[v];
 }
 
+// Whether a 3-D grid is small: at most one 16 x 16 tile of its planes per CU.
+// As in 2-D, 8 x 8 tiles then shorten the workgroup's chain of passes.
+inline bool small_3d(const Geo &g) { return ((g.n[1] + 15LL) / 16) * ((g.n[2] + 15) / 16) * g.n[0] <= 256; }
+
 // Cells per workgroup along the only axis of a 1-D grid: one pencil of 32, so
 // that the 297 (variable, face) items of SRMHD take two passes of the threads
 // and 400 cells 13 workgroups. On the 16 x 16 tile of the strided x sweep 15
@@ -1726,6 +1733,12 @@ void launch_sweep_t(const SweepArgs &a, int quirk, hipStream_t s) {
 template <class M, int ORDER, int MODE>
 void launch_sweep_o(const SweepArgs &a, int dir, int quirk, hipStream_t s) {
   if (a.geo.dims == 3) {
+    if constexpr (MODE == kSweepWrite && !M::kStored) {
+      if (dir == 0 && small_3d(a.geo)) {
+        launch_sweep_t<M, ORDER, 0, 2, false, MODE, 8, 8>(a, quirk, s);
+        return;
+      }
+    }
     if (dir == 0) launch_sweep_t<M, ORDER, 0, 2, false, MODE>(a, quirk, s);
     else if (dir == 1) launch_sweep_t<M, ORDER, 1, 2, false, MODE>(a, quirk, s);
     else launch_sweep_t<M, ORDER, 2, 1, true, MODE>(a, quirk, s);
@@ -1782,13 +1795,30 @@ void launch_sweep_yz(const SweepArgs &a, int model, int order, int quirk, hipStr
   }
 }
 
+template <class M, int ORDER, int MODE, int TY, int TZ>
+void launch_sweep_yzf_t(const SweepArgs &a, int quirk, hipStream_t s) {
+  const int tiles = ((a.geo.n[1] + TY - 1) / TY) * ((a.geo.n[2] + TZ - 1) / TZ) * a.geo.n[0];
+  if (quirk)
+    hipLaunchKernelGGL((k_sweep_yzf<M, ORDER, MODE, true, TY, TZ>), dim3(tiles), dim3(kThreads), 0, s, a);
+  else
+    hipLaunchKernelGGL((k_sweep_yzf<M, ORDER, MODE, false, TY, TZ>), dim3(tiles), dim3(kThreads), 0, s, a);
+}
+
+// Tiles of the fused launch (KH SRMHD RK2 steps, us, 8 x 32 | 16 x 16 | 8 x 8):
+//   WENO5  32^3 - | 69.4 | 58.6, 64^3 134 | 133, 128^3 727 | 733, 256^3 5,420 | 5,577
+//   WENO3  32^3 - | 61.3 | 55.4, 64^3 108 | 105, 97 x 64 x 130 324 | 354
+// SRMHD takes 8 rows of 32 cells on grids longer than 64 along z: the z phase
+// recomputes 38/32 halo cells instead of 22/16 (the y phase 14/8), and rows
+// are read in 256-byte runs.
 template <class M, int ORDER, int MODE>
 void launch_sweep_yzf_o(const SweepArgs &a, int quirk, hipStream_t s) {
-  const int tiles = ((a.geo.n[1] + 15) / 16) * ((a.geo.n[2] + 15) / 16) * a.geo.n[0];
-  if (quirk)
-    hipLaunchKernelGGL((k_sweep_yzf<M, ORDER, MODE, true>), dim3(tiles), dim3(kThreads), 0, s, a);
+  constexpr int kRows = M::NC <= 9 ? 8 : 16, kCols = M::NC <= 9 ? 32 : 16;
+  if (small_3d(a.geo))
+    launch_sweep_yzf_t<M, ORDER, MODE, 8, 8>(a, quirk, s);
+  else if (a.geo.n[2] > 64)
+    launch_sweep_yzf_t<M, ORDER, MODE, kRows, kCols>(a, quirk, s);
   else
-    hipLaunchKernelGGL((k_sweep_yzf<M, ORDER, MODE, false>), dim3(tiles), dim3(kThreads), 0, s, a);
+    launch_sweep_yzf_t<M, ORDER, MODE, 16, 16>(a, quirk, s);
 }
 
 template <class M, int ORDER>
