@@ -36,12 +36,12 @@ namespace {
 
 constexpr int kRegimeThreads = 256;
 
-// The grid spacings as the reference's Data holds them, and 1 / (2 d) for
-// the centred differences of K and of D (the reference divides by 2 d; the
-// product differs from that quotient by at most one rounding).
+// 1 / (2 d) for the centred differences of K and of D and 1 / (12 d) for q's,
+// d the grid spacings (the reference divides by 2 d and 12 d; the product
+// differs from that quotient by at most one rounding).
 struct Spacing {
-  double d[3];
   double ih2[3];
+  double ih12[3];
 };
 
 // n / d for 0 <= n < 2^31 by a multiply-high and a shift: with l the
@@ -138,7 +138,7 @@ __global__ __launch_bounds__(kRegimeThreads) void k_regime_q(Geo g, PadGeo pg, P
       if (ax >= g.dims) break;
       const double *Ea = E + ax * pg.ntot;
       const long long s = pstride(pg, ax);
-      const double t = (-Ea[p + 2 * s] + 8 * Ea[p + s] - 8 * Ea[p - s] + Ea[p - 2 * s]) / (12 * sp.d[ax]);
+      const double t = (-Ea[p + 2 * s] + 8 * Ea[p + s] - 8 * Ea[p - s] + Ea[p - 2 * s]) * sp.ih12[ax];
       acc = ax == 0 ? t : acc + t;
     }
   }
@@ -198,12 +198,13 @@ __global__ __launch_bounds__(kRegimeThreads) void k_regime_flux(Geo g, PadGeo pg
     F[v * pg.ntot + p] = Weno<ORDER>::face([&](int m) { return fp[v][m]; }, [&](int m) { return fm[v][m]; });
 }
 
-// Tile of padded cells per block of k_regime_fq (the same shapes as the
-// source's tiles).
+// Tile of padded cells per block of k_regime_fq. In 3-D, rows of 16 cells (128
+// bytes): at 128^3 the launch takes 123 us (WENO3) and 164 (WENO5), against 136
+// and 165 on 4 x 8 x 8, 142 and 196 on 2 x 8 x 16, 149 and 217 on 2 x 4 x 32.
 template <int DIMS>
 struct FqTile {
-  static constexpr int T[3] = {DIMS == 3 ? 4 : (DIMS == 2 ? 16 : 256), DIMS == 3 ? 8 : (DIMS == 2 ? 16 : 1),
-                               DIMS == 3 ? 8 : 1};
+  static constexpr int T[3] = {DIMS == 3 ? 4 : (DIMS == 2 ? 16 : 256), DIMS == 3 ? 4 : (DIMS == 2 ? 16 : 1),
+                               DIMS == 3 ? 16 : 1};
   static_assert(T[0] * T[1] * T[2] == kRegimeThreads, "one padded cell per thread");
 };
 
@@ -299,7 +300,7 @@ __device__ __forceinline__ void regime_fq_phase(const Geo &g, const PadGeo &pg, 
     }
     if (qin) {
       const double *ea = &s_eb[AX][base + LO * kStep];  // E_AX at this cell
-      const double t = (-ea[2 * kStep] + 8 * ea[kStep] - 8 * ea[-kStep] + ea[-2 * kStep]) / (12 * sp.d[AX]);
+      const double t = (-ea[2 * kStep] + 8 * ea[kStep] - 8 * ea[-kStep] + ea[-2 * kStep]) * sp.ih12[AX];
       qacc = AX == 0 ? t : qacc + t;
     }
   }
@@ -378,35 +379,6 @@ __device__ __forceinline__ void regime_dwdsb(double q, double sig, const double 
     for (int m = 0; m < 3; ++m) dw[l][m] *= alpha;
 }
 
-// Rows 1..4, columns 5..10 of df/dw along axis ax (REGIME.cc:404-548), and
-// its (row, ax+1) entries of rows 0 and 4.
-__device__ __forceinline__ void regime_dfdw(int ax, double gam, const double P[8], const double E[3], double J[5][6],
-                                            double &j0, double &j4) {
-  for (int l = 0; l < 5; ++l)
-    for (int n = 0; n < 6; ++n) J[l][n] = 0.0;
-  // column index n - 5 for w entries 5..10 (B, E)
-  if (ax == 0) {
-    j0 = P[0];
-    J[1][0] = -P[5]; J[1][1] = P[6]; J[1][2] = P[7]; J[1][3] = -E[0]; J[1][4] = E[1]; J[1][5] = E[2];
-    J[2][0] = -P[6]; J[2][1] = -P[5]; J[2][3] = -E[1]; J[2][4] = -E[0];
-    J[3][0] = -P[7]; J[3][2] = -P[5]; J[3][3] = -E[2]; J[3][5] = -E[0];
-    J[4][1] = -E[2]; J[4][2] = E[1]; J[4][4] = P[7]; J[4][5] = -P[6];
-  } else if (ax == 1) {
-    j0 = P[0];
-    J[1][0] = -P[6]; J[1][1] = -P[5]; J[1][3] = -E[1]; J[1][4] = -E[0];
-    J[2][0] = P[5]; J[2][1] = -P[6]; J[2][2] = P[7]; J[2][3] = E[0]; J[2][4] = -E[1]; J[2][5] = E[2];
-    J[3][1] = -P[7]; J[3][2] = -P[6]; J[3][4] = -E[2]; J[3][5] = -E[1];
-    J[4][0] = E[2]; J[4][2] = -E[0]; J[4][3] = -P[7]; J[4][5] = P[5];
-  } else {
-    j0 = P[0];
-    J[1][0] = -P[7]; J[1][2] = -P[5]; J[1][3] = -E[2]; J[1][5] = -E[0];
-    J[2][1] = -P[7]; J[2][2] = -P[6]; J[2][4] = -E[2]; J[2][5] = -E[1];
-    J[3][0] = P[5]; J[3][1] = P[6]; J[3][2] = -P[7]; J[3][3] = E[0]; J[3][4] = E[1]; J[3][5] = -E[2];
-    J[4][0] = -E[1]; J[4][1] = E[0]; J[4][3] = P[6]; J[4][4] = -P[5];
-  }
-  j4 = gam * P[4] / (gam - 1);
-}
-
 // K at padded cell p (REGIME.cc:293-370): centred differences of the E-face
 // fluxes, zero outside [1, N - 1) along each axis.
 __device__ __forceinline__ void regime_k(const Geo &g, const PadGeo &pg, const Spacing &sp, const double *F,
@@ -422,52 +394,59 @@ __device__ __forceinline__ void regime_k(const Geo &g, const PadGeo &pg, const S
   }
 }
 
-// The per-cell quantities D is formed from: primitives, E, q, alpha
-// (REGIME.cc:141-224) and dw/ds_b (REGIME.cc:226-290).
+// The per-cell quantities D is formed from: primitives, E, alpha
+// (REGIME.cc:141-224) and dw/ds_b K (REGIME.cc:226-290), whose velocity, B and
+// E rows are, with qs = q^2 + sigma^2 and the matrix written out as vectors,
+//   t_v = alpha (-q qs K - sigma^2 q (B.K) B + sigma qs K x B)
+//   t_B = alpha (-sigma^3 (B.K) E + sigma qs v x K)
+//   t_E = alpha (-sigma^3 (B.K) B - sigma qs K).
 struct RegimeCell {
-  double P[8], Ec[3], q, alpha;
-  double dw[12][3];
+  double P[8], E[3], alpha;
+  double tv[3], tB[3], tE[3];
 };
 
 __device__ __forceinline__ void regime_cell(const Geo &g, const PadGeo &pg, const double *V, const double *Q,
-                                            long long p, const int pos[3], double sig, RegimeCell &c) {
+                                            long long p, const int pos[3], const double K[3], double sig,
+                                            RegimeCell &c) {
   load_prims(V, g.vstride, image_of(g, pg, pos), c.P);
-  regime_e_of(c.P, c.Ec);
-  c.q = Q[p];
-  const double qs = c.q * c.q + sig * sig;
-  c.alpha = 1 / (qs * (qs + sig * sig * (c.P[5] * c.P[5] + c.P[6] * c.P[6] + c.P[7] * c.P[7])));
-  regime_dwdsb(c.q, sig, c.P, c.Ec, c.alpha, c.dw);
+  regime_e_of(c.P, c.E);
+  const double q = Q[p], *v = c.P + 1, *B = c.P + 5;
+  const double sig2 = sig * sig, qs = fma(q, q, sig2);
+  c.alpha = 1 / (qs * fma(sig2, fma(B[0], B[0], fma(B[1], B[1], B[2] * B[2])), qs));
+  const double BK = fma(B[0], K[0], fma(B[1], K[1], B[2] * K[2]));
+  const double a1 = c.alpha * sig * qs, a2 = -c.alpha * q * qs;         // of K x B, v x K, -K; of K
+  const double aB = -c.alpha * sig2 * BK, aq = aB * q, as = aB * sig;  // of B in t_v; of E in t_B, B in t_E
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const int i = (k + 1) % 3, j = (k + 2) % 3;
+    c.tv[k] = fma(a1, fma(K[i], B[j], -K[j] * B[i]), fma(a2, K[k], aq * B[k]));
+    c.tB[k] = fma(a1, fma(v[i], K[j], -v[j] * K[i]), as * c.E[k]);
+    c.tE[k] = fma(-a1, K[k], as * B[k]);
+  }
 }
 
-// D = M K along axis AX with M as REGIME::set_Dx/Dy/Dz form it
-// (REGIME.cc:551-774): M = -df/dw dw/ds_b.
+// D = -df/dw (dw/ds_b K) along axis AX (REGIME::set_Dx/Dy/Dz, REGIME.cc:551-774,
+// with the df/dw of REGIME.cc:404-548): the derivative of the flux vector
+// along t, with its sign. The reference multiplies out M = -df/dw dw/ds_b, an
+// 8 x 3 matrix, and then M K; applying the two factors to K one after the
+// other is the same sum in another order, at 32 operations an axis instead of
+// 137, and keeps 9 values between the axes instead of 36.
 template <int AX>
-__device__ __forceinline__ void regime_d_axis(const RegimeCell &c, const double K[3], double gam, double D[8]) {
-  double J[5][6], j0, j4;
-  regime_dfdw(AX, gam, c.P, c.Ec, J, j0, j4);
-  constexpr int a = 1 + AX;
-  double M[8][3];
-  for (int l = 0; l < 8; ++l)
-    for (int m = 0; m < 3; ++m) M[l][m] = 0.0;
-  for (int m = 0; m < 3; ++m) {
-    M[0][m] -= j0 * c.dw[a][m];
-    M[4][m] -= j4 * c.dw[a][m];
-  }
-  // the induction rows with one unit entry each
-  if (AX == 0) {
-    for (int m = 0; m < 3; ++m) M[6][m] -= (-c.dw[10][m]);
-    for (int m = 0; m < 3; ++m) M[7][m] -= c.dw[9][m];
-  } else if (AX == 1) {
-    for (int m = 0; m < 3; ++m) M[5][m] -= c.dw[10][m];
-    for (int m = 0; m < 3; ++m) M[7][m] -= (-c.dw[8][m]);
-  } else {
-    for (int m = 0; m < 3; ++m) M[5][m] -= (-c.dw[9][m]);
-    for (int m = 0; m < 3; ++m) M[6][m] -= c.dw[8][m];
-  }
-  for (int l = 1; l < 5; ++l)
-    for (int m = 0; m < 3; ++m)
-      for (int n = 0; n < 6; ++n) M[l][m] = fma(-J[l][n], c.dw[5 + n][m], M[l][m]);
-  for (int l = 0; l < 8; ++l) D[l] = fma(M[l][2], K[2], fma(M[l][1], K[1], M[l][0] * K[0]));
+__device__ __forceinline__ void regime_d_axis(const RegimeCell &c, double gam, double D[8]) {
+  constexpr int i = (AX + 1) % 3, j = (AX + 2) % 3;
+  const double *B = c.P + 5, *E = c.E, *tB = c.tB, *tE = c.tE;
+  D[0] = -c.P[0] * c.tv[AX];
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+    if (k != AX) D[1 + k] = fma(tB[k], B[AX], fma(B[k], tB[AX], fma(tE[k], E[AX], E[k] * tE[AX])));
+  // along AX: 2 (B tB + E tE)_AX - B.tB - E.tE
+  D[1 + AX] = fma(tB[AX], B[AX], tE[AX] * E[AX]) -
+              fma(tB[i], B[i], fma(tB[j], B[j], fma(tE[i], E[i], tE[j] * E[j])));
+  D[4] = -fma(gam * rcp_pos(gam - 1) * c.P[4], c.tv[AX],
+              fma(tE[i], B[j], fma(E[i], tB[j], -fma(tE[j], B[i], E[j] * tB[i]))));
+  D[5 + AX] = 0.0;
+  D[5 + i] = tE[j];
+  D[5 + j] = -tE[i];
 }
 
 // K (REGIME.cc:293-370), then D = M K per active axis, into the work arrays
@@ -484,18 +463,18 @@ __global__ __launch_bounds__(kRegimeThreads) void k_regime_d(Geo g, PadGeo pg, P
   double K[3];
   regime_k(g, pg, sp, F, p, pos, K);
   RegimeCell c;
-  regime_cell(g, pg, V, Q, p, pos, sig, c);
+  regime_cell(g, pg, V, Q, p, pos, K, sig, c);
   for (int v = 0; v < 3; ++v) Kout[v * nt + p] = K[v];
   Aout[p] = c.alpha;
   double Dl[8];
-  regime_d_axis<0>(c, K, gam, Dl);
+  regime_d_axis<0>(c, gam, Dl);
   for (int l = 0; l < 8; ++l) D[l * nt + p] = Dl[l];
   if (g.dims > 1) {
-    regime_d_axis<1>(c, K, gam, Dl);
+    regime_d_axis<1>(c, gam, Dl);
     for (int l = 0; l < 8; ++l) D[(8 + l) * nt + p] = Dl[l];
   }
   if (g.dims > 2) {
-    regime_d_axis<2>(c, K, gam, Dl);
+    regime_d_axis<2>(c, gam, Dl);
     for (int l = 0; l < 8; ++l) D[(16 + l) * nt + p] = Dl[l];
   }
 }
@@ -516,8 +495,8 @@ __device__ __forceinline__ void regime_d_at(const Geo &g, const PadGeo &pg, cons
   double K[3];
   regime_k(g, pg, sp, F, p, ppos, K);
   RegimeCell c;
-  regime_cell(g, pg, V, Q, p, ppos, sig, c);
-  regime_d_axis<AX>(c, K, gam, D);
+  regime_cell(g, pg, V, Q, p, ppos, K, sig, c);
+  regime_d_axis<AX>(c, gam, D);
 }
 
 // Interior cells per block of the fused D + source kernel, by grid dimension.
@@ -573,10 +552,10 @@ __global__ __launch_bounds__(kRegimeThreads) void k_regime_ds(Geo g, PadGeo pg, 
       double K[3];
       regime_k(g, pg, sp, F, p, pp, K);
       RegimeCell c;
-      regime_cell(g, pg, V, Q, p, pp, sig, c);
-      regime_d_axis<0>(c, K, gam, D0);
-      if (DIMS > 1) regime_d_axis<(DIMS > 1 ? 1 : 0)>(c, K, gam, D1);
-      if (DIMS > 2) regime_d_axis<(DIMS > 2 ? 2 : 0)>(c, K, gam, D2);
+      regime_cell(g, pg, V, Q, p, pp, K, sig, c);
+      regime_d_axis<0>(c, gam, D0);
+      if (DIMS > 1) regime_d_axis<(DIMS > 1 ? 1 : 0)>(c, gam, D1);
+      if (DIMS > 2) regime_d_axis<(DIMS > 2 ? 2 : 0)>(c, gam, D2);
     }
     for (int l = 0; l < 8; ++l) sD[l][slot0(c0 + 1, c1, c2)] = D0[l];
     if (DIMS > 1)
@@ -701,7 +680,8 @@ void launch_regime_dwdsb(const Geo &g, const PadGeo &pg, const double *V, const 
 void launch_regime_source(const Geo &g, const PadGeo &pg, const double dx[3], const double *V, double *work,
                           double *src, double gam, double sigma, int order, bool fused, hipStream_t s) {
   const long long nt = pg.ntot;
-  const Spacing sp = {{dx[0], dx[1], dx[2]}, {1.0 / (2 * dx[0]), 1.0 / (2 * dx[1]), 1.0 / (2 * dx[2])}};
+  const Spacing sp = {{1.0 / (2 * dx[0]), 1.0 / (2 * dx[1]), 1.0 / (2 * dx[2])},
+                      {1.0 / (12 * dx[0]), 1.0 / (12 * dx[1]), 1.0 / (12 * dx[2])}};
   const RegimeFields fl = regime_fields_of(pg, work);
   double *E = fl.E, *Q = fl.q, *F = fl.F, *D = fl.D;
   const PadDiv dv = pad_div(pg);
@@ -714,9 +694,10 @@ void launch_regime_source(const Geo &g, const PadGeo &pg, const double dx[3], co
   if (fused) {
     // face fluxes and q in one launch, E formed where it is used
     {
-      const int n1 = (pg.N[1] + 7) / 8, n2 = (pg.N[2] + 7) / 8;  // 3-D tiles 4 x 8 x 8
       if (g.dims == 3) {
-        const unsigned nb = (unsigned)(((pg.N[0] + 3) / 4) * n1 * n2);
+        using T = FqTile<3>;
+        const int n1 = (pg.N[1] + T::T[1] - 1) / T::T[1], n2 = (pg.N[2] + T::T[2] - 1) / T::T[2];
+        const unsigned nb = (unsigned)(((pg.N[0] + T::T[0] - 1) / T::T[0]) * n1 * n2);
         const int run = std::max(1, n1 * n2 / 8);
         if (order == 3) hipLaunchKernelGGL((k_regime_fq<3, 3>), dim3(nb), block, 0, s, g, pg, sp, V, F, Q, run);
         else hipLaunchKernelGGL((k_regime_fq<5, 3>), dim3(nb), block, 0, s, g, pg, sp, V, F, Q, run);
