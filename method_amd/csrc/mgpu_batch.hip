@@ -105,10 +105,7 @@ __device__ __forceinline__ void split_flux(const BatchArgs &a, long long org, un
   double f[9];
   srmhd_flux<DIR, false>(u, vx, vy, vz, p, f);
 #pragma unroll
-  for (int v = 0; v < 9; ++v) {
-    fp[v] = f[v] + u[v];
-    fm[v] = f[v] - u[v];
-  }
+  for (int v = 0; v < 9; ++v) split_pm(f[v], u[v], fp[v], fm[v]);
 }
 
 // The WENO face values of one tile phase along DIR, left in s_f[v FACES + f]

@@ -203,20 +203,22 @@ constexpr int kSrmhdCons = 9, kSrmhdPrims = 8, kSrmhdAux = 13;
 // Flux vector in direction DIR from the cell's cons and (vx, vy, vz, p)
 // (SRMHD::fluxVector, srmhd.cc:72-206). W and b^mu are formed from the
 // primitives as SRMHD::primsToAll does (srmhd.cc:596-622). QUIRK_PHI_Z: the
-// z flux of phi is By as at srmhd.cc:200.
+// z flux of phi is By as at srmhd.cc:200. Every sum of products is written as
+// explicit fused multiply-adds: left to the compiler, which of the products is
+// fused depends on the surrounding code, and kernels would round differently.
 template <int DIR, bool QUIRK_PHI_Z>
 __device__ __forceinline__ void srmhd_flux(const double u[9], double vx, double vy, double vz, double p,
                                            double f[9]) {
   const double Bx = u[5], By = u[6], Bz = u[7];
-  const double v2 = vx * vx + vy * vy + vz * vz;
+  const double v2 = fma(vx, vx, fma(vy, vy, vz * vz));
   const double W = rsqrt_pos(1.0 - v2);
   const double iW = (1.0 - v2) * W;  // 1/W
-  const double b0 = W * (vx * Bx + vy * By + vz * Bz);
+  const double b0 = W * fma(vx, Bx, fma(vy, By, vz * Bz));
   const double bx = fma(Bx, iW, b0 * vx), by = fma(By, iW, b0 * vy), bz = fma(Bz, iW, b0 * vz);
-  const double bsq = (Bx * Bx + By * By + Bz * Bz + b0 * b0) * (iW * iW);
+  const double bsq = fma(Bx, Bx, fma(By, By, fma(Bz, Bz, b0 * b0))) * (iW * iW);
   const double vd = DIR == 0 ? vx : (DIR == 1 ? vy : vz);
   const double Bd = DIR == 0 ? Bx : (DIR == 1 ? By : Bz);
-  const double ptot = p + 0.5 * bsq;
+  const double ptot = fma(0.5, bsq, p);
   const double BdiW = Bd * iW;
   f[0] = u[0] * vd;
   f[1] = fma(u[1], vd, -bx * BdiW);
@@ -228,6 +230,14 @@ __device__ __forceinline__ void srmhd_flux(const double u[9], double vx, double 
   f[6] = DIR == 1 ? u[8] : fma(By, vd, -Bd * vy);
   f[7] = DIR == 2 ? u[8] : fma(Bz, vd, -Bd * vz);
   f[8] = (DIR == 2 && QUIRK_PHI_Z) ? By : Bd;
+}
+
+// Lax-Friedrichs split fluxes, doubled: f + u and f - u, each one rounding
+// (an f that ends in a product is not fused into the sum).
+__device__ __forceinline__ void split_pm(double f, double u, double &fp, double &fm) {
+#pragma clang fp contract(off)
+  fp = f + u;
+  fm = f - u;
 }
 
 // SRMHD::primsToAll for one cell (srmhd.cc:573-673).

@@ -392,8 +392,7 @@ __device__ __forceinline__ void sweep_tile_faces(const SweepArgs &a, double (&s_
           M::template flux<DAX, QUIRK>(u, pl, a, o, f);
   #pragma unroll
           for (int v = 0; v < NV; ++v) {
-            fp[v] = f[v] + u[v];  // doubled
-            fm_keep[cp][v] = f[v] - u[v];
+            split_pm(f[v], u[v], fp[v], fm_keep[cp][v]);
           }
         }
   #pragma unroll
@@ -477,8 +476,7 @@ __device__ __forceinline__ void sweep_tile_faces(const SweepArgs &a, double (&s_
         M::template flux<DAX, QUIRK>(u, pl, a, o, f);
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
-          fp[v] = f[v] + u[v];  // doubled
-          fm[v] = f[v] - u[v];
+          split_pm(f[v], u[v], fp[v], fm[v]);
         }
       }
 #pragma unroll
@@ -567,8 +565,7 @@ __global__ __launch_bounds__(kThreads) void k_sweep(SweepArgs a) {
           M::template flux<DAX, QUIRK>(u, pl, a, o, f);
   #pragma unroll
           for (int v = 0; v < NV; ++v) {
-            fp[v] = f[v] + u[v];  // doubled
-            fm_keep[cp][v] = f[v] - u[v];
+            split_pm(f[v], u[v], fp[v], fm_keep[cp][v]);
           }
         }
   #pragma unroll
@@ -640,8 +637,7 @@ __global__ __launch_bounds__(kThreads) void k_sweep(SweepArgs a) {
         M::template flux<DAX, QUIRK>(u, pl, a, o, f);
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
-          fp[v] = f[v] + u[v];  // doubled
-          fm[v] = f[v] - u[v];
+          split_pm(f[v], u[v], fp[v], fm[v]);
         }
       }
 #pragma unroll
@@ -920,6 +916,123 @@ __global__ __launch_bounds__(kThreads) void k_sweep_xyf(SweepArgs a) {
   if (MODE >= kSweepStage1) reduce_stats(a.stats, cs.cells, cs.iters, cs.fails, cs.maxit);
 }
 
+// The x sweep of a 3-D grid (write mode) as a march along x, for SRMHD. A lane
+// takes one (y, z) column of the x planes laid end to end, so the 64 lanes of
+// a wave read 512 bytes in a row whatever the extents, and walks the segment's
+// cells with the last 2R - 1 split fluxes of its variables in registers: each
+// cell's flux is formed once per segment, nothing goes through LDS and there
+// is no barrier. The 9 variables are split over the workgroup's three waves
+// (D Sx Sy | Sz tau phi | B), 3 windows of 2 x 5 values each; the B waves need
+// no Lorentz factor. The next two cells' values are on their way meanwhile.
+// The tiled sweep forms 22/16 (20/16) fluxes a cell and reads rows of 16 cells,
+// which straddle two 128-byte lines on most grids: 128 x 120 x 136 WENO5
+// 152 -> 113 us and WENO3 138 -> 95, 97 x 64 x 130 WENO3 57 -> 47; on aligned
+// rows it gains less, 256^3 WENO5 780-811 -> 757 us (4.1 TB/s of the 176 bytes
+// a cell needs), 128^3 WENO3 113 -> 103.
+template <int ORDER, int G>
+__device__ __forceinline__ void march_x(const SweepArgs &a, unsigned co, bool live, int xs, int xe) {
+  constexpr int R = Weno<ORDER>::R, W = 2 * R - 1;
+  constexpr int v0 = G == 0 ? 0 : (G == 1 ? 3 : 5), v1 = v0 + 1, v2 = G == 1 ? 8 : v0 + 2;
+  constexpr int vars[3] = {v0, v1, v2};
+  const Geo &g = a.geo;
+  const long long vs = g.vstride, plane = g.stride[0];
+  const int nx = g.n[0], px = g.periodic[0];
+  // cons and vx, vy, vz, p of the column's cell at x index i
+  struct Cell {
+    double u[9], pl[4];
+  };
+  // (the offset is made anew in each block, which is where the compiler looks
+  // for the extension that lets it ride in the access)
+  auto load = [&](int i, Cell &c) {
+    unsigned o = co;
+    asm("" : "+v"(o));
+    const double *U = a.U + remap(i, nx, px) * plane, *V = a.V + remap(i, nx, px) * plane;
+#pragma unroll
+    for (int v = 0; v < 9; ++v)
+      c.u[v] = (v == v0 || v == v1 || v == v2 || (v >= 5 && v < 8) || (G == 2 && v == 8)) ? ld(U + v * vs, o) : 0.0;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) c.pl[v] = v < 3 || G != 2 ? ld(V + (1 + v) * vs, o) : 0.0;
+  };
+  double fp[3][W], fm[3][W], left[3];
+  // the split fluxes of a cell into slot s of the windows (f+ after, f- before
+  // the faces that end there)
+  auto split = [&](const Cell &c, double sp[3], double sm[3]) {
+    double f[9];
+    srmhd_flux<0, false>(c.u, c.pl[0], c.pl[1], c.pl[2], c.pl[3], f);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) split_pm(f[vars[k]], c.u[vars[k]], sp[k], sm[k]);
+  };
+  const int last = xe + R - 1;
+  Cell cur, nxt, far;
+  load(xs - R, nxt);
+  load(xs - R + 1, far);
+#pragma unroll
+  for (int s = 0; s < W; ++s) {
+    cur = nxt;
+    nxt = far;
+    load(min(xs - R + s + 2, last), far);
+    asm volatile("" : : : "memory");
+    double sp[3], sm[3];
+    split(cur, sp, sm);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      fp[k][s] = sp[k];
+      fm[k][s] = sm[k];
+    }
+  }
+  // face j (left of cell j) ends at cell j + R - 1, whose window slot is (j - xs) mod W
+  double *out = a.fnet + (long long)(xs - 1) * plane;
+  const double half = g.half_inv_d[0];
+#pragma unroll 1
+  for (int base = xs; base <= xe; base += W) {
+#pragma unroll
+    for (int s = 0; s < W; ++s) {
+      if (base + s <= xe) {
+        cur = nxt;
+        nxt = far;
+        load(min(base + s + R + 1, last), far);
+        asm volatile("" : : : "memory");
+        double sp[3], sm[3];
+        split(cur, sp, sm);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          double nu, du, nd, dd;
+          Weno<ORDER, true>::up([&](int m) { return fp[k][(s + m) % W]; }, nu, du);
+          fm[k][s] = sm[k];
+          Weno<ORDER, true>::down([&](int m) { return fm[k][(s + m) % W]; }, nd, dd);
+          fp[k][s] = sp[k];
+          const double face = weno_combine(nu, du, nd, dd);
+          if (live && base + s > xs) {
+            unsigned o = co;
+            asm("" : "+v"(o));
+            st_nt(out + vars[k] * vs, o, (face - left[k]) * half);
+          }
+          left[k] = face;
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        out += plane;
+      }
+    }
+  }
+}
+
+constexpr int kMarchThreads = 192;  // three waves of 64 columns
+
+template <int ORDER>
+__global__ __launch_bounds__(kMarchThreads, ORDER == 5 ? 2 : 4) void k_march_x(SweepArgs a, int nseg, int len) {
+  const int lb = xcd_block(blockIdx.x, gridDim.x);
+  const int cols = (int)a.geo.stride[0], nb = gridDim.x / nseg;
+  const int seg = lb / nb, col = (lb - seg * nb) * 64 + (threadIdx.x & 63);
+  const int xs = seg * len, xe = min(xs + len, a.geo.n[0]);
+  const bool live = col < cols;
+  const unsigned co = min(col, cols - 1) * 8u;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (w == 0) march_x<ORDER, 0>(a, co, live, xs, xe);
+  else if (w == 1) march_x<ORDER, 1>(a, co, live, xs, xe);
+  else march_x<ORDER, 2>(a, co, live, xs, xe);
+}
+
 // Fused z and y sweeps of a 3-D grid (FVS::F's z and y terms,
 // fluxVectorSplitting.cc:92-112). A TYT x TZT tile of one x plane
 // reconstructs its z faces, then its y faces, through LDS, and accumulates
@@ -947,8 +1060,7 @@ __device__ __forceinline__ void split_cell(const SweepArgs &a, long long q, doub
   M::template flux<DIR, QUIRK>(u, pl, a, (unsigned)q * 8u, f);
 #pragma unroll
   for (int v = 0; v < M::NC; ++v) {
-    fp[v] = f[v] + u[v];  // doubled
-    fm[v] = f[v] - u[v];
+    split_pm(f[v], u[v], fp[v], fm[v]);
   }
 }
 
@@ -1709,6 +1821,18 @@ __global__ __launch_bounds__(kThreads) void k_flux_vector_srrmhd(Geo g, PadGeo p
 // As in 2-D, 8 x 8 tiles then shorten the workgroup's chain of passes.
 inline bool small_3d(const Geo &g) { return ((g.n[1] + 15LL) / 16) * ((g.n[2] + 15) / 16) * g.n[0] <= 256; }
 
+// Segments along x of the marching x sweep, or 0 where the tiled one is used:
+// about 4,600 waves (three rounds of 1,536 at two per SIMD overlap their ends)
+// of segments no shorter than 16 cells, whose 5 cells of lead-in are loaded and
+// split for nothing. A wave is one long chain, so a grid that fills fewer than
+// 1,536 is faster on tiles (64^3, 768 waves: 21.8 us against 15.8; 160 x 61 x
+// 33, 960: 35 against 33 with WENO5; 97 x 64 x 130, 2,340: 55 against 64).
+inline int march_segments(const Geo &g) {
+  const long long nb = (g.stride[0] + 63) / 64;
+  const long long nseg = std::max(1LL, std::min((1536 + nb / 2) / nb, (long long)g.n[0] / 16));
+  return 3 * nb * nseg < 1536 ? 0 : (int)nseg;
+}
+
 // Cells per workgroup along the only axis of a 1-D grid: one pencil of 32, so
 // that the 297 (variable, face) items of SRMHD take two passes of the threads
 // and 400 cells 13 workgroups. On the 16 x 16 tile of the strided x sweep 15
@@ -1733,6 +1857,14 @@ void launch_sweep_t(const SweepArgs &a, int quirk, hipStream_t s) {
 template <class M, int ORDER, int MODE>
 void launch_sweep_o(const SweepArgs &a, int dir, int quirk, hipStream_t s) {
   if (a.geo.dims == 3) {
+    if constexpr (MODE == kSweepWrite && !M::kStored && M::NC <= 9) {
+      const int nseg = dir == 0 ? march_segments(a.geo) : 0;
+      if (nseg > 0) {
+        const int nb = (int)((a.geo.stride[0] + 63) / 64), len = (a.geo.n[0] + nseg - 1) / nseg;
+        hipLaunchKernelGGL(k_march_x<ORDER>, dim3(nb * nseg), dim3(kMarchThreads), 0, s, a, nseg, len);
+        return;
+      }
+    }
     if constexpr (MODE == kSweepWrite && !M::kStored) {
       if (dir == 0 && small_3d(a.geo)) {
         launch_sweep_t<M, ORDER, 0, 2, false, MODE, 8, 8>(a, quirk, s);
