@@ -88,7 +88,7 @@ struct mgpu_engine {
   int fused_yz = 0;                      // 3-D: fused z+y sweep launch (off: slower here)
   int xyz_order = 1;                     // 3-D: sweeps x, y, z with the last (contiguous) one finishing
   int fused_yzf = 1;                     // plan 3: 3-D x sweep, then y + z as one launch; 2-D y + x as one
-  // SRMHD RK2 and RKSplit steps keep the cons2prim root (v^2, Z) of each cell
+  // SRMHD steps (RK4_10's aside) keep the cons2prim root (v^2, Z) of each cell
   // instead of writing its 13 aux values, and SRRMHD SSP2 steps the root Z
   // instead of 17: no kernel of those steps reads aux, and what does (state
   // download, wavespeed) forms it from the root first.
@@ -191,24 +191,26 @@ int run_sweeps(mgpu_engine *e, SweepArgs a, int last_mode) {
     if (mark(e, "sweep_yz_write")) return -1;
     const int mode = (last_mode == kSweepWrite || last_mode == kSweepAdd) ? kSweepAdd : last_mode;
     launch_sweep(a, e->cfg.model, order, 0, mode, quirk, e->stream);
-    static const char *xnames[6] = {"sweep_x_write", "sweep_x_add", "sweep_x_stage1_c2p", "sweep_x_stage2_c2p",
-                                    "sweep_x_imex2", "sweep_x_final"};
+    static const char *xnames[7] = {"sweep_x_write", "sweep_x_add", "sweep_x_stage1_c2p", "sweep_x_stage2_c2p",
+                                    "sweep_x_imex2", "sweep_x_final", "sweep_x_rk_c2p"};
     if (mark(e, xnames[mode])) return -1;
     HIP_OK(hipGetLastError());
     return 0;
   }
-  static const char *names[3][6] = {
-      {"sweep_x_write", "sweep_x_add", "sweep_x_stage1_c2p", "sweep_x_stage2_c2p", "sweep_x_imex2", "sweep_x_final"},
-      {"sweep_y_write", "sweep_y_add", "sweep_y_stage1_c2p", "sweep_y_stage2_c2p", "sweep_y_imex2", "sweep_y_final"},
+  static const char *names[3][7] = {
+      {"sweep_x_write", "sweep_x_add", "sweep_x_stage1_c2p", "sweep_x_stage2_c2p", "sweep_x_imex2", "sweep_x_final",
+       "sweep_x_rk_c2p"},
+      {"sweep_y_write", "sweep_y_add", "sweep_y_stage1_c2p", "sweep_y_stage2_c2p", "sweep_y_imex2", "sweep_y_final",
+       "sweep_y_rk_c2p"},
       {"sweep_z_write", "sweep_z_add", "sweep_z_stage1_c2p", "sweep_z_stage2_c2p", "sweep_z_imex2",
-       "sweep_z_final"}};
+       "sweep_z_final", "sweep_z_rk_c2p"}};
   if (dims == 3 && e->fused_yzf) {
     launch_sweep(a, e->cfg.model, order, 0, kSweepWrite, quirk, e->stream);
     if (mark(e, names[0][kSweepWrite])) return -1;
     const int mode = (last_mode == kSweepWrite || last_mode == kSweepAdd) ? kSweepAdd : last_mode;
     launch_sweep_yzf(a, e->cfg.model, order, mode, quirk, e->stream);
-    static const char *yzf_names[6] = {"sweep_yz_add", "sweep_yz_add", "sweep_yz_stage1_c2p",
-                                       "sweep_yz_stage2_c2p", "sweep_yz_imex2", "sweep_yz_final"};
+    static const char *yzf_names[7] = {"sweep_yz_add", "sweep_yz_add", "sweep_yz_stage1_c2p",
+                                       "sweep_yz_stage2_c2p", "sweep_yz_imex2", "sweep_yz_final", "sweep_yz_rk_c2p"};
     if (mark(e, yzf_names[mode])) return -1;
     HIP_OK(hipGetLastError());
     return 0;
@@ -216,8 +218,8 @@ int run_sweeps(mgpu_engine *e, SweepArgs a, int last_mode) {
   if (dims == 2 && e->fused_yzf) {
     const int mode = (last_mode == kSweepWrite || last_mode == kSweepAdd) ? kSweepAdd : last_mode;
     launch_sweep_xyf(a, e->cfg.model, order, mode, e->stream);
-    static const char *xyf_names[6] = {"sweep_yx_add", "sweep_yx_add", "sweep_yx_stage1_c2p",
-                                       "sweep_yx_stage2_c2p", "sweep_yx_imex2", "sweep_yx_final"};
+    static const char *xyf_names[7] = {"sweep_yx_add", "sweep_yx_add", "sweep_yx_stage1_c2p",
+                                       "sweep_yx_stage2_c2p", "sweep_yx_imex2", "sweep_yx_final", "sweep_yx_rk_c2p"};
     if (mark(e, xyf_names[mode])) return -1;
     HIP_OK(hipGetLastError());
     return 0;
@@ -390,10 +392,10 @@ RkStageArgs rk_args(mgpu_engine *e, double dt, C2PCounters *st) {
 int rk_rhs(mgpu_engine *e, RkStageArgs &a, const double *Ub, const double *Vb, const double *Ab) {
   SweepArgs s = sweep_args(e, Ub, Vb, nullptr);
   if (run_sweeps(e, s, kSweepAdd)) return -1;
-  a.Ub = Ub;
-  a.Ab = Ab;
+  a.t.Ub = Ub;
+  a.t.Ab = Ab;
   a.fnet = e->fnet;
-  a.ext = extension_source(e, Vb);
+  a.t.ext = extension_source(e, Vb);
   HIP_OK(hipGetLastError());
   return 0;
 }
@@ -413,10 +415,10 @@ int rk_rhs_stored(mgpu_engine *e, RkStageArgs &a, const double *Ub, const double
     HIP_OK(hipGetLastError());
     if (mark(e, "sweep_stored")) return -1;
   }
-  a.Ub = Ub;
-  a.Ab = Ab;
+  a.t.Ub = Ub;
+  a.t.Ab = Ab;
   a.fnet = e->fnet;
-  a.ext = extension_source(e, Vb);
+  a.t.ext = extension_source(e, Vb);
   HIP_OK(hipGetLastError());
   return 0;
 }
@@ -431,11 +433,11 @@ int rk_finish(mgpu_engine *e, const RkStageArgs &a, C2PCounters *st) {
 }
 
 void rk_terms(RkStageArgs &a, std::initializer_list<const double *> x, std::initializer_list<double> w) {
-  a.nx = 0;
+  a.t.nx = 0;
   auto wi = w.begin();
   for (const double *p : x) {
-    a.X[a.nx] = p;
-    a.w[a.nx++] = *wi++;
+    a.t.X[a.t.nx] = p;
+    a.t.w[a.t.nx++] = *wi++;
   }
 }
 
@@ -448,43 +450,66 @@ void rk_out(RkStageArgs &a, double *U, double *V, double *A, const double *Vg) {
 
 // RK2B, RK3, RK4 and RK4_10::step (RKPlus.cc:127-726). A stage's cons2prim
 // starts from the previous stage's prims, the last stage's from the step's.
+// The rhs of (Ub, Vb, Ab) and the stage a (whose terms and outputs are set)
+// from it, in the sweeps' own launches: the last sweep combines the stage and
+// runs its cons2prim, so the net flux of a 2-D grid never goes to HBM and no
+// pointwise launch follows (RK4 200^2 WENO3, a step of five stages with their
+// retries: 106 us as sweep and stage launches, now 77). The stage's output must be another state than the
+// one swept. Only the last stage needs prims beyond rho .. p, unless the model
+// extension reads them, and SRMHD's aux is kept as its root there.
+int rk_stage(mgpu_engine *e, const RkStageArgs &a, const double *Ub, const double *Vb, const double *Ab,
+             C2PCounters *st, bool last = false) {
+  const bool res = e->cfg.model != MGPU_SRMHD;
+  SweepArgs s = sweep_args(e, Ub, Vb, st);
+  s.dt = a.dt;
+  s.rk = a.t;
+  s.rk.Ub = Ub;
+  s.rk.Ab = Ab;
+  s.rk.ext = extension_source(e, Vb);
+  s.Vg = a.Vg;
+  s.Uout = a.Uout;
+  s.Vout = a.Vout;
+  s.Aout = res ? a.Aout : nullptr;
+  s.root = last ? e->root : nullptr;
+  s.vout_n = last || s.rk.ext ? 0 : 5;
+  if (run_sweeps(e, s, kSweepRk)) return -1;
+  if (retry(e, a.Uout, a.Vout, s.Aout, st, s.root)) return -1;
+  if (last && s.root) e->aux_stale = true;
+  return 0;
+}
+
 int rkplus_step(mgpu_engine *e, double dt, C2PCounters *st) {
   double *U = e->U, *V = e->V, *A = e->A;
   double **Us = e->rkU, **Vs = e->rkV, **As = e->rkA;
   switch (e->cfg.integrator) {
     case MGPU_RK2B: {
       RkStageArgs a = rk_args(e, dt, st);
-      if (rk_rhs(e, a, U, V, A)) return -1;
       rk_terms(a, {U}, {1.0});
-      a.wr = 1.0;
+      a.t.wr = 1.0;
       rk_out(a, Us[0], Vs[0], As[0], V);
-      if (rk_finish(e, a, st)) return -1;
+      if (rk_stage(e, a, U, V, A, st)) return -1;
       RkStageArgs b = rk_args(e, dt, st);
-      if (rk_rhs(e, b, Us[0], Vs[0], As[0])) return -1;
       rk_terms(b, {U, Us[0]}, {1.0, 1.0});
-      b.half_sum = 1;
+      b.t.half_sum = 1;
       rk_out(b, U, V, A, V);
-      return rk_finish(e, b, st);
+      return rk_stage(e, b, Us[0], Vs[0], As[0], st, true);
     }
     case MGPU_RK3: {
       RkStageArgs a = rk_args(e, dt, st);
-      if (rk_rhs(e, a, U, V, A)) return -1;
       rk_terms(a, {U}, {1.0});
-      a.wr = 1.0;
+      a.t.wr = 1.0;
       rk_out(a, Us[0], Vs[0], As[0], V);
-      if (rk_finish(e, a, st)) return -1;
+      if (rk_stage(e, a, U, V, A, st)) return -1;
       RkStageArgs b = rk_args(e, dt, st);
-      if (rk_rhs(e, b, Us[0], Vs[0], As[0])) return -1;
       rk_terms(b, {U, Us[0]}, {3.0 / 4.0, 1.0 / 4.0});
-      b.wr = 1.0 / 4.0;
+      b.t.wr = 1.0 / 4.0;
       rk_out(b, Us[1], Vs[1], As[1], Vs[0]);
-      if (rk_finish(e, b, st)) return -1;
+      if (rk_stage(e, b, Us[0], Vs[0], As[0], st)) return -1;
       RkStageArgs c = rk_args(e, dt, st);
-      if (rk_rhs(e, c, Us[1], Vs[1], As[1])) return -1;
       rk_terms(c, {U, Us[1]}, {1.0 / 3.0, 2.0 / 3.0});
-      c.wr = 2.0 / 3.0;
+      c.t.wr = 2.0 / 3.0;
       rk_out(c, U, V, A, V);
-      return rk_finish(e, c, st);
+      return rk_stage(e, c, Us[1], Vs[1], As[1], st, true);
     }
     case MGPU_RK4: {
       // RK4::stage1..stage5 (RKPlus.cc:330-470)
@@ -494,24 +519,22 @@ int rkplus_step(mgpu_engine *e, double dt, C2PCounters *st) {
       for (int k = 0; k < 4; ++k) {
         const double *Ub = k ? Us[k - 1] : U, *Vb = k ? Vs[k - 1] : V, *Ab = k ? As[k - 1] : A;
         RkStageArgs a = rk_args(e, dt, st);
-        if (rk_rhs(e, a, Ub, Vb, Ab)) return -1;
         if (k)
           rk_terms(a, {U, Us[k - 1]}, {wn[k], wp[k]});
         else
           rk_terms(a, {U}, {wn[0]});
-        a.wr = wr[k];
-        if (k == 3) a.Rout = e->rkR;
+        a.t.wr = wr[k];
+        if (k == 3) a.t.Rout = e->rkR;
         rk_out(a, Us[k], Vs[k], As[k], Vb);
-        if (rk_finish(e, a, st)) return -1;
+        if (rk_stage(e, a, Ub, Vb, Ab, st)) return -1;
       }
       RkStageArgs a = rk_args(e, dt, st);
-      if (rk_rhs(e, a, Us[3], Vs[3], As[3])) return -1;
       rk_terms(a, {Us[1], Us[2], Us[3]}, {0.517231671970585, 0.096059710526147, 0.386708617503269});
-      a.R = e->rkR;
-      a.wR = 0.063692468666290;
-      a.wr = 0.226007483236906;
+      a.t.R = e->rkR;
+      a.t.wR = 0.063692468666290;
+      a.t.wr = 0.226007483236906;
       rk_out(a, U, V, A, V);
-      return rk_finish(e, a, st);
+      return rk_stage(e, a, Us[3], Vs[3], As[3], st, true);
     }
     default: {
       // RK4_10::prepare1, stageRepeat x 5, prepare2, stageRepeat x 4,
@@ -546,14 +569,14 @@ int rkplus_step(mgpu_engine *e, double dt, C2PCounters *st) {
           return -1;
         }
         rk_terms(a, {Us[0]}, {1.0});
-        a.wr = 1.0 / 6.0;
+        a.t.wr = 1.0 / 6.0;
         rk_out(a, Us[0], Vs[0], As[0], Vs[0]);
         if (rk_finish(e, a, st)) return -1;
       }
       RkStageArgs a = rk_args(e, dt, st);
       if (rk_rhs(e, a, Us[0], Vs[0], As[0])) return -1;
       rk_terms(a, {Us[1], Us[0]}, {1.0, 3.0 / 5.0});
-      a.wr = 1.0 / 10.0;
+      a.t.wr = 1.0 / 10.0;
       rk_out(a, U, V, A, V);
       return rk_finish(e, a, st);
     }
@@ -680,7 +703,7 @@ int mgpu_create(const mgpu_config *cfg, mgpu_engine **out) {
       return cleanup(fail("hipMalloc of %zu bytes failed", b.elems * sizeof(double)));
     if (hipMemset(*b.ptr, 0, b.elems * sizeof(double)) != hipSuccess) return cleanup(fail("hipMemset failed"));
   }
-  if (c.model == MGPU_SRMHD && (c.integrator == MGPU_RK2 || c.integrator == MGPU_RKSPLIT)) {
+  if (c.model == MGPU_SRMHD && c.integrator != MGPU_RK4_10) {
     if (hipMalloc(&e->root, 2 * n * sizeof(double)) != hipSuccess)
       return cleanup(fail("hipMalloc of the cons2prim root store failed"));
   }

@@ -317,6 +317,52 @@ __device__ __forceinline__ void imex_final_apply(const SweepArgs &a, unsigned o,
 template <class M>
 __device__ __forceinline__ void finish_rk2(const SweepArgs &, unsigned, const double *, StoredM<M>, CellC2P &) {}
 
+// The combined cons of an RKPlus stage at one cell (RkTerms): r is -fnet on
+// entry (zero without a rhs) and gets the source of the rhs state
+// (Model::sourceTerm, srmhd.cc:233-250, srrmhd.cc:194-207, plus the model
+// extension's, RKPlus.cc:26-38).
+template <class M>
+__device__ __forceinline__ void rk_combine(const RkTerms &t, long long vs, unsigned o, double dt, double cp,
+                                           bool with_rhs, double r[M::NC], double un[M::NC]) {
+  constexpr int NC = M::NC;
+  if (with_rhs) {
+    if constexpr (NC == kSrrmhdCons) {
+      double u[kSrrmhdCons], A[kSrrmhdAux], s5[5];
+#pragma unroll
+      for (int v = 8; v < kSrrmhdCons; ++v) u[v] = ld(t.Ub + v * vs, o);
+#pragma unroll
+      for (int v = 4; v < 7; ++v) A[v] = ld(t.Ab + v * vs, o);
+      srrmhd_source5(u, A, cp, s5);
+#pragma unroll
+      for (int m = 0; m < 5; ++m) r[8 + m] = s5[m] + r[8 + m];
+    } else {
+      r[8] = -ld(t.Ub + 8 * vs, o) / (cp * cp) + r[8];
+      if (t.ext) {
+#pragma unroll
+        for (int v = 0; v < 8; ++v) r[v] = ld(t.ext + v * vs, o) + r[v];
+      }
+    }
+  }
+  if (t.half_sum) {
+#pragma unroll
+    for (int v = 0; v < NC; ++v) un[v] = 0.5 * fma(dt, r[v], ld(t.X[0] + v * vs, o) + ld(t.X[1] + v * vs, o));
+  } else {
+    const double cr = t.wr * dt, cR = t.wR * dt;
+#pragma unroll
+    for (int v = 0; v < NC; ++v) {
+      double acc = t.w[0] * ld(t.X[0] + v * vs, o);
+      if (t.nx > 1) acc = fma(t.w[1], ld(t.X[1] + v * vs, o), acc);
+      if (t.nx > 2) acc = fma(t.w[2], ld(t.X[2] + v * vs, o), acc);
+      if (t.R) acc = fma(cR, ld(t.R + v * vs, o), acc);
+      un[v] = fma(cr, r[v], acc);
+    }
+  }
+  if (t.Rout) {
+#pragma unroll
+    for (int v = 0; v < NC; ++v) st(t.Rout + v * vs, o, r[v]);
+  }
+}
+
 // What a sweep does with a cell's net flux fn once its own axis is added
 // (the sweep's mode): keep it for the next sweep, or finish the stage there.
 template <class M, int MODE>
@@ -336,6 +382,12 @@ __device__ __forceinline__ void sweep_apply(const SweepArgs &a, unsigned o, cons
       for (int v = 0; v < NV; ++v)
         un[v] = rk2_stage2(ld_nt(a.Un + v * vs, o), ld(a.U + v * vs, o), fn[v], a.dt);
     }
+    finish_rk2(a, o, un, M(), cs);
+  } else if (MODE == kSweepRk) {
+    double r[NV], un[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) r[v] = -fn[v];
+    rk_combine<M>(a.rk, vs, o, a.dt, a.cp, true, r, un);
     finish_rk2(a, o, un, M(), cs);
   } else if (MODE == kSweepImex2) {
     imex2_apply(a, o, fn, cs);
@@ -690,24 +742,7 @@ __global__ __launch_bounds__(kThreads) void k_sweep(SweepArgs a) {
       for (int v = 0; v < NV; ++v)
         fn[v] = fma(s_f[S::gidx(v, l + 1, cc)] - s_f[S::gidx(v, l, cc)], inv_d,
                     TC_ == 1 ? 0.0 : ld(a.fnet + v * vs, o));
-      if (MODE == kSweepAdd) {
-#pragma unroll
-        for (int v = 0; v < NV; ++v) st(a.fnet + v * vs, o, fn[v]);
-      } else if (MODE == kSweepStage1 || MODE == kSweepStage2) {
-        double un[NV];
-        if (MODE == kSweepStage1) {
-#pragma unroll
-          for (int v = 0; v < NV; ++v) un[v] = rk2_stage1(ld(a.U + v * vs, o), fn[v], a.dt);
-        } else {
-#pragma unroll
-          for (int v = 0; v < NV; ++v) un[v] = rk2_stage2(ld(a.Un + v * vs, o), ld(a.U + v * vs, o), fn[v], a.dt);
-        }
-        finish_rk2(a, o, un, M(), cs);
-      } else if (MODE == kSweepImex2) {
-        imex2_apply(a, o, fn, cs);
-      } else if (MODE == kSweepImexFinal) {
-        imex_final_apply(a, o, fn, cs);
-      }
+      sweep_apply<M, MODE>(a, o, fn, cs);
     }
   }
   if (MODE >= kSweepStage1) reduce_stats(a.stats, cs.cells, cs.iters, cs.fails, cs.maxit);
@@ -1638,51 +1673,10 @@ __global__ __launch_bounds__(kThreads) void k_rkplus_stage(RkStageArgs a) {
   CellC2P cs;
   if (q < a.geo.vstride) {
     const long long vs = a.geo.vstride;
-    double r[NC];
+    double r[NC], un[NC];
 #pragma unroll
-    for (int v = 0; v < NC; ++v) r[v] = 0.0;
-    if (a.fnet) {
-      // Model::sourceTerm of the state whose rhs this is (srmhd.cc:233-250,
-      // srrmhd.cc:194-207), minus its net flux
-      if constexpr (kRes) {
-        double u[kSrrmhdCons], A[kSrrmhdAux], s5[5];
-#pragma unroll
-        for (int v = 0; v < kSrrmhdCons; ++v) u[v] = a.Ub[v * vs + q];
-#pragma unroll
-        for (int v = 4; v < 7; ++v) A[v] = a.Ab[v * vs + q];
-        srrmhd_source5(u, A, a.cp, s5);
-#pragma unroll
-        for (int m = 0; m < 5; ++m) r[8 + m] = s5[m];
-      } else {
-        r[8] = -a.Ub[8 * vs + q] / (a.cp * a.cp);
-        if (a.ext) {
-          // the model extension's source (RKPlus.cc:26-38) on variables 0..7
-#pragma unroll
-          for (int v = 0; v < 8; ++v) r[v] = r[v] + a.ext[v * vs + q];
-        }
-      }
-#pragma unroll
-      for (int v = 0; v < NC; ++v) r[v] = r[v] - a.fnet[v * vs + q];
-    }
-    double un[NC];
-    if (a.half_sum) {
-#pragma unroll
-      for (int v = 0; v < NC; ++v) un[v] = 0.5 * (a.X[0][v * vs + q] + a.X[1][v * vs + q] + a.dt * r[v]);
-    } else {
-      const double cr = a.wr * a.dt, cR = a.wR * a.dt;
-#pragma unroll
-      for (int v = 0; v < NC; ++v) {
-        double acc = a.w[0] * a.X[0][v * vs + q];
-        for (int m = 1; m < a.nx; ++m) acc += a.w[m] * a.X[m][v * vs + q];
-        if (a.R) acc += cR * a.R[v * vs + q];
-        acc += cr * r[v];
-        un[v] = acc;
-      }
-    }
-    if (a.Rout) {
-#pragma unroll
-      for (int v = 0; v < NC; ++v) a.Rout[v * vs + q] = r[v];
-    }
+    for (int v = 0; v < NC; ++v) r[v] = a.fnet ? -a.fnet[v * vs + q] : 0.0;
+    rk_combine<M>(a.t, vs, (unsigned)q * 8u, a.dt, a.cp, a.fnet != nullptr, r, un);
     if constexpr (kRes) {
       const double Zg = srrmhd_guess_Z(a.Vg[0 * vs + q], a.Vg[1 * vs + q], a.Vg[2 * vs + q], a.Vg[3 * vs + q],
                                        a.Vg[4 * vs + q], a.gamma);
@@ -1894,6 +1888,7 @@ void launch_sweep_m(const SweepArgs &a, int dir, int mode, int quirk, hipStream_
     case kSweepAdd: launch_sweep_o<M, ORDER, kSweepAdd>(a, dir, quirk, s); break;
     case kSweepStage1: launch_sweep_o<M, ORDER, kSweepStage1>(a, dir, quirk, s); break;
     case kSweepStage2: launch_sweep_o<M, ORDER, kSweepStage2>(a, dir, quirk, s); break;
+    case kSweepRk: launch_sweep_o<M, ORDER, kSweepRk>(a, dir, quirk, s); break;
     default:
       if constexpr (M::NC == kSrrmhdCons) {
         if (mode == kSweepImex2) launch_sweep_o<M, ORDER, kSweepImex2>(a, dir, quirk, s);
@@ -1959,6 +1954,7 @@ void launch_sweep_yzf_m(const SweepArgs &a, int mode, int quirk, hipStream_t s) 
     case kSweepAdd: launch_sweep_yzf_o<M, ORDER, kSweepAdd>(a, quirk, s); break;
     case kSweepStage1: launch_sweep_yzf_o<M, ORDER, kSweepStage1>(a, quirk, s); break;
     case kSweepStage2: launch_sweep_yzf_o<M, ORDER, kSweepStage2>(a, quirk, s); break;
+    case kSweepRk: launch_sweep_yzf_o<M, ORDER, kSweepRk>(a, quirk, s); break;
     default:
       if constexpr (M::NC == kSrrmhdCons) {
         if (mode == kSweepImex2) launch_sweep_yzf_o<M, ORDER, kSweepImex2>(a, quirk, s);
@@ -2015,6 +2011,7 @@ void launch_sweep_xyf_m(const SweepArgs &a, int mode, hipStream_t s) {
     case kSweepAdd: launch_sweep_xyf_o<M, ORDER, kSweepAdd>(a, s); break;
     case kSweepStage1: launch_sweep_xyf_o<M, ORDER, kSweepStage1>(a, s); break;
     case kSweepStage2: launch_sweep_xyf_o<M, ORDER, kSweepStage2>(a, s); break;
+    case kSweepRk: launch_sweep_xyf_o<M, ORDER, kSweepRk>(a, s); break;
     default:
       if constexpr (M::NC == kSrrmhdCons) {
         if (mode == kSweepImex2) launch_sweep_xyf_o<M, ORDER, kSweepImex2>(a, s);

@@ -28,9 +28,27 @@ constexpr int kStatBuckets = 128;
 // it to the accumulator, finish an RK2 stage (RK2.cc:58-66 / 81-90, with
 // cons2prim), finish SSP2 stage two (flux1 complete: store it and solve the
 // stage-two implicit equation, SSP2.cc:112-152) or finish the SSP2 step
-// (flux2 complete: final combination and cons2prim, SSP2.cc:156-170).
+// (flux2 complete: final combination and cons2prim, SSP2.cc:156-170), or
+// finish an RKPlus stage (RKPlus.cc:56-726, with cons2prim).
 enum SweepMode { kSweepWrite = 0, kSweepAdd = 1, kSweepStage1 = 2, kSweepStage2 = 3, kSweepImex2 = 4,
-                 kSweepImexFinal = 5 };
+                 kSweepImexFinal = 5, kSweepRk = 6 };
+
+// How an RKPlus stage state is put together per cell: with rhs = source(Ub,
+// Ab) - fnet (RKPlus::rhs, RKPlus.cc:15-50), it is
+//   half_sum: 0.5 (X0 + X1 + dt rhs)                  (RK2B's corrector)
+//   else:     sum_m w[m] Xm + (wR dt) R + (wr dt) rhs
+// with rhs kept in Rout when that is given.
+struct RkTerms {
+  const double *X[4];
+  double w[4];
+  int nx, half_sum;
+  const double *Ub, *Ab;  // the rhs state's cons and (resistive model) aux
+  double wr;
+  const double *R;
+  double wR;
+  double *Rout;
+  const double *ext;  // SRMHD model-extension source of the rhs state (variables 0..7), or null
+};
 
 struct SweepArgs {
   Geo geo;
@@ -54,6 +72,7 @@ struct SweepArgs {
   long long *fail_list;
   unsigned char *fail_flag;
   const double *Fin;  // stored flux vectors [dir][var][cell] (model ids 2, 3)
+  RkTerms rk;         // kSweepRk
 };
 
 // model: 0 SRMHD, 1 SRRMHD, or 2 / 3 for the same models with the flux vector
@@ -108,24 +127,13 @@ void launch_split_srrmhd(const Geo &g, double *U, double *V, double *A, double d
 // (bit patterns of non-negative doubles; out must be zero on entry).
 void launch_max_wavespeed_srmhd(const Geo &g, const double *V, const double *A, unsigned long long *out,
                                 hipStream_t s);
-// One RKPlus stage over interior cells (RKPlus.cc:56-726): with
-// rhs = source(Ub, Ab) - fnet (RKPlus::rhs, RKPlus.cc:15-50; no rhs when fnet
-// is null), the stage state is
-//   half_sum: 0.5 (X0 + X1 + dt rhs)                  (RK2B's corrector)
-//   else:     sum_m w[m] Xm + (wR dt) R + (wr dt) rhs
-// optionally keeping rhs in Rout, then cons2prim from the primitives Vg into
-// (Uout, Vout, Aout); Aout may be null. Uout may alias X0 and Vout Vg.
+// One RKPlus stage over interior cells after its net flux went to fnet (null:
+// no rhs): t's combination, then cons2prim from the primitives Vg into (Uout,
+// Vout, Aout); Aout may be null. Uout may alias X0 and Vout Vg.
 struct RkStageArgs {
   Geo geo;
-  const double *X[4];
-  double w[4];
-  int nx, half_sum;
-  const double *Ub, *Ab, *fnet;
-  double wr;
-  const double *R;
-  double wR;
-  double *Rout;
-  const double *ext;  // SRMHD model-extension source of the rhs state (variables 0..7), or null
+  RkTerms t;
+  const double *fnet;
   const double *Vg;
   double *Uout, *Vout, *Aout;
   double dt, gamma, sigma, cp;

@@ -170,3 +170,36 @@ def test_marching_x_sweep_equals_tiles_bitwise(n, weno, periodic):
             got.append(e.download())
     for a, b in zip(*got):
         assert np.isfinite(a).all() and np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("integrator", [eng.RK2B, eng.RK3, eng.RK4])
+@pytest.mark.parametrize("n,resistive", [((41, 0, 0), False), ((37, 23, 0), False), ((37, 23, 0), True),
+                                         ((230, 229, 0), False), ((9, 14, 11), True)])
+def test_rkplus_stages_in_the_sweeps(integrator, n, resistive):
+    """RKPlus stages are put together by the last sweep, whichever launch that is:
+    the fused one (plan 3) and the separate one that sums in the same order (plan
+    2 in 3-D, 0 in 2-D) give the same bits, the aux among them, which for SRMHD
+    is formed from the kept root and has to be the one of the downloaded prims:
+    h, W and v^2 recomputed from them agree to a few roundings (1e-13)."""
+    print(f"gpu: rkplus {integrator} {n} resistive={resistive}", flush=True)
+    g = idt.Grid(*n, -0.5, 0.5, -1.0, 1.0, 0.0, 1.0)
+    p = idt.kh_prims(g, seed=8)
+    p[5], p[6] = 0.2, 0.1
+    cfg = dict(model=eng.SRMHD, cp=1.0)
+    if resistive:
+        p = np.concatenate([p, -np.cross(p[1:4], p[5:8], axis=0)])
+        cfg = dict(model=eng.SRRMHD, sigma=1.0, cp=1.0)
+    got = []
+    for plan in (3, 2 if n[2] else 0):
+        with eng.Engine(eng.Config(*n, -0.5, 0.5, -1.0, 1.0, 0.0, 1.0, integrator=integrator, **cfg)) as e:
+            e.set_sweep_plan(plan)
+            e.set_prims(p)
+            for _ in range(2):
+                assert e.update_time() == 0
+            got.append(e.download())
+    for a, b in zip(*got):
+        assert np.isfinite(a).all() and np.array_equal(a, b)
+    _, q, a = got[0]
+    v2 = (q[1:4] ** 2).sum(0)
+    assert np.abs(a[9] - v2).max() <= 1e-13
+    assert np.abs(a[1] * np.sqrt(1 - v2) - 1).max() <= 1e-12
