@@ -282,6 +282,7 @@ void launch_flux_recon(const PadGeo &pg, int order, int dir, int nvars, const do
 void launch_c2p_cells(int model, long long n, const double *cons, double *prims, double *aux, double gam,
                       double sigma, CellCounters *partial, CellCounters *total, hipStream_t s) {
   const long long nb = cells_blocks(n);
+  if (nb == 1) partial = total;  // one workgroup's record is the total
   if (nb > 0) {
     if (model == MGPU_SRMHD)
       hipLaunchKernelGGL(k_c2p_cells_srmhd, dim3((unsigned)nb), dim3(kCellThreads), 0, s, n, cons, prims, aux, gam,
@@ -290,8 +291,9 @@ void launch_c2p_cells(int model, long long n, const double *cons, double *prims,
       hipLaunchKernelGGL(k_c2p_cells_srrmhd, dim3((unsigned)nb), dim3(kCellThreads), 0, s, n, cons, prims, aux, gam,
                          sigma, partial);
   }
-  hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(kCellThreads), 0, s, (const CellCounters *)partial, (int)nb,
-                     total);
+  if (nb != 1)
+    hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(kCellThreads), 0, s, (const CellCounters *)partial, (int)nb,
+                       total);
 }
 
 void launch_source_cells(int model, long long n, const double *cons, const double *aux, double cp, double *src,

@@ -100,6 +100,7 @@ struct mgpu_engine {
   double *cells_buf = nullptr;
   size_t cells_elems = 0;
   CellCounters *cells_part = nullptr;
+  CellCounters *cells_total = nullptr;  // pinned host memory that the kernels write a call's total to
   long long cells_part_n = 0;
 };
 
@@ -732,6 +733,8 @@ int mgpu_create(const mgpu_config *cfg, mgpu_engine **out) {
     if (c.integrator == MGPU_RK4_10 && hipMalloc(&e->rkF, n * e->ncons * g.dims * sizeof(double)) != hipSuccess)
       return cleanup(fail("hipMalloc of the RK4_10 flux store failed"));
   }
+  if (hipHostMalloc(reinterpret_cast<void **>(&e->cells_total), sizeof(CellCounters), hipHostMallocDefault) != hipSuccess)
+    return cleanup(fail("hipHostMalloc of the cell-list counters failed"));
   if (hipMalloc(&e->dstats, sizeof(C2PCounters) * kStatBuckets) != hipSuccess || hipMalloc(&e->fail_count, 2 * sizeof(int)) != hipSuccess ||
       hipMalloc(&e->fail_list, n * sizeof(long long)) != hipSuccess || hipMalloc(&e->fail_flag, n) != hipSuccess)
     return cleanup(fail("hipMalloc of C2P work arrays failed"));
@@ -767,6 +770,7 @@ int mgpu_destroy(mgpu_engine *e) {
   if (e->hist) hipFree(e->hist);
   if (e->cells_buf) hipFree(e->cells_buf);
   if (e->cells_part) hipFree(e->cells_part);
+  if (e->cells_total) hipHostFree(e->cells_total);
   if (e->stream) hipStreamDestroy(e->stream);
   delete e;
   return 0;
@@ -1041,16 +1045,14 @@ int mgpu_c2p_cells(mgpu_engine *e, long long n, const double *cons, double *prim
     HIP_OK(hipMemcpyAsync(dp, prims, bp, hipMemcpyHostToDevice, e->stream));
     HIP_OK(hipMemcpyAsync(da, aux, ba, hipMemcpyHostToDevice, e->stream));
   }
-  CellCounters *total = e->cells_part + cells_blocks(n);
-  launch_c2p_cells(e->cfg.model, n, dc, dp, da, e->cfg.gamma, e->cfg.sigma, e->cells_part, total, e->stream);
+  launch_c2p_cells(e->cfg.model, n, dc, dp, da, e->cfg.gamma, e->cfg.sigma, e->cells_part, e->cells_total, e->stream);
   HIP_OK(hipGetLastError());
-  CellCounters t;
   if (n > 0) {
     HIP_OK(hipMemcpyAsync(prims, dp, bp, hipMemcpyDeviceToHost, e->stream));
     HIP_OK(hipMemcpyAsync(aux, da, ba, hipMemcpyDeviceToHost, e->stream));
   }
-  HIP_OK(hipMemcpyAsync(&t, total, sizeof t, hipMemcpyDeviceToHost, e->stream));
   HIP_OK(hipStreamSynchronize(e->stream));
+  const CellCounters t = *e->cells_total;
   if (stats) {
     memset(stats, 0, sizeof *stats);
     stats->cells = (long long)t.cells;
@@ -1070,14 +1072,15 @@ int mgpu_c2p_cells_noalloc(mgpu_engine *e, long long n, const double *cons, doub
   if (n > 0 && (!cons || !prims || !aux)) return fail("mgpu_c2p_cells_noalloc: null array");
   CellCounters *part = noalloc_scratch(e->cfg.device);
   if (!part) return fail("mgpu_c2p_cells_noalloc: no scratch address for device %d", e->cfg.device);
-  // every record the launch reads is written by it first: nothing to clear
-  CellCounters *total = part + cells_blocks(n);
+  // every record the launch reads is written by it first: nothing to clear.
+  // With stats the kernel stores the total where the host reads it after its
+  // wait: the copy that fetched it took 8 us of a 28 us call.
+  CellCounters *total = stats ? e->cells_total : part + cells_blocks(n);
   launch_c2p_cells(e->cfg.model, n, cons, prims, aux, e->cfg.gamma, e->cfg.sigma, part, total, e->stream);
   HIP_OK(hipGetLastError());
   if (!stats) return 0;
-  CellCounters t;
-  HIP_OK(hipMemcpyAsync(&t, total, sizeof t, hipMemcpyDeviceToHost, e->stream));
   HIP_OK(hipStreamSynchronize(e->stream));
+  const CellCounters t = *e->cells_total;
   memset(stats, 0, sizeof *stats);
   stats->cells = (long long)t.cells;
   stats->iterations = (long long)t.iterations;
