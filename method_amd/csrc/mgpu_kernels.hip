@@ -955,15 +955,20 @@ __global__ __launch_bounds__(kThreads) void k_sweep_xyf(SweepArgs a) {
 // takes one (y, z) column of the x planes laid end to end, so the 64 lanes of
 // a wave read 512 bytes in a row whatever the extents, and walks the segment's
 // cells with the last 2R - 1 split fluxes of its variables in registers: each
-// cell's flux is formed once per segment, nothing goes through LDS and there
-// is no barrier. The 9 variables are split over the workgroup's three waves
-// (D Sx Sy | Sz tau phi | B), 3 windows of 2 x 5 values each; the B waves need
-// no Lorentz factor. The next two cells' values are on their way meanwhile.
-// The tiled sweep forms 22/16 (20/16) fluxes a cell and reads rows of 16 cells,
-// which straddle two 128-byte lines on most grids: 128 x 120 x 136 WENO5
-// 152 -> 113 us and WENO3 138 -> 95, 97 x 64 x 130 WENO3 57 -> 47; on aligned
-// rows it gains less, 256^3 WENO5 780-811 -> 757 us (4.1 TB/s of the 176 bytes
-// a cell needs), 128^3 WENO3 113 -> 103.
+// cell's flux is formed once per segment and nothing goes through LDS. The 9
+// variables are split over the workgroup's three waves (D Sx Sy | Sz tau phi |
+// B), 3 windows of 2 x 5 values each; the B waves need no Lorentz factor. The
+// next two cells' values are on their way meanwhile. The tiled sweep forms
+// 22/16 (20/16) fluxes a cell and reads rows of 16 cells, which straddle two
+// 128-byte lines on most grids: 128 x 120 x 136 WENO5 152 -> 113 us and WENO3
+// 138 -> 95, 97 x 64 x 130 WENO3 57 -> 48; on aligned rows it gains less,
+// 256^3 WENO5 780-811 -> 752 us (5.6 TB/s), 128^3 WENO3 113 -> 103.
+// The three waves read the same prims and B and drift apart until the L2 has
+// dropped them (181 bytes read per cell of 256^3, not 104). A barrier once per
+// window keeps them together (109 bytes): with four waves per SIMD (WENO3) that
+// is faster, 97 x 64 x 130 48.4 -> 44.8 us; with the two that WENO5 has, nothing
+// runs while a wave waits there and 256^3 takes 794 us instead of 752, so WENO5
+// goes without. All waves of a workgroup make the same trips.
 template <int ORDER, int G>
 __device__ __forceinline__ void march_x(const SweepArgs &a, unsigned co, bool live, int xs, int xe) {
   constexpr int R = Weno<ORDER>::R, W = 2 * R - 1;
@@ -1027,6 +1032,7 @@ __device__ __forceinline__ void march_x(const SweepArgs &a, unsigned co, bool li
         nxt = far;
         load(min(base + s + R + 1, last), far);
         asm volatile("" : : : "memory");
+        if (ORDER == 3 && s == 0) __builtin_amdgcn_s_barrier();
         double sp[3], sm[3];
         split(cur, sp, sm);
         __builtin_amdgcn_sched_barrier(0);
