@@ -103,13 +103,14 @@ __device__ __forceinline__ void srrmhd_flux_stored(const double u[14], const dou
 
 // Residual of the recovery equation in Z = rho h W^2 (srrmhd.cc:512-537), with
 // gf = (gam - 1) / gam and iD = 1 / D: v^2 = Sbar^2 / Z^2, 1 / W^2 = 1 - v^2,
-// rho = D / W and h = Z / (rho W^2) = Z / (D W).
+// rho = D / W and h = Z / (rho W^2) = Z / (D W). An undefined Z (or 0 / 0) gives
+// NaN and not the 1e6 of an unphysical one: the secant keeps the iterate of the
+// smallest residual, which a NaN iterate must never become.
 __device__ __forceinline__ double srrmhd_c2p_residual(double Z, double SbSq, double D, double tauBar, double gf,
                                                       double iD) {
-  const double iZ = rcp_pos(Z);
-  const double vsq = SbSq * iZ * iZ;
-  if (!(vsq < 1.0) || Z < 0) return 1.0e6;
-  const double s = 1.0 - vsq;
+  const double Z2 = Z * Z;
+  if ((SbSq >= Z2 && SbSq > 0.0) || Z < 0.0) return 1.0e6;
+  const double s = 1.0 - div_pos(SbSq, Z2);
   const double iW = s * rsqrt_pos(s);
   const double rho = D * iW;
   const double h = Z * iD * iW;
