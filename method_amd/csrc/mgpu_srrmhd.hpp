@@ -161,7 +161,9 @@ __device__ __forceinline__ void srrmhd_aux_of_cons(const double u[14], double A[
 
 // Prims and aux from the cons and the root Z = rho h W^2 (srrmhd.cc:539-581,
 // after the secant): a pure function of (u, Z), so an aux formed later from a
-// kept root equals the one the cons2prim would have written, bit for bit.
+// kept root equals the one the cons2prim would have written, bit for bit. h is
+// formed as in srmhd_recover. The secant may fail and Z be anything (there is no
+// retry), so these divisions keep the IEEE rules for zeros and infinities.
 __device__ __forceinline__ void srrmhd_recover(const double u[14], double gam, double sigma, double Z, double P[11],
                                                double A[17]) {
   P[5] = u[5];
@@ -172,12 +174,13 @@ __device__ __forceinline__ void srrmhd_recover(const double u[14], double gam, d
   P[10] = u[10];
   srrmhd_aux_of_cons(u, A);
   A[10] = Z;
-  const double iZ = rcp_pos(Z);
-  A[9] = A[15] * iZ * iZ;
-  A[1] = rsqrt_pos(1.0 - A[9]);
-  P[0] = u[0] * ((1.0 - A[9]) * A[1]);
-  A[0] = div_pos(Z, P[0] * A[1] * A[1]);
-  A[2] = (A[0] - 1.0) * rcp_pos(gam);
+  const double iZ = 1.0 / Z;
+  A[9] = A[15] / (Z * Z);
+  double iW;
+  A[1] = rsqrt_pos(1.0 - A[9], iW);
+  P[0] = u[0] * iW;
+  A[0] = Z * iW / u[0];
+  A[2] = (A[0] - 1.0) / gam;
   A[3] = sqrt((A[2] * gam * (gam - 1.0)) / A[0]);
   P[4] = P[0] * A[2] * (gam - 1.0);
   P[1] = A[12] * iZ;

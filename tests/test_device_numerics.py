@@ -75,3 +75,79 @@ def test_secant_keeps_the_best_iterate(lib, guess, tauBar):
                 assert abs(Z[k] - z) <= 1e-11 * max(1.0, abs(z)), (k, Z[k], z)
             else:
                 assert np.array_equal(Z[k], z, equal_nan=True), (k, Z[k], z)
+
+
+EPS = 2.0 ** -53  # one rounding
+
+
+def cold_states(n, ratio, W, seed):
+    """rho, p, v, B of n states with p / rho about `ratio` and Lorentz factors up to W."""
+    rng = np.random.default_rng(seed)
+    rho = np.exp(rng.uniform(np.log(0.1), np.log(10.0), n))
+    p = rho * ratio * rng.uniform(0.5, 1.5, n)
+    v = rng.normal(size=(3, n))
+    v *= np.sqrt(1 - 1 / (1 + (W - 1) * rng.uniform(0.01, 1.0, n)) ** 2) / np.sqrt((v * v).sum(0))
+    return rho, p, v, rng.normal(size=(3, n)) * 0.3 * np.sqrt(rho)
+
+
+@pytest.mark.parametrize("ratio", [1.0, 1e-3, 1e-4, 1e-6])
+@pytest.mark.parametrize("W", [1.2, 5.0, 50.0])
+def test_recovery_rounds_h_once(lib, ratio, W):
+    """rho and h from a given root against extended precision, and p, which in a
+    cold cell is what is left of h - 1. With s = 1 - v^2 a rounding of at most
+    1/2 in sqrt(s), sqrt(s), its product and the quotient one each, h is within
+    3.5 roundings (3 more of the rsqrt's would not be) and 1.5 on average (four
+    uniform errors add to 0.5 on average), rho within 2.5; p = (h - 1) rho (gam -
+    1) / gam adds four to h's, weighed by h / (h - 1), and e as many."""
+    n, gam = 20000, 5.0 / 3.0
+    rho, p, v, B = cold_states(n, ratio, W, 5)
+    v2 = (v * v).sum(0)
+    Z = (rho + p * gam / (gam - 1)) / (1 - v2)
+    U = np.ascontiguousarray(np.concatenate([[rho / np.sqrt(1 - v2)], Z * v, [Z], B, 0 * rho[None]]).T)
+    root = np.ascontiguousarray(np.stack([v2, Z], 1))
+    P, A = np.zeros((n, 8)), np.zeros((n, 13))
+    lib.recover(n, ptr(U), ptr(root), ctypes.c_double(gam), ptr(P), ptr(A))
+    L = np.longdouble
+    iW = np.sqrt(1 - L(v2))
+    r, h = L(U[:, 0]) * iW, L(Z) * iW / L(U[:, 0])
+    check_recovered(P[:, 0], P[:, 4], A[:, 0], r, (h - 1) * r * (L(gam) - 1) / L(gam), h)
+
+
+def check_recovered(rho, p, h, r, q, H):
+    def err(x, y):
+        return np.abs((x - y) / y).astype(float) / EPS
+
+    assert err(h, H).max() <= 3.6 and err(h, H).mean() <= 1.0
+    assert err(rho, r).max() <= 2.6
+    weight = (H / (H - 1)).astype(float)
+    assert (err(p, q) / (4 + 3.6 * weight)).max() <= 1.0
+    assert (err(p, q) / (4 + weight)).mean() <= 1.0
+
+
+@pytest.mark.parametrize("ratio", [1.0, 1e-3, 1e-6])
+@pytest.mark.parametrize("W", [1.2, 5.0])
+def test_resistive_recovery_rounds_h_once(lib, ratio, W):
+    """The same for the resistive model, whose root is Z alone: v^2 = Sbar^2 / Z^2
+    takes two more roundings, which W^2 v^2 / 2 weighs in 1/W; the states here have
+    Sbar along x alone (E = 0), so h is within 3.5 + W^2 roundings."""
+    n, gam = 20000, 5.0 / 3.0
+    rho, p, v, B = cold_states(n, ratio, W, 6)
+    v2 = (v * v).sum(0)
+    Z = (rho + p * gam / (gam - 1)) / (1 - v2)
+    zero = 0 * rho
+    U = np.ascontiguousarray(np.stack([rho / np.sqrt(1 - v2), Z * np.sqrt(v2), zero, zero, Z] + [zero] * 9, 1))
+    P, A = np.zeros((n, 11)), np.zeros((n, 17))
+    lib.recover_resistive(n, ptr(U), ptr(Z), ctypes.c_double(gam), ctypes.c_double(10.0), ptr(P), ptr(A))
+    L = np.longdouble
+    vsq = (L(U[:, 1]) / L(Z)) ** 2
+    iW = np.sqrt(1 - vsq)
+    h = L(Z) * iW / L(U[:, 0])
+
+    def err(x, y):
+        return np.abs((x - y) / y).astype(float) / EPS
+
+    W2 = (1 / (1 - vsq)).astype(float)
+    assert (err(A[:, 0], h) / (3.6 + W2)).max() <= 1.0
+    e = (L(A[:, 0]) - 1) / L(gam)  # e and p from the h and rho that were returned: five roundings at most
+    assert err(P[:, 4], L(P[:, 0]) * e * (L(gam) - 1)).max() <= 5.0
+    assert err(A[:, 9], vsq).max() <= 3.1  # Sbar^2, Z^2 and the quotient
