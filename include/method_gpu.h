@@ -76,7 +76,9 @@ const char *mgpu_last_error(void);
 
 /* Allocates device state for one simulation. Replaces the allocations of
  * Simulation::Simulation (Project/CPU/Src/simulation.cc:22-30) and the
- * integrator's work arrays (RK2.cc:5-18, SSP2.cc:13-34, RKPlus.cc:56-586). */
+ * integrator's work arrays (RK2.cc:5-18, SSP2.cc:13-34, RKPlus.cc:56-586). At
+ * most 2^29 interior cells: the kernels index a variable with 32-bit byte
+ * offsets (with the staging of mgpu_upload_state, 2^29 cells take 378 GB). */
 int mgpu_create(const mgpu_config *cfg, mgpu_engine **out);
 int mgpu_destroy(mgpu_engine *e);
 
@@ -275,7 +277,7 @@ typedef struct {
 } mgpu_batch_config;
 
 typedef struct {
-  int nx, ny;      /* interior cells */
+  int nx, ny;      /* interior cells, at most 2^29 */
   double xmin, xmax, ymin, ymax;
   double cfl;
   double end_time; /* the instance stops stepping when t reaches it */

@@ -810,6 +810,9 @@ int mgpu_batch_create(const mgpu_batch_config *cfg, const mgpu_instance *inst, i
   for (int i = 0; i < ninst; ++i) {
     const mgpu_instance &in = inst[i];
     if (in.nx < c.Ng || in.ny < c.Ng) return engine_fail("mgpu_batch_create: instance %d has fewer than Ng cells", i);
+    if ((double)in.nx * in.ny > kMaxCells)
+      return engine_fail("mgpu_batch_create: instance %d has %d x %d cells, more than the maximum of %lld", i, in.nx,
+                         in.ny, kMaxCells);
     if (!(in.xmax > in.xmin) || !(in.ymax > in.ymin) || !(in.cfl > 0.0))
       return engine_fail("mgpu_batch_create: instance %d has a bad domain or cfl", i);
     // An instance that could never step would keep no cons2prim root, and the

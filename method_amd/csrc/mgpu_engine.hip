@@ -646,6 +646,8 @@ int mgpu_create(const mgpu_config *cfg, mgpu_engine **out) {
   const int n2 = c.nz > 0 ? c.nz : 1;
   if (c.nx < c.Ng || (c.ny > 0 && c.ny < c.Ng) || (c.nz > 0 && c.nz < c.Ng))
     return fail("mgpu_create: every active axis needs at least Ng interior cells");
+  if ((double)c.nx * n1 * n2 > kMaxCells)
+    return fail("mgpu_create: %d x %d x %d cells exceed the maximum of %lld per engine", c.nx, n1, n2, kMaxCells);
   HIP_OK(hipSetDevice(c.device));
   // the allocation-free cell-list cons2prim's scratch address on this GPU
   if (noalloc_scratch_setup(c.device))

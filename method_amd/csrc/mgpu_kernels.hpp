@@ -24,6 +24,10 @@ struct C2PCounters {
 };
 constexpr int kStatBuckets = 128;
 
+// Most cells of a grid (of an ensemble: of one instance): the sweeps take a
+// cell's place in a variable's plane as a 32-bit byte offset (mgpu_tile.hpp).
+constexpr long long kMaxCells = 1LL << 29;
+
 // What the last phase of a sweep does with a cell's net flux: write it, add
 // it to the accumulator, finish an RK2 stage (RK2.cc:58-66 / 81-90, with
 // cons2prim), finish SSP2 stage two (flux1 complete: store it and solve the

@@ -62,9 +62,8 @@ __device__ __forceinline__ void pass_end(double &a, double &b) { asm volatile(""
 
 // A cell's place in a variable's plane as a 32-bit byte offset from the
 // plane's base: base and offset then are a scalar pair and one register of the
-// access itself, where a 64-bit index takes an addition or two per access. An
-// engine of 2^29 cells or more could not be given a state: with the staging of
-// an upload it takes 88 doubles a cell and more, 378 GB of the card's 288.
+// access itself, where a 64-bit index takes an addition or two per access. Grids
+// of more than 2^29 cells are refused (kMaxCells).
 // The empty asm keeps the base a scalar pair: left to itself the compiler adds
 // the offset first and then steps that sum from plane to plane.
 // (It hides the pointer's origin too, so the address space is stated.)

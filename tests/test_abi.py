@@ -46,6 +46,17 @@ def test_create_rejects_bad_configuration(kw, msg):
         eng.Engine(_make(**kw))
 
 
+@pytest.mark.parametrize("n", [(2**29 + 1, 0, 0), (23171, 23171, 0), (1024, 1024, 513), (2**31 - 1,) * 3])
+def test_create_refuses_grids_beyond_32_bit_offsets(n):
+    """A cell's byte offset in its plane has 32 bits: more than 2^29 cells are
+    refused before anything is allocated, also where their number overflows."""
+    with pytest.raises(eng.EngineError, match="maximum of 536870912"):
+        eng.Engine(_make(nx=n[0], ny=n[1], nz=n[2], zmin=0.0, zmax=1.0))
+    if n[1]:
+        with pytest.raises(eng.EngineError, match="maximum of 536870912"):
+            eng.Batch([eng.Instance(16, 16), eng.Instance(max(n[0], 23171), max(n[1], 23171))])
+
+
 def test_missing_library_raises(tmp_path):
     saved = eng._lib
     try:
