@@ -70,10 +70,10 @@ struct BatchArgs {
   double *root;          // stage two: cons2prim root (v^2, Z) [2][cell], from which the aux is formed
   double gamma;
   C2PCounters *stats;
-  int *fail_count;
+  int *fail;             // the failed cells' list, see note_failed
   long long *fail_list;
   unsigned char *fail_flag;
-  int *sync;             // kSyncStep apart: 8 per-XCD tile counters, then the workgroups done with a retry
+  int *sync;             // 8 per-XCD tile counters, kSyncStep apart
   int quirks;
 };
 
@@ -280,10 +280,7 @@ __device__ __forceinline__ void batch_tile(const BatchArgs &a, double *s_f, doub
   acc.cells += 1;
   if (its < 0) {
     acc.fails += 1;
-    const int slot = atomicAdd(a.fail_count, 1);
-    const long long q = I.off + (o >> 3);
-    a.fail_list[slot] = q;
-    a.fail_flag[q] = 1;
+    note_failed(a.fail, a.fail_list, a.fail_flag, I.off + (o >> 3));
   } else {
     acc.iters += its;
     acc.maxit = max(acc.maxit, its);
@@ -435,8 +432,6 @@ __global__ void k_batch_clock(const InstDev *inst, Clock *clock, int ninst, int 
 // back, one after the other: a 12-member, 130,000-cell WENO3 step took 145 us
 // with 256 workgroups of 8 x 32 tiles per stage and 231 with 768, against 94
 // and 59 now.
-// As in k_c2p_retry_srmhd, the last workgroup to finish a retry clears the
-// flags and counters.
 template <int STAGE>
 __global__ __launch_bounds__(kThreads) void k_batch_end(BatchArgs a, Clock *clock) {
   if (blockIdx.x == 0) {
@@ -444,8 +439,9 @@ __global__ __launch_bounds__(kThreads) void k_batch_end(BatchArgs a, Clock *cloc
     if (STAGE == 2)
       for (int b = threadIdx.x; b < a.ninst; b += kThreads) clock[b] = next_clock(a.inst[b], clock[b], true);
   }
-  const int nfail = *a.fail_count;
+  const int nfail = a.fail[kFailCount];
   if (nfail == 0) return;
+  const unsigned char mark = (unsigned char)(a.fail[kFailMark] + 1);
   const long long vs = a.vs;
   const double gam = a.gamma;
   for (int f = blockIdx.x * kThreads + threadIdx.x; f < nfail; f += gridDim.x * kThreads) {
@@ -468,7 +464,7 @@ __global__ __launch_bounds__(kThreads) void k_batch_end(BatchArgs a, Clock *cloc
         const int np = pos[ax] + s;
         if (np < 0 || np >= ext[ax] || ext[ax] == 1) continue;
         const long long m = q + s * stride[ax];
-        if (a.fail_flag[m]) continue;
+        if (a.fail_flag[m] == mark) continue;
         double v2, Z;
         srmhd_plain_guess(a.Vout[m], a.Vout[vs + m], a.Vout[2 * vs + m], a.Vout[3 * vs + m], a.Vout[4 * vs + m], gam,
                           v2, Z);
@@ -495,18 +491,7 @@ __global__ __launch_bounds__(kThreads) void k_batch_end(BatchArgs a, Clock *cloc
     }
     if (its < 0) atomicAdd(&a.stats->retry_failures, 1ull);
   }
-  __shared__ int s_last;
-  __threadfence();
-  __syncthreads();
-  if (threadIdx.x == 0) s_last = atomicAdd(&a.sync[kXcds * kSyncStep], 1) == (int)gridDim.x - 1;
-  __syncthreads();
-  if (!s_last) return;
-  __threadfence();
-  for (int f = threadIdx.x; f < nfail; f += kThreads) a.fail_flag[a.fail_list[f]] = 0;
-  if (threadIdx.x == 0) {
-    *a.fail_count = 0;
-    a.sync[kXcds * kSyncStep] = 0;
-  }
+  end_retry(a.fail, a.fail_flag, a.vs);
 }
 
 // ------------------------------------------------------------- dispatch
@@ -570,7 +555,7 @@ struct mgpu_batch {
   int *dtile_inst = nullptr;
   int ntiles = 0;
   C2PCounters *dstats = nullptr;
-  int *fail_count = nullptr;
+  int *fail = nullptr;
   long long *fail_list = nullptr;
   unsigned char *fail_flag = nullptr;
   int *dsync = nullptr;
@@ -646,7 +631,7 @@ BatchArgs stage_args(mgpu_batch *b, int stage) {
   a.py = b->cfg.bc[1] == MGPU_BC_PERIODIC;
   a.gamma = b->cfg.gamma;
   a.stats = b->dstats;
-  a.fail_count = b->fail_count;
+  a.fail = b->fail;
   a.fail_list = b->fail_list;
   a.fail_flag = b->fail_flag;
   a.sync = b->dsync;
@@ -859,11 +844,11 @@ int mgpu_batch_create(const mgpu_batch_config *cfg, const mgpu_instance *inst, i
   if (hipMalloc(&b->dinst, ninst * sizeof(InstDev)) != hipSuccess ||
       hipMalloc(&b->dclock, ninst * sizeof(Clock)) != hipSuccess ||
       hipMalloc(&b->dstats, kStatBuckets * sizeof(C2PCounters)) != hipSuccess ||
-      hipMalloc(&b->fail_count, sizeof(int)) != hipSuccess || hipMalloc(&b->fail_list, n * sizeof(long long)) != hipSuccess ||
-      hipMalloc(&b->fail_flag, n) != hipSuccess || hipMalloc(&b->dsync, (kXcds + 1) * kSyncStep * sizeof(int)) != hipSuccess)
+      hipMalloc(&b->fail, kFailInts * sizeof(int)) != hipSuccess || hipMalloc(&b->fail_list, n * sizeof(long long)) != hipSuccess ||
+      hipMalloc(&b->fail_flag, n) != hipSuccess || hipMalloc(&b->dsync, kXcds * kSyncStep * sizeof(int)) != hipSuccess)
     return cleanup(engine_fail("hipMalloc of batch work arrays failed"));
-  if (hipMemset(b->dclock, 0, ninst * sizeof(Clock)) != hipSuccess || hipMemset(b->fail_count, 0, sizeof(int)) != hipSuccess ||
-      hipMemset(b->fail_flag, 0, n) != hipSuccess || hipMemset(b->dsync, 0, (kXcds + 1) * kSyncStep * sizeof(int)) != hipSuccess ||
+  if (hipMemset(b->dclock, 0, ninst * sizeof(Clock)) != hipSuccess || hipMemset(b->fail, 0, kFailInts * sizeof(int)) != hipSuccess ||
+      hipMemset(b->fail_flag, 0, n) != hipSuccess || hipMemset(b->dsync, 0, kXcds * kSyncStep * sizeof(int)) != hipSuccess ||
       hipMemset(b->dstats, 0, kStatBuckets * sizeof(C2PCounters)) != hipSuccess)
     return cleanup(engine_fail("hipMemset failed"));
   // default tuning until the autotuner runs: 16 x 16 tiles, static schedule,
@@ -886,7 +871,7 @@ int mgpu_batch_destroy(mgpu_batch *b) {
   double *bufs[] = {b->U, b->V, b->A, b->root, b->U1, b->V1, b->stage_pad, b->backup};
   for (double *p : bufs)
     if (p) hipFree(p);
-  void *other[] = {b->dinst, b->dclock, b->dclock_backup, b->dtile_inst, b->dstats, b->fail_count, b->fail_list,
+  void *other[] = {b->dinst, b->dclock, b->dclock_backup, b->dtile_inst, b->dstats, b->fail, b->fail_list,
                    b->fail_flag, b->dsync};
   for (void *p : other)
     if (p) hipFree(p);

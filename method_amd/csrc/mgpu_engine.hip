@@ -75,7 +75,7 @@ struct mgpu_engine {
   double *staging = nullptr;
   size_t staging_elems = 0;
   C2PCounters *dstats = nullptr;
-  int *fail_count = nullptr;  // failed cells in the list, workgroups done with their retry
+  int *fail = nullptr;  // the failed cells' list, see note_failed
   long long *fail_list = nullptr;
   unsigned char *fail_flag = nullptr;
   double t = 0.0, dt = 0.0, dx = 0.0, dy = 0.0, dz = 0.0;
@@ -170,7 +170,7 @@ SweepArgs sweep_args(mgpu_engine *e, const double *U, const double *V, C2PCounte
   a.sigma = e->cfg.sigma;
   a.cp = e->cfg.cp;
   a.stats = st;
-  a.fail_count = e->fail_count;
+  a.fail = e->fail;
   a.fail_list = e->fail_list;
   a.fail_flag = e->fail_flag;
   return a;
@@ -253,7 +253,7 @@ int run_sweeps(mgpu_engine *e, SweepArgs a, int last_mode) {
 int retry(mgpu_engine *e, const double *U, double *V, double *A, C2PCounters *st, double *root = nullptr) {
   if (e->cfg.model != MGPU_SRMHD) return 0;  // the resistive recovery has no retry (srrmhd.cc:574-579)
   const long long last = e->cfg.quirks ? e->geo.vstride - 1 : -1;
-  launch_c2p_retry_srmhd(e->geo, U, V, A, root, e->cfg.gamma, e->fail_count, e->fail_list, e->fail_flag, last, st,
+  launch_c2p_retry_srmhd(e->geo, U, V, A, root, e->cfg.gamma, e->fail, e->fail_list, e->fail_flag, last, st,
                          e->stream);
   HIP_OK(hipGetLastError());
   return mark(e, "c2p_retry");
@@ -362,7 +362,7 @@ int rksplit_step(mgpu_engine *e, double dt, C2PCounters *st) {
     const double *ext = extension_source(e, e->V);
     HIP_OK(hipGetLastError());
     launch_split_srmhd(e->geo, e->U, e->V, e->root ? nullptr : e->A, e->root, dt, e->cfg.gamma, e->cfg.cp, st,
-                       e->fail_count, e->fail_list, e->fail_flag, ext, e->stream);
+                       e->fail, e->fail_list, e->fail_flag, ext, e->stream);
   }
   else
     launch_split_srrmhd(e->geo, e->U, e->V, e->A, dt, e->cfg.gamma, e->cfg.sigma, e->cfg.cp, st, e->stream);
@@ -382,7 +382,7 @@ RkStageArgs rk_args(mgpu_engine *e, double dt, C2PCounters *st) {
   a.sigma = e->cfg.sigma;
   a.cp = e->cfg.cp;
   a.stats = st;
-  a.fail_count = e->fail_count;
+  a.fail = e->fail;
   a.fail_list = e->fail_list;
   a.fail_flag = e->fail_flag;
   return a;
@@ -737,10 +737,10 @@ int mgpu_create(const mgpu_config *cfg, mgpu_engine **out) {
   }
   if (hipHostMalloc(reinterpret_cast<void **>(&e->cells_total), sizeof(CellCounters), hipHostMallocDefault) != hipSuccess)
     return cleanup(fail("hipHostMalloc of the cell-list counters failed"));
-  if (hipMalloc(&e->dstats, sizeof(C2PCounters) * kStatBuckets) != hipSuccess || hipMalloc(&e->fail_count, 2 * sizeof(int)) != hipSuccess ||
+  if (hipMalloc(&e->dstats, sizeof(C2PCounters) * kStatBuckets) != hipSuccess || hipMalloc(&e->fail, kFailInts * sizeof(int)) != hipSuccess ||
       hipMalloc(&e->fail_list, n * sizeof(long long)) != hipSuccess || hipMalloc(&e->fail_flag, n) != hipSuccess)
     return cleanup(fail("hipMalloc of C2P work arrays failed"));
-  if (hipMemset(e->fail_count, 0, 2 * sizeof(int)) != hipSuccess || hipMemset(e->fail_flag, 0, n) != hipSuccess ||
+  if (hipMemset(e->fail, 0, kFailInts * sizeof(int)) != hipSuccess || hipMemset(e->fail_flag, 0, n) != hipSuccess ||
       hipMemset(e->dstats, 0, sizeof(C2PCounters) * kStatBuckets) != hipSuccess)
     return cleanup(fail("hipMemset failed"));
   *out = e;
@@ -765,7 +765,7 @@ int mgpu_destroy(mgpu_engine *e) {
   if (e->rg_src) hipFree(e->rg_src);
   if (e->dstats) hipFree(e->dstats);
   if (e->dspeed) hipFree(e->dspeed);
-  if (e->fail_count) hipFree(e->fail_count);
+  if (e->fail) hipFree(e->fail);
   if (e->fail_list) hipFree(e->fail_list);
   if (e->fail_flag) hipFree(e->fail_flag);
   if (e->mlp) hipFree(e->mlp);
@@ -1115,7 +1115,7 @@ int launch_c2p(mgpu_engine *e) {
   if (e->cfg.model == MGPU_SRMHD && e->guess_mode == MGPU_GUESS_LEARNED)
     launch_c2p_learned_srmhd(e->geo, e->U, e->V, e->A, e->mlp, e->cfg.gamma, e->dstats, e->hist, e->stream);
   else if (e->cfg.model == MGPU_SRMHD)
-    launch_c2p_srmhd(e->geo, e->U, e->V, e->A, e->cfg.gamma, e->dstats, e->fail_count, e->fail_list, e->fail_flag,
+    launch_c2p_srmhd(e->geo, e->U, e->V, e->A, e->cfg.gamma, e->dstats, e->fail, e->fail_list, e->fail_flag,
                      e->guess_mode == MGPU_GUESS_COLD, e->hist, e->stream);
   else
     launch_c2p_srrmhd(e->geo, e->U, e->V, e->A, e->cfg.gamma, e->cfg.sigma, e->dstats, e->stream);

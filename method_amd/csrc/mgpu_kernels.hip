@@ -233,9 +233,7 @@ __device__ __forceinline__ void finish_rk2(const SweepArgs &a, unsigned o, const
   }
   cs.add(its);
   if (its < 0) {
-    const int slot = atomicAdd(a.fail_count, 1);
-    a.fail_list[slot] = o >> 3;
-    a.fail_flag[o >> 3] = 1;
+    note_failed(a.fail, a.fail_list, a.fail_flag, o >> 3);
   }
 }
 
@@ -1280,7 +1278,7 @@ __global__ __launch_bounds__(kThreads) void k_aux_srrmhd(Geo g, const double *U,
 // (srmhd.cc:390-562).
 // cold: start from v^2 = 0, Z = tau + D instead of the previous primitives.
 __global__ __launch_bounds__(kThreads) void k_c2p_srmhd(Geo g, const double *U, double *V, double *A, double gam,
-                                                         C2PCounters *st, int *fail_count, long long *fail_list,
+                                                         C2PCounters *st, int *fail, long long *fail_list,
                                                          unsigned char *fail_flag, int cold,
                                                          unsigned long long *hist) {
   const long long q = (long long)blockIdx.x * kThreads + threadIdx.x;
@@ -1311,9 +1309,7 @@ __global__ __launch_bounds__(kThreads) void k_c2p_srmhd(Geo g, const double *U, 
     steps = its;
     if (its < 0) {
       fails = 1;
-      const int slot = atomicAdd(fail_count, 1);
-      fail_list[slot] = q;
-      fail_flag[q] = 1;
+      note_failed(fail, fail_list, fail_flag, q);
     } else {
       iters = its;
       maxit = its;
@@ -1326,20 +1322,18 @@ __global__ __launch_bounds__(kThreads) void k_c2p_srmhd(Geo g, const double *U, 
 // Retry of failed cells from the mean root of converged interior face
 // neighbours (srmhd.cc:465-507). With `last_cell` >= 0 the system solved is
 // that cell's, as the reference's retry reuses the last cell's arguments.
-// fail_count[0] holds the list's length, fail_count[1] the workgroups done:
-// the last workgroup to finish clears the flags and both counters, so the
-// whole retry is one launch. Almost always the list is empty, every workgroup
-// leaves at once and the launch itself is the cost: as three launches (retry,
-// clear, zero) the KH 64^2 RK2 step took 35.7 us and the KH 331 x 517 one
-// 79.9; with this one they take 28.2 and 73.4.
-// An empty list leaves the counters as they are; otherwise no workgroup resets
-// them before all have read the length, since each counts itself after that.
+// The last workgroup to finish empties the list, so the whole retry is one
+// launch. Almost always the list is empty, every workgroup leaves at once and the
+// launch itself is the cost: as three launches (retry, clear, zero) the KH 64^2
+// RK2 step took 35.7 us and the KH 331 x 517 one 79.9; with this one they take
+// 28.2 and 73.4.
 __global__ __launch_bounds__(kThreads) void k_c2p_retry_srmhd(Geo g, const double *U, double *V, double *A,
-                                                               double *root, double gam, int *fail_count,
+                                                               double *root, double gam, int *fail,
                                                                const long long *fail_list, unsigned char *fail_flag,
                                                                long long last_cell, C2PCounters *st) {
-  const int nfail = *fail_count;
+  const int nfail = fail[kFailCount];
   if (nfail == 0) return;
+  const unsigned char mark = (unsigned char)(fail[kFailMark] + 1);
   const long long vs = g.vstride;
   for (int f = blockIdx.x * kThreads + threadIdx.x; f < nfail; f += gridDim.x * kThreads) {
     const long long q = fail_list[f];
@@ -1354,7 +1348,7 @@ __global__ __launch_bounds__(kThreads) void k_c2p_retry_srmhd(Geo g, const doubl
         const int np = pos[ax] + s;
         if (np < 0 || np >= g.n[ax] || g.n[ax] == 1) continue;
         const long long m = q + s * g.stride[ax];
-        if (fail_flag[m]) continue;
+        if (fail_flag[m] == mark) continue;
         double rho = V[m], vx = V[vs + m], vy = V[2 * vs + m], vz = V[3 * vs + m], p = V[4 * vs + m];
         double v2, Z;
         srmhd_plain_guess(rho, vx, vy, vz, p, gam, v2, Z);
@@ -1384,20 +1378,7 @@ __global__ __launch_bounds__(kThreads) void k_c2p_retry_srmhd(Geo g, const doubl
     }
     if (st && its < 0) atomicAdd(&st->retry_failures, 1ull);
   }
-  // this workgroup's flag reads come before its count, and the clearing
-  // workgroup's stores after every count
-  __shared__ int s_last;
-  __threadfence();
-  __syncthreads();
-  if (threadIdx.x == 0) s_last = atomicAdd(&fail_count[1], 1) == (int)gridDim.x - 1;
-  __syncthreads();
-  if (!s_last) return;
-  __threadfence();
-  for (int f = threadIdx.x; f < nfail; f += kThreads) fail_flag[fail_list[f]] = 0;
-  if (threadIdx.x == 0) {
-    fail_count[0] = 0;
-    fail_count[1] = 0;
-  }
+  end_retry(fail, fail_flag, vs);
 }
 
 // Per-axis maximum of srmhd_max_speed over interior cells: grid-stride
@@ -1532,7 +1513,7 @@ __global__ __launch_bounds__(kThreads) void k_source_srmhd(Geo g, PadGeo pg, con
 // extension only phi changes, so only phi is written back.
 __global__ __launch_bounds__(kThreads) void k_split_srmhd(Geo g, double *U, double *V, double *A, double *root,
                                                            double dt, double gam, double cp, C2PCounters *st,
-                                                           int *fail_count, long long *fail_list,
+                                                           int *fail, long long *fail_list,
                                                            unsigned char *fail_flag, const double *ext) {
   const long long q = (long long)blockIdx.x * kThreads + threadIdx.x;
   int cells = 0, iters = 0, fails = 0, maxit = 0;
@@ -1573,9 +1554,7 @@ __global__ __launch_bounds__(kThreads) void k_split_srmhd(Geo g, double *U, doub
     cells = 1;
     if (its < 0) {
       fails = 1;
-      const int slot = atomicAdd(fail_count, 1);
-      fail_list[slot] = q;
-      fail_flag[q] = 1;
+      note_failed(fail, fail_list, fail_flag, q);
     } else {
       iters = its;
       maxit = its;
@@ -1716,9 +1695,7 @@ __global__ __launch_bounds__(kThreads) void k_rkplus_stage(RkStageArgs a) {
       }
       cs.add(its);
       if (its < 0) {
-        const int slot = atomicAdd(a.fail_count, 1);
-        a.fail_list[slot] = q;
-        a.fail_flag[q] = 1;
+        note_failed(a.fail, a.fail_list, a.fail_flag, q);
       }
     }
   }
@@ -2075,16 +2052,16 @@ void launch_aux_srrmhd(const Geo &g, const double *U, const double *root, double
 }
 
 void launch_c2p_srmhd(const Geo &g, const double *U, double *V, double *A, double gam, C2PCounters *st,
-                      int *fail_count, long long *fail_list, unsigned char *fail_flag, int cold,
+                      int *fail, long long *fail_list, unsigned char *fail_flag, int cold,
                       unsigned long long *hist, hipStream_t s) {
-  hipLaunchKernelGGL(k_c2p_srmhd, dim3(blocks_for(g.vstride)), dim3(kThreads), 0, s, g, U, V, A, gam, st, fail_count,
+  hipLaunchKernelGGL(k_c2p_srmhd, dim3(blocks_for(g.vstride)), dim3(kThreads), 0, s, g, U, V, A, gam, st, fail,
                      fail_list, fail_flag, cold, hist);
 }
 
 void launch_c2p_retry_srmhd(const Geo &g, const double *U, double *V, double *A, double *root, double gam,
-                            int *fail_count, const long long *fail_list, unsigned char *fail_flag,
+                            int *fail, const long long *fail_list, unsigned char *fail_flag,
                             long long last_cell, C2PCounters *st, hipStream_t s) {
-  hipLaunchKernelGGL(k_c2p_retry_srmhd, dim3(64), dim3(kThreads), 0, s, g, U, V, A, root, gam, fail_count,
+  hipLaunchKernelGGL(k_c2p_retry_srmhd, dim3(64), dim3(kThreads), 0, s, g, U, V, A, root, gam, fail,
                      fail_list, fail_flag, last_cell, st);
 }
 
@@ -2095,10 +2072,10 @@ void launch_max_wavespeed_srmhd(const Geo &g, const double *V, const double *A, 
 }
 
 void launch_split_srmhd(const Geo &g, double *U, double *V, double *A, double *root, double dt, double gam,
-                        double cp, C2PCounters *st, int *fail_count, long long *fail_list, unsigned char *fail_flag,
+                        double cp, C2PCounters *st, int *fail, long long *fail_list, unsigned char *fail_flag,
                         const double *ext, hipStream_t s) {
   hipLaunchKernelGGL(k_split_srmhd, dim3(blocks_for(g.vstride)), dim3(kThreads), 0, s, g, U, V, A, root, dt, gam,
-                     cp, st, fail_count, fail_list, fail_flag, ext);
+                     cp, st, fail, fail_list, fail_flag, ext);
 }
 
 void launch_split_srrmhd(const Geo &g, double *U, double *V, double *A, double dt, double gam, double sigma,

@@ -28,6 +28,11 @@ constexpr int kStatBuckets = 128;
 // cell's place in a variable's plane as a 32-bit byte offset (mgpu_tile.hpp).
 constexpr long long kMaxCells = 1LL << 29;
 
+// What `fail` holds of the failed cells' list (mgpu_tile.hpp, note_failed): its
+// length, the workgroups done with its retry and, in a 128-byte line of its own,
+// the marks used up.
+enum { kFailCount = 0, kFailDone = 1, kFailMark = 32, kFailInts = 64 };
+
 // What the last phase of a sweep does with a cell's net flux: write it, add
 // it to the accumulator, finish an RK2 stage (RK2.cc:58-66 / 81-90, with
 // cons2prim), finish SSP2 stage two (flux1 complete: store it and solve the
@@ -72,7 +77,7 @@ struct SweepArgs {
   const double *S1;  // SSP2: source1 (components 8..12)
   double *Sout;      // SSP2 stage one: its source, source1 (components 8..12)
   C2PCounters *stats;
-  int *fail_count;
+  int *fail;
   long long *fail_list;
   unsigned char *fail_flag;
   const double *Fin;  // stored flux vectors [dir][var][cell] (model ids 2, 3)
@@ -115,15 +120,15 @@ void launch_aux_srrmhd(const Geo &g, const double *U, const double *root, double
                        hipStream_t s);
 // hist: null, or kHistBins Newton-step counters the cells are added to.
 void launch_c2p_srmhd(const Geo &g, const double *U, double *V, double *A, double gam, C2PCounters *st,
-                      int *fail_count, long long *fail_list, unsigned char *fail_flag, int cold,
+                      int *fail, long long *fail_list, unsigned char *fail_flag, int cold,
                       unsigned long long *hist, hipStream_t s);
 void launch_c2p_retry_srmhd(const Geo &g, const double *U, double *V, double *A, double *root, double gam,
-                            int *fail_count, const long long *fail_list, unsigned char *fail_flag,
+                            int *fail, const long long *fail_list, unsigned char *fail_flag,
                             long long last_cell, C2PCounters *st, hipStream_t s);
 // RKSplit's source half-step and cons2prim over interior cells.
 // A null: the cons2prim root (v^2, Z) goes to `root` in place of the aux.
 void launch_split_srmhd(const Geo &g, double *U, double *V, double *A, double *root, double dt, double gam,
-                        double cp, C2PCounters *st, int *fail_count, long long *fail_list, unsigned char *fail_flag,
+                        double cp, C2PCounters *st, int *fail, long long *fail_list, unsigned char *fail_flag,
                         const double *ext, hipStream_t s);
 void launch_split_srrmhd(const Geo &g, double *U, double *V, double *A, double dt, double gam, double sigma,
                          double cp, C2PCounters *st, hipStream_t s);
@@ -142,7 +147,7 @@ struct RkStageArgs {
   double *Uout, *Vout, *Aout;
   double dt, gamma, sigma, cp;
   C2PCounters *stats;
-  int *fail_count;
+  int *fail;
   long long *fail_list;
   unsigned char *fail_flag;
 };

@@ -3,7 +3,7 @@
 // at a 32-bit offset from a scalar base.
 #pragma once
 
-#include <hip/hip_runtime.h>
+#include "mgpu_kernels.hpp"
 
 namespace mgpu {
 
@@ -78,5 +78,52 @@ __device__ __forceinline__ double ld(const double *p, unsigned o) { return *at_o
 __device__ __forceinline__ double ld_nt(const double *p, unsigned o) { return __builtin_nontemporal_load(at_offset(p, o)); }
 __device__ __forceinline__ void st(double *p, unsigned o, double x) { *at_offset(p, o) = x; }
 __device__ __forceinline__ void st_nt(double *p, unsigned o, double x) { __builtin_nontemporal_store(x, at_offset(p, o)); }
+
+// Cells whose cons2prim failed in a stage, for the retry that ends it: their
+// list, its length fail[kFailCount] and a flag per cell, which is up if it equals
+// this stage's mark. A retry that is over raises the mark (fail[kFailMark] + 1,
+// up to 255) instead of taking the flags down again: that was the last
+// workgroup's work, and with every cell of 200^3 failed a cons2prim took 16.7 ms
+// where it takes 4.2 now (4.6 with a launch of 64 workgroups for the flags). The
+// mark has its own cache line: read from the line that the length's atomics keep
+// moving, it cost as much again as the Newton solves. Zeroed memory is an empty
+// list.
+constexpr int kFailMarks = 255;
+
+__device__ __forceinline__ void note_failed(int *fail, long long *list, unsigned char *flag, long long q) {
+  list[atomicAdd(&fail[kFailCount], 1)] = q;
+  flag[q] = (unsigned char)(fail[kFailMark] + 1);
+}
+
+// Empties the list, by one workgroup of kThreads; n: the number of flags, which
+// go down only when the marks are used up, once in 255 lists (hipMalloc aligns
+// them, so 16 at a time).
+__device__ __forceinline__ void forget_failed(int *fail, unsigned char *flag, long long n) {
+  const int mark = fail[kFailMark] + 1;
+  if (mark == kFailMarks) {
+    for (long long k = threadIdx.x; k < n / 16; k += kThreads) reinterpret_cast<uint4 *>(flag)[k] = uint4{0, 0, 0, 0};
+    for (long long k = n / 16 * 16 + threadIdx.x; k < n; k += kThreads) flag[k] = 0;
+  }
+  __syncthreads();  // every thread has read the mark
+  if (threadIdx.x == 0) {
+    fail[kFailCount] = 0;
+    fail[kFailDone] = 0;
+    fail[kFailMark] = mark == kFailMarks ? 0 : mark;
+  }
+}
+
+// The end of a retry of a non-empty list over the whole grid: the last workgroup
+// to get here empties the list. No workgroup does so before all have read its
+// length and the flags, since each counts itself after that.
+__device__ __forceinline__ void end_retry(int *fail, unsigned char *flag, long long n) {
+  __shared__ int s_last;
+  __threadfence();
+  __syncthreads();
+  if (threadIdx.x == 0) s_last = atomicAdd(&fail[kFailDone], 1) == (int)gridDim.x - 1;
+  __syncthreads();
+  if (!s_last) return;
+  __threadfence();
+  forget_failed(fail, flag, n);
+}
 
 }  // namespace mgpu
