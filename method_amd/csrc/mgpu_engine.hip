@@ -1152,6 +1152,10 @@ int mgpu_timed_c2p(mgpu_engine *e, int reps, double *ms_per_call, mgpu_stats *st
     HIP_OK(hipEventRecord(a, e->stream));
     if (rc == 0 && launch_c2p(e)) rc = -1;
     HIP_OK(hipEventRecord(b, e->stream));
+    // no retry follows: the list would grow from call to call, past its end, and
+    // the next step's retry would take these cells for its own
+    launch_forget_failed(e->geo, e->fail, e->fail_flag, e->stream);
+    HIP_OK(hipGetLastError());
     HIP_OK(hipEventSynchronize(b));
     float ms = 0.f;
     HIP_OK(hipEventElapsedTime(&ms, a, b));

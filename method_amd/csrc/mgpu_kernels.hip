@@ -1381,6 +1381,11 @@ __global__ __launch_bounds__(kThreads) void k_c2p_retry_srmhd(Geo g, const doubl
   end_retry(fail, fail_flag, vs);
 }
 
+// Empties the list of a cons2prim that no retry follows.
+__global__ __launch_bounds__(kThreads) void k_forget_failed(int *fail, unsigned char *fail_flag, long long n) {
+  if (fail[kFailCount] > 0) forget_failed(fail, fail_flag, n);
+}
+
 // Per-axis maximum of srmhd_max_speed over interior cells: grid-stride
 // per-thread maxima, a butterfly over the 64 lanes with __shfl_xor, one LDS
 // slot per wave, then one atomicMax per block on the bit pattern (for
@@ -2063,6 +2068,10 @@ void launch_c2p_retry_srmhd(const Geo &g, const double *U, double *V, double *A,
                             long long last_cell, C2PCounters *st, hipStream_t s) {
   hipLaunchKernelGGL(k_c2p_retry_srmhd, dim3(64), dim3(kThreads), 0, s, g, U, V, A, root, gam, fail,
                      fail_list, fail_flag, last_cell, st);
+}
+
+void launch_forget_failed(const Geo &g, int *fail, unsigned char *fail_flag, hipStream_t s) {
+  hipLaunchKernelGGL(k_forget_failed, dim3(1), dim3(kThreads), 0, s, fail, fail_flag, g.vstride);
 }
 
 void launch_max_wavespeed_srmhd(const Geo &g, const double *V, const double *A, unsigned long long *out,

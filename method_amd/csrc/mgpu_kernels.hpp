@@ -125,6 +125,8 @@ void launch_c2p_srmhd(const Geo &g, const double *U, double *V, double *A, doubl
 void launch_c2p_retry_srmhd(const Geo &g, const double *U, double *V, double *A, double *root, double gam,
                             int *fail, const long long *fail_list, unsigned char *fail_flag,
                             long long last_cell, C2PCounters *st, hipStream_t s);
+// Empties the list of failed cells without a retry.
+void launch_forget_failed(const Geo &g, int *fail, unsigned char *fail_flag, hipStream_t s);
 // RKSplit's source half-step and cons2prim over interior cells.
 // A null: the cons2prim root (v^2, Z) goes to `root` in place of the aux.
 void launch_split_srmhd(const Geo &g, double *U, double *V, double *A, double *root, double dt, double gam,

@@ -264,3 +264,30 @@ def test_retry_of_every_cell_takes_no_longer_than_the_cells_do():
                 best = min(best, time.perf_counter() - t)
             took.append(best)
     assert took[1] <= 14 * took[0], took
+
+
+def test_timed_c2p_leaves_no_failed_cells_behind():
+    """The timed cons2prim runs without a retry. Its failed cells are forgotten,
+    three lists of every cell among them: the prims stay those of the first pass,
+    and the step after it, from good prims, is the step of an engine that timed
+    nothing, bit for bit (a cell found on an old list would be solved again, from
+    its neighbours' mean root)."""
+    n = 10
+    g = idt.kh3d_grid(n)
+    cfg = eng.Config(n, n, n, -0.5, 0.5, -1.0, 1.0, 0.0, 1.0, quirks=0)
+    print("gpu: timed cons2prim with failures", flush=True)
+    got = []
+    for timed in (False, True):
+        with eng.Engine(cfg) as e:
+            e.set_prims(idt.kh_prims(g, seed=3))
+            cons, true, aux = e.download()
+            if timed:
+                e.upload(prims=failing(true, np.ones(true.shape[1:], bool)))
+                _, st, _ = e.timed_c2p(3)
+                assert st["failures"] == n**3
+                e.upload(cons, true, aux)
+            rc, st = e.update_time(stats=True)
+            assert rc == 0 and st["failures"] == 0
+            got.append(e.download())
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
