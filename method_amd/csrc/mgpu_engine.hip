@@ -91,7 +91,9 @@ struct mgpu_engine {
   // SRMHD steps (RK4_10's aside) keep the cons2prim root (v^2, Z) of each cell
   // instead of writing its 13 aux values, and SRRMHD SSP2 steps the root Z
   // instead of 17: no kernel of those steps reads aux, and what does (state
-  // download, wavespeed) forms it from the root first.
+  // download, wavespeed) forms it from the root first. The root takes the aux
+  // array's first planes, which nothing reads while the aux is stale; each
+  // cell's aux replaces its own root.
   double *root = nullptr;
   bool aux_stale = false;
   // cell-list operators (single-cell model calls): device copies of the
@@ -706,14 +708,7 @@ int mgpu_create(const mgpu_config *cfg, mgpu_engine **out) {
       return cleanup(fail("hipMalloc of %zu bytes failed", b.elems * sizeof(double)));
     if (hipMemset(*b.ptr, 0, b.elems * sizeof(double)) != hipSuccess) return cleanup(fail("hipMemset failed"));
   }
-  if (c.model == MGPU_SRMHD && c.integrator != MGPU_RK4_10) {
-    if (hipMalloc(&e->root, 2 * n * sizeof(double)) != hipSuccess)
-      return cleanup(fail("hipMalloc of the cons2prim root store failed"));
-  }
-  if (c.model == MGPU_SRRMHD && c.integrator == MGPU_SSP2) {
-    if (hipMalloc(&e->root, n * sizeof(double)) != hipSuccess)
-      return cleanup(fail("hipMalloc of the cons2prim root store failed"));
-  }
+  if (c.model == MGPU_SRMHD ? c.integrator != MGPU_RK4_10 : c.integrator == MGPU_SSP2) e->root = e->A;
   if (c.integrator >= MGPU_RK2B) {
     // stage states of RK2B, RK3, RK4, RK4_10 (RKPlus.cc:56-586)
     static const int kStages[4] = {1, 2, 4, 2};
@@ -751,7 +746,7 @@ int mgpu_destroy(mgpu_engine *e) {
   if (!e) return 0;
   if (e->stream) hipStreamSynchronize(e->stream);
   double *bufs[] = {e->U,  e->V,  e->A,  e->U1, e->V1, e->fnet,     e->staging,
-                    e->U2, e->V2, e->Pf, e->S1, e->root};
+                    e->U2, e->V2, e->Pf, e->S1};
   for (double *b : bufs)
     if (b) hipFree(b);
   for (int k = 0; k < 4; ++k) {

@@ -1,6 +1,7 @@
 """Edges of how the step's work is split over launches and workgroups: lists
 longer than one launch's threads, tiles smaller than the default and grids on
 either side of a rule's line. Needs an MI355X."""
+import ctypes
 import time
 
 import numpy as np
@@ -291,3 +292,34 @@ def test_timed_c2p_leaves_no_failed_cells_behind():
             got.append(e.download())
     for a, b in zip(*got):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("integrator,stages", [(eng.RK2B, 1), (eng.RK3, 2), (eng.RK4, 4)])
+def test_rkplus_engines_hold_no_root_beside_the_aux(integrator, stages):
+    """Device memory of an SRMHD RKPlus engine: cons, prims and aux (30 doubles a
+    cell), one stage's cons and prims and the net flux (26), 17 per stage state, 9
+    for RK4's kept rhs, 9 bytes of the failed cells' list and flags, and less than
+    half a double of rounding up to whole pages. The cons2prim root lives in the
+    aux array, and the aux formed from it there is the one a fresh array gets."""
+    hip = ctypes.CDLL("libamdhip64.so.7")
+
+    def free_memory():
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipDeviceSynchronize() == 0
+        assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    n = 1024
+    print(f"gpu: memory of integrator {integrator}", flush=True)
+    eng.Engine(eng.Config(8, 8, 0, 0.0, 1.0, 0.0, 1.0, integrator=integrator)).close()
+    free = free_memory()
+    with eng.Engine(eng.Config(n, n, 0, -0.5, 0.5, -1.0, 1.0, integrator=integrator)) as e:
+        used = (free - free_memory()) / (8 * n * n)
+        assert used <= 56 + 17 * stages + (9 if integrator == eng.RK4 else 0) + 9 / 8 + 0.5, used
+        e.set_prims(idt.kh_prims(idt.Grid(n, n, 0, -0.5, 0.5, -1.0, 1.0), seed=8))
+        assert e.update_time() == 0
+        _, q, a = e.download()
+        again = e.download()[2]
+    v2 = (q[1:4] ** 2).sum(0)
+    assert np.abs(a[9] - v2).max() <= 1e-13 and np.abs(a[1] * np.sqrt(1 - v2) - 1).max() <= 1e-12
+    assert np.array_equal(a, again)
