@@ -1024,7 +1024,7 @@ int mgpu_batch_autotune(mgpu_batch *b, int trial_steps, mgpu_batch_tuning *best,
   for (int s = 0; s < kNumShapes && rc == 0; ++s) {
     for (int sched = kSchedStatic; sched <= kSchedDynamic && rc == 0; ++sched) {
       const int maxb = max_blocks_per_cu(b, s, sched);
-      for (int bpc = std::max(1, maxb - 1); bpc <= maxb && rc == 0; ++bpc) {
+      for (int bpc = 1; bpc <= maxb && rc == 0; ++bpc) {
         mgpu_batch_tuning cand;
         cand.tile_x = kShapes[s].tx;
         cand.tile_y = kShapes[s].ty;

@@ -323,3 +323,20 @@ def test_rkplus_engines_hold_no_root_beside_the_aux(integrator, stages):
     v2 = (q[1:4] ** 2).sum(0)
     assert np.abs(a[9] - v2).max() <= 1e-13 and np.abs(a[1] * np.sqrt(1 - v2) - 1).max() <= 1e-12
     assert np.array_equal(a, again)
+
+
+def test_autotuner_tries_every_workgroup_count():
+    """The autotuner's list holds each tile shape and schedule with 1, 2, ... up to
+    the resident number of workgroups per CU, and the fastest is the one chosen."""
+    print("gpu: autotuner candidates", flush=True)
+    with eng.Batch([eng.Instance(40, 31)], weno_order=3) as b:
+        b.set_prims(0, idt.kh_prims(idt.Grid(40, 31, 0, -0.5, 0.5, -1.0, 1.0), seed=1))
+        best, tried = b.autotune(2)
+    counts = {}
+    for c in tried:
+        counts.setdefault((c["tile_x"], c["tile_y"], c["schedule"]), []).append(c["blocks"])
+    assert len(counts) == 8  # four shapes, two schedules
+    for blocks in counts.values():
+        assert blocks == [blocks[0] * k for k in range(1, len(blocks) + 1)] and len(blocks) >= 3, counts
+    fastest = min(tried, key=lambda c: c["ms_per_step"])
+    assert all(best[k] == fastest[k] for k in ("tile_x", "tile_y", "schedule", "blocks"))
