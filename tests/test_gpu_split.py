@@ -340,3 +340,60 @@ def test_autotuner_tries_every_workgroup_count():
         assert blocks == [blocks[0] * k for k in range(1, len(blocks) + 1)] and len(blocks) >= 3, counts
     fastest = min(tried, key=lambda c: c["ms_per_step"])
     assert all(best[k] == fastest[k] for k in ("tile_x", "tile_y", "schedule", "blocks"))
+
+
+def waves_3d(n, ng=4):
+    """SRMHD prims that vary along all three axes, each with its own wavelengths."""
+    x, y, z = np.meshgrid(*[np.linspace(0.0, 1.0, k + 2 * ng) for k in n], indexing="ij")
+    p = np.zeros((8,) + x.shape)
+    p[0], p[4] = 1.0 + 0.3 * np.sin(9 * x + 17 * y + 23 * z), 1.0 + 0.3 * np.cos(7 * x - 13 * y + 19 * z)
+    p[1], p[2], p[3] = 0.3 * np.cos(5 * x + 29 * z), 0.2 * np.sin(3 * x + 31 * y), 0.2 * np.cos(11 * y - 8 * z)
+    p[5], p[6], p[7] = 0.4 * np.sin(6 * y), 0.3 * np.sin(2 * x + 37 * z), 0.2 * np.cos(x + 21 * y)
+    return p
+
+
+@pytest.mark.parametrize("n", [(50, 131, 129), (17, 190, 190), (48, 127, 129), (6007, 11, 17)])
+@pytest.mark.parametrize("weno,periodic", [(3, 1), (3, 0), (5, 1), (5, 0)])
+def test_marching_x_sweep_keeps_to_its_columns(n, weno, periodic):
+    """The marching x sweep on a state that varies along y and z, with a last wave
+    of 3, 4 and 63 columns in use and, on the long thin grid, of 59 and hundreds of
+    segments: the net flux against plan 0, whose x sweep is tiled and sums the axes
+    the other way round. Same terms in another order: three roundings, 3.4e-16 of
+    the terms, which are within ten times the largest net flux."""
+    print(f"gpu: marching x sweep with structure {n} weno={weno} periodic={periodic}", flush=True)
+    got = []
+    for plan in (3, 0):
+        with eng.Engine(eng.Config(*n, 0.0, 1.0, 0.0, 1.0, 0.0, 1.0, weno_order=weno, bc=(periodic,) * 3)) as e:
+            e.set_sweep_plan(plan)
+            e.set_prims(waves_3d(n))
+            got.append(e.fnet())
+    for v, (a, b) in enumerate(zip(*got)):
+        assert np.isfinite(a).all() and np.abs(a - b).max() <= 3.4e-15 * np.abs(got[1]).max(), v
+
+
+TILES_3D = [(70, 17, 33), (9, 130, 97), (9, 130, 104)]  # 16 x 16, 8 x 32 and, by its aligned rows, 16 x 16 again
+
+
+@pytest.mark.parametrize("n", TILES_3D)
+@pytest.mark.parametrize("kind,weno", [("rk2", 3), ("rk2", 5), ("rk3", 3), ("rk4", 5), ("ssp2", 3), ("ssp2", 5),
+                                       ("resistive rk2", 5), ("resistive rk3", 3)])
+def test_3d_modes_on_every_tile_bitwise(n, kind, weno):
+    """What the fused y + z launch does with a cell (RK2, RKPlus and both SSP2
+    stages) on the tiles of grids beyond 256 16 x 16 tiles, against plan 2's
+    separate launches: the same bits."""
+    print(f"gpu: 3-D {kind} {n} weno={weno}", flush=True)
+    p = waves_3d(n)
+    cfg = dict(integrator={"rk2": eng.RK2, "rk3": eng.RK3, "rk4": eng.RK4, "ssp2": eng.SSP2}[kind.split()[-1]])
+    if kind == "ssp2" or kind.startswith("resistive"):
+        p = np.concatenate([p, -np.cross(p[1:4], p[5:8], axis=0)])
+        cfg.update(model=eng.SRRMHD, sigma=1.0)
+    got = []
+    for plan in (3, 2):
+        with eng.Engine(eng.Config(*n, -0.5, 0.5, -1.0, 1.0, 0.0, 1.0, weno_order=weno, cp=1.0, **cfg)) as e:
+            e.set_sweep_plan(plan)
+            e.set_prims(p)
+            for _ in range(2):
+                e.update_time()
+            got.append(e.download())
+    for a, b in zip(*got):
+        assert np.isfinite(a).all() and np.array_equal(a, b)
