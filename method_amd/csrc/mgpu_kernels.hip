@@ -1924,16 +1924,28 @@ void launch_sweep_yzf_t(const SweepArgs &a, int quirk, hipStream_t s) {
 //   WENO3  32^3 - | 61.3 | 55.4, 64^3 108 | 105, 97 x 64 x 130 324 | 354
 // SRMHD takes 8 rows of 32 cells on grids longer than 64 along z: the z phase
 // recomputes 38/32 halo cells instead of 22/16 (the y phase 14/8), and rows
-// are read in 256-byte runs.
+// are read in 256-byte runs. Where rows are aligned to 64 bytes (nz a multiple of
+// 8) and 16 x 16 tiles cover the plane with fewer cells, those runs gain less than
+// the idle lanes cost (97 x 64 x nz, WENO3 and WENO5, us, 8 x 32 | 16 x 16: nz =
+// 80 166, 213 | 159, 193; 112 222, 282 | 217, 266; 144 271, 338 | 262, 322); on
+// other rows they gain more (65 188, 223 | 203, 225; 76 188, 225 | 192, 220; 100
+// 232, 283 | 245, 281; 129 286, 345 | 335, 371), and with as many cells they are
+// ahead or even (88 198, 241 | 206, 248; 160 283, 343 | 284, 347).
+inline bool square_tiles_3d(const Geo &g) {
+  const long long square = (g.n[1] + 15LL) / 16 * 16 * ((g.n[2] + 15) / 16 * 16);
+  const long long rows = (g.n[1] + 7LL) / 8 * 8 * ((g.n[2] + 31) / 32 * 32);
+  return g.n[2] <= 64 || (g.n[2] % 8 == 0 && square < rows);
+}
+
 template <class M, int ORDER, int MODE>
 void launch_sweep_yzf_o(const SweepArgs &a, int quirk, hipStream_t s) {
   constexpr int kRows = M::NC <= 9 ? 8 : 16, kCols = M::NC <= 9 ? 32 : 16;
   if (small_3d(a.geo))
     launch_sweep_yzf_t<M, ORDER, MODE, 8, 8>(a, quirk, s);
-  else if (a.geo.n[2] > 64)
-    launch_sweep_yzf_t<M, ORDER, MODE, kRows, kCols>(a, quirk, s);
-  else
+  else if (square_tiles_3d(a.geo))
     launch_sweep_yzf_t<M, ORDER, MODE, 16, 16>(a, quirk, s);
+  else
+    launch_sweep_yzf_t<M, ORDER, MODE, kRows, kCols>(a, quirk, s);
 }
 
 template <class M, int ORDER>
