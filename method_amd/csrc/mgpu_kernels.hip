@@ -1840,9 +1840,10 @@ template <class M, int ORDER, int MODE>
 void launch_sweep_o(const SweepArgs &a, int dir, int quirk, hipStream_t s) {
   if (a.geo.dims == 3) {
     if constexpr (MODE == kSweepWrite && !M::kStored && M::NC <= 9) {
-      const int nseg = dir == 0 ? march_segments(a.geo) : 0;
-      if (nseg > 0) {
-        const int nb = (int)((a.geo.stride[0] + 63) / 64), len = (a.geo.n[0] + nseg - 1) / nseg;
+      const int asked = dir == 0 ? march_segments(a.geo) : 0;
+      if (asked > 0) {
+        const int nb = (int)((a.geo.stride[0] + 63) / 64), len = (a.geo.n[0] + asked - 1) / asked;
+        const int nseg = (a.geo.n[0] + len - 1) / len;  // none past the grid's end
         hipLaunchKernelGGL(k_march_x<ORDER>, dim3(nb * nseg), dim3(kMarchThreads), 0, s, a, nseg, len);
         return;
       }
