@@ -309,8 +309,9 @@ int mgpu_batch_get_time(mgpu_batch *b, int i, double *t, double *dt, int *iters)
 int mgpu_batch_use_graph(mgpu_batch *b, int on);
 int mgpu_batch_get_tuning(const mgpu_batch *b, mgpu_batch_tuning *t);
 int mgpu_batch_set_tuning(mgpu_batch *b, const mgpu_batch_tuning *t);
-/* Times every candidate tuning (tile shape, schedule and workgroups per CU up to
- * the resident number) on trial_steps steps of this batch, keeps
+/* Times the candidate tunings on trial_steps steps of this batch: every tile
+ * shape and schedule, each with the two largest resident numbers of workgroups per
+ * CU and then with fewer, until fewer are 2 % slower than the best of them. Keeps
  * the fastest and restores the state and clocks as they were on entry. all
  * (may be NULL) receives up to max_all candidates; *nall the count. */
 int mgpu_batch_autotune(mgpu_batch *b, int trial_steps, mgpu_batch_tuning *best, mgpu_batch_tuning *all,

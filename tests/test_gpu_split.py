@@ -325,19 +325,27 @@ def test_rkplus_engines_hold_no_root_beside_the_aux(integrator, stages):
     assert np.array_equal(a, again)
 
 
-def test_autotuner_tries_every_workgroup_count():
-    """The autotuner's list holds each tile shape and schedule with 1, 2, ... up to
-    the resident number of workgroups per CU, and the fastest is the one chosen."""
-    print("gpu: autotuner candidates", flush=True)
-    with eng.Batch([eng.Instance(40, 31)], weno_order=3) as b:
-        b.set_prims(0, idt.kh_prims(idt.Grid(40, 31, 0, -0.5, 0.5, -1.0, 1.0), seed=1))
+@pytest.mark.parametrize("n", [(40, 31), (700, 650)])
+def test_autotuner_descends_the_workgroup_counts(n):
+    """The autotuner takes each tile shape and schedule with the two largest resident
+    numbers of workgroups per CU, then down to one or to the first number that is
+    2 % slower than the best, and chooses the fastest of all it tried."""
+    print(f"gpu: autotuner candidates {n}", flush=True)
+    with eng.Batch([eng.Instance(*n)], weno_order=3) as b:
+        b.set_prims(0, idt.kh_prims(idt.Grid(*n, 0, -0.5, 0.5, -1.0, 1.0), seed=1))
         best, tried = b.autotune(2)
-    counts = {}
+    rows = {}
     for c in tried:
-        counts.setdefault((c["tile_x"], c["tile_y"], c["schedule"]), []).append(c["blocks"])
-    assert len(counts) == 8  # four shapes, two schedules
-    for blocks in counts.values():
-        assert blocks == [blocks[0] * k for k in range(1, len(blocks) + 1)] and len(blocks) >= 3, counts
+        rows.setdefault((c["tile_x"], c["tile_y"], c["schedule"]), []).append((c["blocks"], c["ms_per_step"]))
+    assert len(rows) == 8  # four shapes, two schedules
+    ncu = min(row[1][0] - row[0][0] for row in rows.values())
+    for row in rows.values():
+        counts, ms = [k // ncu for k, _ in row], [t for _, t in row]
+        top = counts[1]
+        assert counts == [top - 1, top] + list(range(top - 2, counts[-1] - 1, -1))[:len(row) - 2], rows
+        down = [0] + list(range(2, len(row)))  # tried one after the other downwards
+        slower = [ms[k] > 1.02 * min(ms[:max(k, 1) + 1]) for k in down]
+        assert not any(slower[:-1]) and (1 in counts or slower[-1]), rows
     fastest = min(tried, key=lambda c: c["ms_per_step"])
     assert all(best[k] == fastest[k] for k in ("tile_x", "tile_y", "schedule", "blocks"))
 
