@@ -158,12 +158,14 @@ int mgpu_c2p_cells(mgpu_engine *e, long long n, const double *cons, double *prim
  * harnesses that forbid hipMalloc): cons, prims and aux are DEVICE arrays
  * in the same single-cell layout, read and written on the engine's stream
  * (order earlier writes to them before the call). The call allocates
- * nothing: its per-block counters and their total live in a static device
- * array of each GPU, sized for at most 4,194,304 cells per call (larger n is
- * an error). Calls on one GPU share that array, so calls that overlap on one
- * GPU (from several threads or streams) race. With stats NULL the call only
- * launches and returns 0 (mgpu_sync before reading the results); otherwise
- * it waits, fills stats and returns the failure count as mgpu_c2p_cells. */
+ * nothing: its per-block counters live in a static device array of each GPU,
+ * sized for at most 4,194,304 cells per call (larger n is an error), and their
+ * total goes there too, or with stats to a pinned host record that the engine
+ * owns. Calls on one GPU share the array and calls on one engine the record, so
+ * calls that overlap on one GPU (from several threads or streams) race. With
+ * stats NULL the call only launches and returns 0 (mgpu_sync before reading the
+ * results); otherwise it waits, fills stats and returns the failure count as
+ * mgpu_c2p_cells. */
 int mgpu_c2p_cells_noalloc(mgpu_engine *e, long long n, const double *cons, double *prims, double *aux,
                            mgpu_stats *stats);
 

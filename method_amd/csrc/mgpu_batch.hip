@@ -5,12 +5,13 @@
 // WENO3/5 (fluxVectorSplitting.cc:58-131); the instances differ in grid size,
 // initial state and time step. One persistent kernel per RK stage advances
 // the tiles of all instances: for a TX x TY tile it reconstructs the y faces
-// and then the x faces through LDS, keeps the y net flux in registers, and
+// and then the x faces through LDS, where the y net flux waits meanwhile, and
 // applies the stage update and the Newton cons2prim in place, so the net flux
 // never goes to HBM. A short launch ends each stage: it retries failed cells
 // and, after stage two, advances each instance's t, iteration count and dt.
-// One step (two stages and their ends) is captured in a hipGraph and replayed. Tile shape, schedule and workgroup
-// count come from an autotuner that times the candidates on the batch itself.
+// One step (two stages and their ends) is captured in a hipGraph and replayed.
+// Tile shape, schedule and workgroup count come from an autotuner that times the
+// candidates on the batch itself.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -451,15 +451,15 @@ void rk_out(RkStageArgs &a, double *U, double *V, double *A, const double *Vg) {
   a.Vg = Vg;
 }
 
-// RK2B, RK3, RK4 and RK4_10::step (RKPlus.cc:127-726). A stage's cons2prim
-// starts from the previous stage's prims, the last stage's from the step's.
 // The rhs of (Ub, Vb, Ab) and the stage a (whose terms and outputs are set)
 // from it, in the sweeps' own launches: the last sweep combines the stage and
 // runs its cons2prim, so the net flux of a 2-D grid never goes to HBM and no
 // pointwise launch follows (RK4 200^2 WENO3, a step of five stages with their
-// retries: 106 us as sweep and stage launches, now 77). The stage's output must be another state than the
-// one swept. Only the last stage needs prims beyond rho .. p, unless the model
-// extension reads them, and SRMHD's aux is kept as its root there.
+// retries: 106 us as sweep and stage launches, now 77). The stage's output must
+// be another state than the one swept, so RK4_10's, which are formed in place,
+// keep the pointwise launch. Only the last stage needs prims beyond rho .. p,
+// unless the model extension reads them, and SRMHD's aux is kept as its root
+// there.
 int rk_stage(mgpu_engine *e, const RkStageArgs &a, const double *Ub, const double *Vb, const double *Ab,
              C2PCounters *st, bool last = false) {
   const bool res = e->cfg.model != MGPU_SRMHD;
@@ -481,6 +481,8 @@ int rk_stage(mgpu_engine *e, const RkStageArgs &a, const double *Ub, const doubl
   return 0;
 }
 
+// RK2B, RK3, RK4 and RK4_10::step (RKPlus.cc:127-726). A stage's cons2prim
+// starts from the previous stage's prims, the last stage's from the step's.
 int rkplus_step(mgpu_engine *e, double dt, C2PCounters *st) {
   double *U = e->U, *V = e->V, *A = e->A;
   double **Us = e->rkU, **Vs = e->rkV, **As = e->rkA;

@@ -16,7 +16,7 @@ constexpr int kThreads = 256;  // per workgroup
 // its variables, pass by pass: its LDS addresses are one base plus constants,
 // and the few faces left over make one or two passes more. Dealing the items
 // out in one flat row took a division and a bounds check per item and half,
-// and the sweeps are bound by VALU issue (79-85 % of the cycles): with this
+// and the sweeps were bound by VALU issue then (79-85 % of the cycles): with this
 // and the 32-bit offsets below the fused y + z launch has 2,090 FP64 of 2,625
 // VALU instructions instead of 3,069, the x sweep 948 of 1,108 instead of
 // 1,292, and the KH 256^3 WENO5 step went from 5.82-5.88 to 5.44 ms, 128^3
