@@ -196,3 +196,29 @@ def test_flux_error_is_that_of_ieee_operations(lib, ratio, W):
     size = np.sqrt((exact * exact).sum(1))[:, None]
     mean = [(np.abs(x - exact) / size).astype(float).mean(0) for x in (got, ieee)]
     assert (mean[0] <= 1.03 * mean[1]).all(), (mean[0] / EPS, mean[1] / EPS)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("resistive", [False, True])
+def test_recovered_density_and_lorentz_factor_on_the_device(resistive):
+    """With the hardware's own estimates: 1/W is D's factor in rho and W its
+    reciprocal, rounded once each, so rho W gives D back to two roundings."""
+    from method_amd import engine as eng
+    from method_amd import initdata as idt
+
+    n, ng = 96, 4
+    g = idt.Grid(n, n, 0, -0.5, 0.5, -1.0, 1.0)
+    p = idt.kh_prims(g, seed=2)
+    p[4] *= 1e-3
+    cfg = dict(model=eng.SRMHD, integrator=eng.RK2)
+    if resistive:
+        p = np.concatenate([p, -np.cross(p[1:4], p[5:8], axis=0)])
+        cfg = dict(model=eng.SRRMHD, integrator=eng.SSP2, sigma=10.0)
+    print(f"gpu: rho W = D, resistive={resistive}", flush=True)
+    with eng.Engine(eng.Config(n, n, 0, -0.5, 0.5, -1.0, 1.0, **cfg)) as e:
+        e.set_prims(p)
+        for _ in range(3):
+            e.update_time()
+        c, q, a = (x[:, ng:-ng, ng:-ng] for x in e.download())
+    assert np.isfinite(q).all()
+    assert (np.abs(np.longdouble(q[0]) * a[1] / c[0] - 1) / EPS).max() <= 2.05
